@@ -385,23 +385,25 @@ __global__ void __launch_bounds__(WAVES * 64) flash_attention_kernel(const float
     if (query_in)
     {
         const float inv = 1.f / l;
+        // A lane holds four consecutive channels of its query: one store each.
 #pragma unroll
         for (int t = 0; t < 4; ++t)
-#pragma unroll
-            for (int r = 0; r < 4; ++r)
+        {
+            const size_t at = (size_t) query * width + column + 16 * t + 4 * g;
+            if constexpr (OUT == kF32)
+                *reinterpret_cast<f32x4*>(out + at) = o[t] * inv;
+            else
             {
-                const size_t at = (size_t) query * width + column + 16 * t + 4 * g + r;
-                if constexpr (OUT == kF32)
-                    out[at] = o[t][r] * inv;
-                else
-                {
-                    uint32_t bits[3];
-                    exact_parts<OUT>(o[t][r] * inv, bits);
+                uint32_t bits[4][3];
 #pragma unroll
-                    for (int p = 0; p < (OUT == kF16 ? 2 : 3); ++p)
-                        out_parts[p * out_part_stride + at] = (uint16_t) bits[p];
-                }
+                for (int r = 0; r < 4; ++r)
+                    exact_parts<OUT>(o[t][r] * inv, bits[r]);
+#pragma unroll
+                for (int p = 0; p < (OUT == kF16 ? 2 : 3); ++p)
+                    *reinterpret_cast<uint2*>(out_parts + p * out_part_stride + at)
+                        = uint2 {bits[0][p] | (bits[1][p] << 16), bits[2][p] | (bits[3][p] << 16)};
             }
+        }
     }
 }
 

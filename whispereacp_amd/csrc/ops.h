@@ -99,7 +99,7 @@ struct SplitProduct
     float scale0 = 1.f, scale1 = 1.f, scale2 = 1.f;
 };
 
-// 16-bit weights, inner % 32 == 0, out, split and split2 multiples of 128.
+// 16-bit weights, inner % 64 == 0, out, split and split2 multiples of 128.
 bool split_product_fits(int wdtype, int inner, int out, int split, int split2);
 hipError_t split_product(hipStream_t stream, const SplitProduct& product);
 // LayerNorm rows (as layernorm) written as the parts of split_product's input;

@@ -10,19 +10,30 @@
 // product's own epilogue (fc1 writes its GELU output as parts for fc2), so
 // the products' inner loops carry no conversion work.
 //
-// A 256-thread block computes a 128 x TN tile (TN 128, or 64 where 128-column
-// tiles would leave most CUs idle) in 32-wide k-steps. Both operands go
-// straight from memory into LDS with direct-to-LDS loads (each lane's 16 bytes
-// land at the wave's slot + 16·lane), into one of kStages stage buffers, so a
-// step's loads are issued kStages - 1 steps before its products and hold no
-// registers meanwhile. A 16-byte chunk c (8 k values) of tile row r sits at
-// slot 4r + (c ^ ((r >> 1) & 3)): a 16-byte operand read serves eight lanes
+// A block computes a TM x TN tile in 64-wide k-steps: every staged row segment
+// is then one whole 128-byte line (with 32-wide steps each request fetched half
+// a line, and the requests bound the products: 14-16 bytes a clock and CU).
+// Both operands go straight from memory into LDS with direct-to-LDS loads (each
+// lane's 16 bytes land at the wave's slot + 16·lane), into one of S stage
+// buffers, so a step's loads are issued S - 1 steps before its products and
+// hold no registers meanwhile. A 16-byte chunk c (8 k values) of tile row r
+// sits at slot 8r + (c ^ (r & 7)): a 16-byte operand read serves eight lanes
 // (128 bytes, the 32 banks) at a time, and the matrix-core operand reads (rows
-// li of a 16-row tile, chunk g, for lanes (li, g)) then give each eight lanes
-// eight different bank groups. The
-// loads are issued from inline assembly with explicit waits: the compiler's
-// own wait insertion would drain every load in flight before each LDS read.
-// The four waves form a 2 x 2 grid of 64 x TN/2 sub-tiles.
+// li of a 16-row tile, one chunk for each g, for lanes (li, g)) then give each
+// eight lanes eight different bank groups. The loads are issued from inline
+// assembly with explicit waits: the compiler's own wait insertion would drain
+// every load in flight before each LDS read.
+//
+// W is the matrix cores' row operand and X their column operand, so a lane ends
+// up with four consecutive outputs of one row and stores them together (16
+// bytes of fp32, 8 of each 16-bit part).
+//
+// Tiles measured at 1500 rows, two parts (us a launch, the same products in
+// 128 x 128 tiles of 32-wide steps on two stages or 128 x 64 on four before):
+//   1280 -> 5120  128 x 256: 38 (46)     5120 -> 1280  64 x 128: 45 (65)
+//   1280 -> 3840  128 x 256: 33 (38)     1280 -> 1280  64 x 128: 15 (19)
+//    384 -> 1152  64 x 128: 6.5 (7.9)    1536 -> 384   32 x 128: 9.8 (20)
+// and at 300 rows 5120 -> 1280 in 32 x 64 tiles 18.5 (57).
 #include "device_common.h"
 #include "ops.h"
 
@@ -35,17 +46,10 @@ typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 typedef __attribute__((address_space(3))) char lds_char;
 
-constexpr int kThreads = 256;
-constexpr int kTileRows = 128;
-constexpr int kStep = 32;       // k per step: four 16-byte chunks of 16-bit values per row
-// Stage buffers: 128-column tiles keep two (64 KB, two blocks a CU), 64-column
-// tiles four (112 KB for bf16, one block a CU): at 1500 rows the 128-column
-// products ran 70 us a launch with two stages against 96 with four, the
-// 64-column ones 72 with four against 84 with two.
-template <int TN>
-constexpr int kStages = TN == 128 ? 2 : 4;
+constexpr int kStep = 64;             // k per step: eight 16-byte chunks of 16-bit values per row
+constexpr int kChunks = kStep / 8;
+constexpr int kLoadRows = 1024 / (2 * kStep); // tile rows one wave load (1 KB) covers
 constexpr int kSplitThreads = 256;
-constexpr int kWaveRows = 4; // waves along the tile's rows (the rest along its columns)
 
 template <int WT>
 constexpr int parts_of()
@@ -187,70 +191,70 @@ __device__ __forceinline__ void wait_loads()
 // Slot of chunk c of tile row r (16-byte slots).
 __device__ __forceinline__ int slot(int r, int c)
 {
-    return 4 * r + (c ^ ((r >> 1) & 3));
+    return kChunks * r + (c ^ (r & 7));
 }
 
-template <int WT, int TN>
-struct Layout
+// WM x WN waves, each TM / WM rows by TN / WN columns; S stage buffers.
+template <int WT, int TM_, int TN_, int WM_, int WN_, int S_>
+struct Tile
 {
     static constexpr int P = parts_of<WT>();
-    static constexpr int kABytes = kTileRows * kStep * 2;          // one part's tile
+    static constexpr int TM = TM_, TN = TN_, WM = WM_, WN = WN_, S = S_;
+    static constexpr int kWaves = WM * WN;
+    static constexpr int kABytes = TM * kStep * 2; // one part's rows
     static constexpr int kStageBytes = P * kABytes + TN * kStep * 2;
-    static constexpr int kLoads = (P * kTileRows + TN) / 16;       // wave loads (1 KB each) per stage
-    static_assert(kLoads % 4 == 0, "whole loads per wave");
-    static constexpr int kPerWave = kLoads / 4;
-    static constexpr int kStages = wsp::ops::kStages<TN>;
+    static constexpr int kLoads = (P * TM + TN) / kLoadRows;
+    static_assert(kLoads % kWaves == 0, "whole loads per wave");
+    static constexpr int kPerWave = kLoads / kWaves;
+    static constexpr int MT = TM / 16 / WM, NT = TN / 16 / WN;
+    static_assert(S * kStageBytes <= 160 * 1024, "the stages fit the LDS");
 };
 
-template <int WT, int TN>
-__global__ void __launch_bounds__(kThreads) split_product_kernel(SplitProduct a)
+template <class T, int WT>
+__global__ void __launch_bounds__(T::kWaves * kWave) split_product_kernel(SplitProduct a)
 {
-    using L = Layout<WT, TN>;
-    constexpr int P = L::P;
-    constexpr int WM = kWaveRows, WN = 4 / WM;   // the waves' grid over the tile
-    constexpr int MT = kTileRows / 16 / WM;     // 16-row tiles per wave
-    constexpr int NT = TN / 16 / WN;            // 16-column tiles per wave
+    constexpr int P = T::P, MT = T::MT, NT = T::NT;
     extern __shared__ __attribute__((aligned(16))) unsigned char stage_mem[];
 
     const int tid = threadIdx.x, lane = tid % kWave;
     const int wave = __builtin_amdgcn_readfirstlane(tid / kWave); // uniform, so the load bases are scalar
     const int li = lane % 16, g = lane / 16;
-    const int wm = wave / WN, wn = wave % WN;
-    const int n_block = blockIdx.x * TN, m_block = blockIdx.y * kTileRows;
+    const int wm = wave / T::WN, wn = wave % T::WN;
+    const int n_block = blockIdx.x * T::TN, m_block = blockIdx.y * T::TM;
     const int steps = a.inner / kStep;
     // The block's columns lie in one of the (up to three) matrices.
     const int seg = n_block < a.split ? 0 : n_block < a.split2 ? 1 : 2;
     const int seg_first = seg == 0 ? 0 : seg == 1 ? a.split : a.split2;
     const void* w = seg == 0 ? a.w0 : seg == 1 ? a.w1 : a.w2;
 
-    // This wave's loads: load q = wave + 4 t of a stage covers 16 tile rows
-    // (parts' rows first, then W's); lane i moves row 16 q' + i / 4, chunk
-    // (i % 4) ^ ((row >> 1) & 3), so it lands in that chunk's slot.
-    const void* src[L::kPerWave];
-    uint32_t offset[L::kPerWave];
-    uint32_t dst[L::kPerWave]; // byte offset in the stage
+    // This wave's loads: load q = wave + waves·t of a stage covers 8 tile rows
+    // (the parts' rows first, then W's); lane i moves row 8 q' + i / 8, chunk
+    // (i % 8) ^ (row & 7), so it lands in that chunk's slot.
+    const void* src[T::kPerWave];
+    uint32_t offset[T::kPerWave];
+    uint32_t dst[T::kPerWave]; // byte offset in the stage
 #pragma unroll
-    for (int t = 0; t < L::kPerWave; ++t)
+    for (int t = 0; t < T::kPerWave; ++t)
     {
-        const int q = wave + 4 * t;
-        const int r = 16 * (q % (kTileRows / 16)) + lane / 4; // row within its tile (parts: 128 rows)
-        if (q < P * (kTileRows / 16))
+        const int q = wave + T::kWaves * t;
+        if (q < P * T::TM / kLoadRows)
         {
-            const int p = q / (kTileRows / 16);
+            const int p = q / (T::TM / kLoadRows), rq = q % (T::TM / kLoadRows);
+            const int r = kLoadRows * rq + lane / kChunks;
             const int row = min(m_block + r, a.rows - 1);
-            const int c = (lane % 4) ^ ((r >> 1) & 3);
+            const int c = (lane % kChunks) ^ (r & 7);
             src[t] = a.parts;
             offset[t] = (uint32_t) (((size_t) p * a.part_stride + (size_t) row * a.inner + 8 * c) * 2);
-            dst[t] = p * L::kABytes + 1024 * (q % (kTileRows / 16));
+            dst[t] = p * T::kABytes + 1024 * rq;
         }
         else
         {
-            const int wq = q - P * (kTileRows / 16);
-            const int col = 16 * wq + lane / 4;
-            const int c = (lane % 4) ^ ((col >> 1) & 3);
+            const int wq = q - P * T::TM / kLoadRows;
+            const int col = kLoadRows * wq + lane / kChunks;
+            const int c = (lane % kChunks) ^ (col & 7);
             src[t] = w;
             offset[t] = (uint32_t) (((size_t) (n_block - seg_first + col) * a.inner + 8 * c) * 2);
-            dst[t] = P * L::kABytes + 1024 * wq;
+            dst[t] = P * T::kABytes + 1024 * wq;
         }
     }
     const uint32_t stage0 = lds_address(stage_mem);
@@ -259,9 +263,9 @@ __global__ void __launch_bounds__(kThreads) split_product_kernel(SplitProduct a)
     auto issue = [&](int step, int buf) {
         const uint32_t k_bytes = (uint32_t) min(step, steps - 1) * (kStep * 2);
 #pragma unroll
-        for (int t = 0; t < L::kPerWave; ++t)
+        for (int t = 0; t < T::kPerWave; ++t)
             load_lds16(src[t], offset[t] + k_bytes,
-                       __builtin_amdgcn_readfirstlane(stage0 + buf * L::kStageBytes + dst[t]));
+                       __builtin_amdgcn_readfirstlane(stage0 + buf * T::kStageBytes + dst[t]));
     };
 
     float4v acc[MT][NT];
@@ -272,39 +276,44 @@ __global__ void __launch_bounds__(kThreads) split_product_kernel(SplitProduct a)
             acc[i][j] = float4v {0.f, 0.f, 0.f, 0.f};
 
 #pragma unroll
-    for (int s = 0; s < L::kStages - 1; ++s)
+    for (int s = 0; s < T::S - 1; ++s)
         issue(s, s);
     int buf = 0;
     for (int s = 0; s < steps; ++s)
     {
-        // This wave's loads of step s are done once at most the later
-        // kStages - 2 steps' loads are in flight; the barrier then makes every
-        // wave's loads visible and ends every read of the buffer refilled next.
-        wait_loads<(L::kStages - 2) * L::kPerWave>();
+        // This wave's loads of step s are done once at most the later S - 2
+        // steps' loads are in flight; the barrier then makes every wave's
+        // loads visible and ends every read of the buffer refilled next.
+        wait_loads<(T::S - 2) * T::kPerWave>();
         __syncthreads();
-        issue(s + L::kStages - 1, buf == 0 ? L::kStages - 1 : buf - 1);
-        const unsigned char* st = stage_mem + buf * L::kStageBytes;
-        u32x4 af[MT][P], bf[NT];
+        issue(s + T::S - 1, buf == 0 ? T::S - 1 : buf - 1);
+        const unsigned char* st = stage_mem + buf * T::kStageBytes;
 #pragma unroll
-        for (int mt = 0; mt < MT; ++mt)
+        for (int kk = 0; kk < kStep / 32; ++kk)
+        {
+            const int c = 4 * kk + g;
+            u32x4 af[MT][P], bf[NT];
 #pragma unroll
-            for (int p = 0; p < P; ++p)
-                af[mt][p] = reinterpret_cast<const u32x4*>(st + p * L::kABytes)[slot(16 * (MT * wm + mt) + li, g)];
-#pragma unroll
-        for (int nt = 0; nt < NT; ++nt)
-            bf[nt] = reinterpret_cast<const u32x4*>(st + P * L::kABytes)[slot(16 * (NT * wn + nt) + li, g)];
-#pragma unroll
-        for (int mt = 0; mt < MT; ++mt)
-#pragma unroll
-            for (int nt = 0; nt < NT; ++nt)
+            for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
                 for (int p = 0; p < P; ++p)
-                    acc[mt][nt] = mfma16<WT>(af[mt][p], bf[nt], acc[mt][nt]);
-        buf = buf == L::kStages - 1 ? 0 : buf + 1;
+                    af[mt][p] = reinterpret_cast<const u32x4*>(st + p * T::kABytes)[slot(16 * (MT * wm + mt) + li, c)];
+#pragma unroll
+            for (int nt = 0; nt < NT; ++nt)
+                bf[nt] = reinterpret_cast<const u32x4*>(st + P * T::kABytes)[slot(16 * (NT * wn + nt) + li, c)];
+#pragma unroll
+            for (int p = 0; p < P; ++p)
+#pragma unroll
+                for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+                    for (int nt = 0; nt < NT; ++nt)
+                        acc[mt][nt] = mfma16<WT>(bf[nt], af[mt][p], acc[mt][nt]);
+        }
+        buf = buf == T::S - 1 ? 0 : buf + 1;
     }
     wait_loads<0>();
 
-    // acc[mt][nt][r] of lane (g, li) is C[4g + r][li] of that 16 x 16 tile.
+    // acc[mt][nt][r] of lane (g, li) is row li, column 4g + r of that 16 x 16 tile.
     float* y = seg == 0 ? a.y0 : seg == 1 ? a.y1 : a.y2;
     const float* bias = seg == 0 ? a.bias0 : seg == 1 ? a.bias1 : a.bias2;
     const float scale = seg == 0 ? a.scale0 : seg == 1 ? a.scale1 : a.scale2;
@@ -312,55 +321,88 @@ __global__ void __launch_bounds__(kThreads) split_product_kernel(SplitProduct a)
 #pragma unroll
     for (int nt = 0; nt < NT; ++nt)
     {
-        const int c = n_block - seg_first + 16 * (NT * wn + nt) + li;
-        const float b = bias != nullptr ? bias[c] : 0.f;
+        const int c = n_block - seg_first + 16 * (NT * wn + nt) + 4 * g;
+        float b[4] = {0.f, 0.f, 0.f, 0.f};
+        if (bias != nullptr)
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+                b[r] = bias[c + r];
 #pragma unroll
         for (int mt = 0; mt < MT; ++mt)
+        {
+            const int row = m_block + 16 * (MT * wm + mt) + li;
+            if (row >= a.rows)
+                continue;
+            float v[4];
 #pragma unroll
             for (int r = 0; r < 4; ++r)
             {
-                const int row = m_block + 16 * (MT * wm + mt) + 4 * g + r;
-                if (row >= a.rows)
-                    continue;
-                float v = acc[mt][nt][r] * scale + b;
+                v[r] = acc[mt][nt][r] * scale + b[r];
                 if (a.flags & kProductGelu)
-                    v = exact_gelu(v);
-                if (a.out_parts != nullptr)
-                {
-                    uint32_t bits[3];
-                    split<WT>(v, bits);
-                    u16* o = static_cast<u16*>(a.out_parts) + (size_t) row * width + c;
-#pragma unroll
-                    for (int p = 0; p < P; ++p)
-                        o[p * a.out_part_stride] = (u16) bits[p];
-                }
-                else if ((seg == 1 && a.y1_halves != nullptr) || (seg == 2 && a.y2_halves_t != nullptr))
-                {
-                    const _Float16 hi = (_Float16) v;
-                    const _Float16 lo = (_Float16) (v - (float) hi);
-                    u16* o = seg == 1 ? static_cast<u16*>(a.y1_halves) + (size_t) row * width + c
-                                      : static_cast<u16*>(a.y2_halves_t) + (size_t) c * a.halves_pitch + row;
-                    o[0] = __builtin_bit_cast(u16, hi);
-                    o[(size_t) a.halves_pitch * width] = __builtin_bit_cast(u16, lo);
-                }
-                else if (a.flags & kProductResidual)
-                    y[(size_t) row * a.ldy + c] += v;
-                else
-                    y[(size_t) row * a.ldy + c] = v;
+                    v[r] = exact_gelu(v[r]);
             }
+            if (a.out_parts != nullptr)
+            {
+                uint32_t bits[4][3];
+#pragma unroll
+                for (int r = 0; r < 4; ++r)
+                    split<WT>(v[r], bits[r]);
+                u16* o = static_cast<u16*>(a.out_parts) + (size_t) row * width + c;
+#pragma unroll
+                for (int p = 0; p < P; ++p)
+                    *reinterpret_cast<uint2*>(o + p * a.out_part_stride)
+                        = uint2 {bits[0][p] | (bits[1][p] << 16), bits[2][p] | (bits[3][p] << 16)};
+            }
+            else if ((seg == 1 && a.y1_halves != nullptr) || (seg == 2 && a.y2_halves_t != nullptr))
+            {
+                uint32_t hi[4], lo[4];
+#pragma unroll
+                for (int r = 0; r < 4; ++r)
+                {
+                    const _Float16 h = (_Float16) v[r];
+                    hi[r] = __builtin_bit_cast(u16, h);
+                    lo[r] = __builtin_bit_cast(u16, (_Float16) (v[r] - (float) h));
+                }
+                const size_t part = (size_t) a.halves_pitch * width;
+                if (seg == 1)
+                {
+                    u16* o = static_cast<u16*>(a.y1_halves) + (size_t) row * width + c;
+                    *reinterpret_cast<uint2*>(o) = uint2 {hi[0] | (hi[1] << 16), hi[2] | (hi[3] << 16)};
+                    *reinterpret_cast<uint2*>(o + part) = uint2 {lo[0] | (lo[1] << 16), lo[2] | (lo[3] << 16)};
+                }
+                else
+                {
+                    u16* o = static_cast<u16*>(a.y2_halves_t) + (size_t) c * a.halves_pitch + row;
+#pragma unroll
+                    for (int r = 0; r < 4; ++r)
+                    {
+                        o[(size_t) r * a.halves_pitch] = (u16) hi[r];
+                        o[(size_t) r * a.halves_pitch + part] = (u16) lo[r];
+                    }
+                }
+            }
+            else
+            {
+                float4v* o = reinterpret_cast<float4v*>(y + (size_t) row * a.ldy + c);
+                float4v sum = {v[0], v[1], v[2], v[3]};
+                if (a.flags & kProductResidual)
+                    sum = *o + sum;
+                *o = sum;
+            }
+        }
     }
 }
 
-template <int WT>
-hipError_t launch(hipStream_t stream, const SplitProduct& a, bool wide)
+template <class T, int WT>
+hipError_t launch(hipStream_t stream, const SplitProduct& a)
 {
-    const dim3 grid(a.out / (wide ? 128 : 64), (a.rows + kTileRows - 1) / kTileRows);
-    constexpr size_t wide_bytes = kStages<128> * Layout<WT, 128>::kStageBytes;
-    constexpr size_t narrow_bytes = kStages<64> * Layout<WT, 64>::kStageBytes;
-    if (wide)
-        hipLaunchKernelGGL((split_product_kernel<WT, 128>), grid, dim3(kThreads), wide_bytes, stream, a);
-    else
-        hipLaunchKernelGGL((split_product_kernel<WT, 64>), grid, dim3(kThreads), narrow_bytes, stream, a);
+    constexpr int bytes = T::S * T::kStageBytes;
+    static const hipError_t allowed = hipFuncSetAttribute(reinterpret_cast<const void*>(&split_product_kernel<T, WT>),
+                                                          hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
+    if (allowed != hipSuccess)
+        return allowed;
+    hipLaunchKernelGGL((split_product_kernel<T, WT>), dim3(a.out / T::TN, (a.rows + T::TM - 1) / T::TM),
+                       dim3(T::kWaves * kWave), bytes, stream, a);
     return hipGetLastError();
 }
 
@@ -376,11 +418,28 @@ int compute_units()
     return units;
 }
 
-template <int WT, int TN>
-hipError_t allow_stages()
+// The largest tile that still occupies half the CUs (the bytes a product moves
+// into LDS fall with the tile's extents, but a launch of fewer blocks leaves
+// CUs idle for all of it): 128 x 256, 64 x 128, 32 x 128, else 32 x 64. At 1500
+// rows 1536 -> 384 ran 9.8 us as 141 blocks of 32 x 128, 13.6 as 72 of 64 x 128
+// and 14.5 as 282 of 32 x 64; 768 -> 2304 17.3 as 432 of 64 x 128, 19.9 in 64 x
+// 64 and 23 as 108 of 128 x 256. With at most one 64 x 128 block a CU, four
+// stages hide the loads (5120 -> 1280: 45 us against 60 with two); with more,
+// two let the blocks share a CU (768 -> 2304: 17.3 against 19.6 with four).
+template <int WT>
+hipError_t launch_tiles(hipStream_t stream, const SplitProduct& a)
 {
-    return hipFuncSetAttribute(reinterpret_cast<const void*>(&split_product_kernel<WT, TN>),
-                               hipFuncAttributeMaxDynamicSharedMemorySize, kStages<TN> * Layout<WT, TN>::kStageBytes);
+    const long long units = compute_units();
+    auto blocks = [&](int tm, int tn) { return (long long) ((a.rows + tm - 1) / tm) * (a.out / tn); };
+    if (a.out % 256 == 0 && a.split % 256 == 0 && a.split2 % 256 == 0 && 2 * blocks(128, 256) >= units)
+        return launch<Tile<WT, 128, 256, 2, 4, 2>, WT>(stream, a);
+    if (blocks(64, 128) > units)
+        return launch<Tile<WT, 64, 128, 2, 4, 2>, WT>(stream, a);
+    if (2 * blocks(64, 128) >= units)
+        return launch<Tile<WT, 64, 128, 2, 4, 4>, WT>(stream, a);
+    if (2 * blocks(32, 128) >= units)
+        return launch<Tile<WT, 32, 128, 2, WT == kF16 ? 4 : 2, 4>, WT>(stream, a); // (bf16: 28 loads a stage)
+    return launch<Tile<WT, 32, 64, 2, 2, 4>, WT>(stream, a);
 }
 } // namespace
 
@@ -424,8 +483,6 @@ hipError_t layernorm_parts(hipStream_t stream, const float* x, const float* gamm
     return hipGetLastError();
 }
 
-// 128-column tiles unless they would leave more than an eighth of the CUs
-// idle (the 1280-column products at 1500 rows: 120 blocks), then 64.
 hipError_t split_product(hipStream_t stream, const SplitProduct& product)
 {
     SplitProduct a = product;
@@ -435,20 +492,6 @@ hipError_t split_product(hipStream_t stream, const SplitProduct& product)
         a.split = a.split2;
     if (!split_product_fits(a.wdtype, a.inner, a.out, a.split, a.split2))
         return hipErrorInvalidValue;
-    static const hipError_t allowed = [] {
-        hipError_t e = allow_stages<kF16, 128>();
-        if (e == hipSuccess)
-            e = allow_stages<kF16, 64>();
-        if (e == hipSuccess)
-            e = allow_stages<kBF16, 128>();
-        if (e == hipSuccess)
-            e = allow_stages<kBF16, 64>();
-        return e;
-    }();
-    if (allowed != hipSuccess)
-        return allowed;
-    const long long wide_blocks = (long long) (a.out / 128) * ((a.rows + kTileRows - 1) / kTileRows);
-    const bool wide = 8 * wide_blocks >= 7 * compute_units();
-    return a.wdtype == kF16 ? launch<kF16>(stream, a, wide) : launch<kBF16>(stream, a, wide);
+    return a.wdtype == kF16 ? launch_tiles<kF16>(stream, a) : launch_tiles<kBF16>(stream, a);
 }
 } // namespace wsp::ops
