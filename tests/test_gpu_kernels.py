@@ -70,6 +70,37 @@ def test_linear_matches_oracle(ctx, oracle, dtype, rows, inner, out, flags):
     assert worst_error(got, expected) <= 1e-5 + 2.4e-7 * inner
 
 
+@pytest.mark.parametrize("dtype", ["F32", "F16", "BF16"])
+@pytest.mark.parametrize("rows,inner,out", [
+    (5, 8, 1), (16, 776, 20), (17, 776, 19), (33, 1288, 260),   # few rows in fp32: part-filled chunks and tiles
+    (17, 32, 128), (31, 1056, 384),                             # few rows in 16-bit parts
+    (700, 36, 386), (1100, 400, 402), (3000, 204, 80),          # fp32 tiles of each size with a short last step
+    (300, 100, 1030), (33, 35, 70)])                            # widened through registers; scalar loads
+def test_linear_paths(ctx, dtype, rows, inner, out):
+    # Every product above four rows at the edges of its tiles, against float64;
+    # the bound is test_linear_matches_oracle's. A non-finite weight reaches
+    # its own column alone, as in fp32 multiply-adds.
+    from whispereacp_amd.decoder import stored_to_device
+    x = S.normal_values(rows * inner, 19, 1.0).reshape(rows, inner)
+    stored, w = weights(out, inner, dtype, 23)
+    bias = S.normal_values(out, 29, 0.1)
+    wdev, wdtype = stored_to_device(S.StoredTensor("w", dtype, (out, inner), stored))
+    y = dev(np.full((rows, out), np.nan, np.float32))
+    ctx.linear(dev(x), rows, inner, wdev, wdtype, dev(bias), y, out, 0)
+    sync()
+    expected = x.astype(np.float64) @ w.astype(np.float64).T + bias
+    assert worst_error(y.cpu().numpy(), expected) <= 1e-5 + 2.4e-7 * inner
+    column, bad = out // 2, wdev.reshape(out, inner)
+    bad[column, inner - 1] = float("inf") if dtype == "F32" else 0x7C00 if dtype == "F16" else 0x7F80
+    ctx.linear(dev(np.abs(x) + 0.5), rows, inner, bad, wdtype, dev(bias), y, out, 0)
+    sync()
+    got = y.cpu().numpy()
+    assert not np.any(np.isfinite(got[:, column])) and np.all(np.isfinite(np.delete(got, column, axis=1)))
+    parts = dtype != "F32" and rows > 16 and inner % 32 == 0 and out % 128 == 0  # (a zero part times inf is NaN)
+    if not parts:
+        assert np.all(got[:, column] == np.inf)
+
+
 def test_linear_without_bias(ctx, oracle):
     x = S.normal_values(2 * 64, 3, 1.0).reshape(2, 64)
     stored, w = weights(32, 64, "F32", 5)

@@ -746,7 +746,7 @@ int wsp_encoder_encode(wsp_encoder* e, const wsp_encoder_tensors* T, const float
             }
             status = ops::split_product(st, p);
         }
-        else if (positions > 16 && ops::tile_product_fits(wt, d, 3 * d, d, e->normed) && d % 128 == 0)
+        else
         {
             // q, k and v side by side in one launch: three times the blocks of one.
             ops::TileProduct p {};
@@ -767,11 +767,8 @@ int wsp_encoder_encode(wsp_encoder* e, const wsp_encoder_tensors* T, const float
             p.ldy = d;
             p.rows_per_group = positions;
             p.wdtype = wt;
-            status = ops::tile_product(st, p);
+            status = ops::product(st, p);
         }
-        else if ((status = ops::linear(st, e->normed, positions, d, L.q_w, wt, L.q_b, e->q, d, 0)) == hipSuccess
-                 && (status = ops::linear(st, e->normed, positions, d, L.k_w, wt, nullptr, e->k, d, 0)) == hipSuccess)
-            status = ops::linear(st, e->normed, positions, d, L.v_w, wt, L.v_b, e->v, d, 0);
         if (status != hipSuccess)
             return encoder_hip(e, status, "self-attention projections");
         if (d / heads == kFlashWidth && d % 4 == 0)

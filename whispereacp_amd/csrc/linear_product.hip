@@ -1,0 +1,528 @@
+// y = X·Wᵀ (bias, GELU, residual) for fp32 X in fp32 arithmetic on the matrix
+// cores, any weight storage and any extents, and the products of few rows
+// (Kernels/Linear.h:129-276, Kernels/SimdTiledMatMul.h:470-486).
+//
+// fp32_tile_kernel: many rows. v_mfma_f32_16x16x4_f32 multiplies and
+// accumulates in fp32 (the same inputs, products and range as fused
+// multiply-adds, twice their rate: 157 TFLOP/s against 79 without packed fp32
+// instructions). 32 x 64 tiles in 32-wide k-steps, operands widened on their
+// way through registers into two LDS buffers, so a step needs one barrier and
+// its loads are in flight over the previous step's products. LDS chunk c (four
+// k) of row r sits at slot 8r + (c ^ (r & 7)): the operand reads of eight rows
+// hit eight bank groups. It takes what split_product's direct-to-LDS loads
+// cannot: 16-bit weights to be widened (the 51865-column logits of 96 rows:
+// 90 us, 153 as 64 x 64 tiles of vector multiply-adds), rows that are not
+// whole 16-byte runs.
+//
+// row_product_kernel: few rows, where tiles over whole rows of K would leave
+// most CUs idle behind a long serial chain (96 x 768 x 768 was 18 blocks of 24
+// dependent steps, 28 us). A block takes a small tile and its eight waves
+// split K; operands go straight from memory into the matrix-core operand
+// registers (a lane's eight consecutive k; any assignment of k to lanes serves
+// as long as both operands share it), and the eight partial tiles are added in
+// wave order through LDS, so the result does not depend on timing. SPLIT takes
+// 16-bit weights in their own type with X cut into exact 16-bit parts (as
+// tile_product_kernel does), otherwise everything is fp32.
+//
+// W is the matrix cores' row operand, X their column operand: a lane ends up
+// with four consecutive outputs of one row.
+#include "device_common.h"
+#include "ops.h"
+
+namespace wsp::ops
+{
+namespace
+{
+typedef uint16_t u16;
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+
+// Output column n's matrix, and its column there.
+struct Column
+{
+    const void* w;
+    const float* bias;
+    float* y;
+    int c;
+};
+
+__device__ __forceinline__ Column column_of(const TileProduct& a, int n)
+{
+    if (n < a.split)
+        return {a.w0, a.bias0, a.y0, n};
+    if (n < a.split2)
+        return {a.w1, a.bias1, a.y1, n - a.split};
+    return {a.w2, a.bias2, a.y2, n - a.split2};
+}
+
+__device__ __forceinline__ void store_output(const TileProduct& a, int row, int n, float v)
+{
+    const Column col = column_of(a, n);
+    if (col.bias != nullptr)
+        v += col.bias[col.c];
+    if (a.flags & 1)
+        v = exact_gelu(v);
+    float* dst = col.y + (size_t) (row / a.rows_per_group) * a.group_stride + (size_t) (row % a.rows_per_group) * a.ldy
+                 + col.c;
+    if (a.flags & 2)
+        v += *dst;
+    *dst = v;
+}
+
+// COUNT consecutive values of a row from element `index` on, as loaded: kept
+// raw until values() so that nothing waits for the load before its use. Past
+// the row's end (`left` elements from `index` on) they read as zero. VEC:
+// 16-byte loads (8 for four 16-bit values), the row's end a multiple of COUNT;
+// a run past it loads the matrix's first values instead.
+template <int WT, int COUNT, bool VEC>
+struct Run
+{
+    static constexpr int kWords = WT == kF32 || !VEC ? COUNT : COUNT / 2;
+    uint32_t raw[kWords];
+
+    __device__ __forceinline__ void load(const void* base, size_t index, int left)
+    {
+        if constexpr (VEC)
+        {
+            const size_t at = left > 0 ? index : 0;
+            constexpr int kPiece = kWords >= 4 ? 4 : 2;
+            typedef uint32_t piece __attribute__((ext_vector_type(kPiece)));
+            const piece* p = reinterpret_cast<const piece*>(static_cast<const char*>(base) + at * (WT == kF32 ? 4 : 2));
+#pragma unroll
+            for (int i = 0; i < kWords / kPiece; ++i)
+            {
+                const piece v = p[i];
+#pragma unroll
+                for (int j = 0; j < kPiece; ++j)
+                    raw[kPiece * i + j] = v[j];
+            }
+        }
+        else
+#pragma unroll
+            for (int i = 0; i < COUNT; ++i)
+                raw[i] = __float_as_uint(i < left ? load1<WT>(base, index + i) : 0.f);
+    }
+
+    __device__ __forceinline__ void values(float (&v)[COUNT], int left) const
+    {
+#pragma unroll
+        for (int i = 0; i < COUNT; ++i)
+        {
+            if constexpr (WT == kF32 || !VEC)
+                v[i] = __uint_as_float(raw[i]);
+            else
+            {
+                const u16 h = (u16) (raw[i / 2] >> (16 * (i % 2)));
+                v[i] = WT == kF16 ? (float) __builtin_bit_cast(_Float16, h) : bf16_to_float(h);
+            }
+            if (VEC)
+                v[i] = left > 0 ? v[i] : 0.f;
+        }
+    }
+};
+
+// ---------------------------------------------------------------------------
+// Many rows
+// ---------------------------------------------------------------------------
+constexpr int kTileThreads = 256;
+constexpr int kTileRows = 32, kTileColumns = 64;
+constexpr int kTileStep = 32;
+
+// Slot of chunk c (four k) of LDS row r.
+__device__ __forceinline__ int slot(int r, int c)
+{
+    return 8 * r + (c ^ (r & 7));
+}
+
+template <int WT, bool VEC>
+__global__ void __launch_bounds__(kTileThreads, 2) fp32_tile_kernel(TileProduct a)
+{
+    constexpr int TM = kTileRows, TN = kTileColumns, KS = kTileStep, CH = KS / 4;
+    constexpr int MT = TM / 32, NT = TN / 32; // 16 x 16 tiles a wave, waves 2 x 2
+    constexpr int RP = kTileThreads / CH;     // rows staged at a time
+    constexpr int XC = TM / RP, WC = TN / RP; // chunks a thread stages per step
+    __shared__ float4v xs[2][TM * CH], ws[2][TN * CH];
+
+    const int tid = threadIdx.x, wave = tid / kWave, lane = tid % kWave, li = lane % 16, g = lane / 16;
+    const int wm = wave / 2, wn = wave % 2;
+    const int m_block = blockIdx.y * TM, n_block = blockIdx.x * TN;
+    const int sc = tid % CH, sr = tid / CH; // this thread's chunk of rows sr, sr + RP, ...
+
+    // Rows and columns past the end re-read the last one; their outputs are
+    // not stored.
+    size_t x_at[XC], w_at[WC];
+    const void* w_base[WC];
+#pragma unroll
+    for (int j = 0; j < XC; ++j)
+        x_at[j] = (size_t) min(m_block + sr + RP * j, a.rows - 1) * a.inner;
+#pragma unroll
+    for (int j = 0; j < WC; ++j)
+    {
+        const Column col = column_of(a, min(n_block + sr + RP * j, a.out - 1));
+        w_base[j] = col.w;
+        w_at[j] = (size_t) col.c * a.inner;
+    }
+    Run<kF32, 4, VEC> xr[XC];
+    Run<WT, 4, VEC> wr[WC];
+    auto fetch = [&](int k0) {
+        const int k = k0 + 4 * sc;
+#pragma unroll
+        for (int j = 0; j < XC; ++j)
+            xr[j].load(a.x, x_at[j] + k, a.inner - k);
+#pragma unroll
+        for (int j = 0; j < WC; ++j)
+            wr[j].load(w_base[j], w_at[j] + k, a.inner - k);
+    };
+    auto stage = [&](int buf, int k0) {
+        const int left = a.inner - k0 - 4 * sc;
+        float v[4];
+#pragma unroll
+        for (int j = 0; j < XC; ++j)
+        {
+            xr[j].values(v, left);
+            xs[buf][slot(sr + RP * j, sc)] = float4v {v[0], v[1], v[2], v[3]};
+        }
+#pragma unroll
+        for (int j = 0; j < WC; ++j)
+        {
+            wr[j].values(v, left);
+            ws[buf][slot(sr + RP * j, sc)] = float4v {v[0], v[1], v[2], v[3]};
+        }
+    };
+
+    float4v acc[MT][NT];
+#pragma unroll
+    for (int i = 0; i < MT; ++i)
+#pragma unroll
+        for (int j = 0; j < NT; ++j)
+            acc[i][j] = float4v {0.f, 0.f, 0.f, 0.f};
+
+    fetch(0);
+    stage(0, 0);
+    __syncthreads();
+    int buf = 0;
+    for (int k0 = 0; k0 < a.inner; k0 += KS)
+    {
+        const bool more = k0 + KS < a.inner;
+        if (more)
+            fetch(k0 + KS);
+        float4v xf[2][MT], wf[2][NT];
+        auto operands = [&](int kk, int set) {
+#pragma unroll
+            for (int mt = 0; mt < MT; ++mt)
+                xf[set][mt] = xs[buf][slot(16 * (MT * wm + mt) + li, 4 * kk + g)];
+#pragma unroll
+            for (int nt = 0; nt < NT; ++nt)
+                wf[set][nt] = ws[buf][slot(16 * (NT * wn + nt) + li, 4 * kk + g)];
+        };
+        operands(0, 0);
+#pragma unroll
+        for (int kk = 0; kk < KS / 16; ++kk)
+        {
+            if (kk + 1 < KS / 16)
+                operands(kk + 1, (kk + 1) % 2);
+            __builtin_amdgcn_sched_barrier(0); // the next operands' reads stay ahead of these products
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+#pragma unroll
+                for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+                    for (int nt = 0; nt < NT; ++nt)
+                        acc[mt][nt] = __builtin_amdgcn_mfma_f32_16x16x4f32(wf[kk % 2][nt][e], xf[kk % 2][mt][e],
+                                                                            acc[mt][nt], 0, 0, 0);
+        }
+        if (more)
+            stage(buf ^ 1, k0 + KS); // last read before the previous step's barrier
+        __syncthreads();
+        buf ^= 1;
+    }
+
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt)
+    {
+        const int row = m_block + 16 * (MT * wm + mt) + li;
+        if (row >= a.rows)
+            continue;
+#pragma unroll
+        for (int nt = 0; nt < NT; ++nt)
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+            {
+                const int n = n_block + 16 * (NT * wn + nt) + 4 * g + r;
+                if (n < a.out)
+                    store_output(a, row, n, acc[mt][nt][r]);
+            }
+    }
+}
+
+// ---------------------------------------------------------------------------
+// Few rows
+// ---------------------------------------------------------------------------
+constexpr int kRowWaves = 8;
+constexpr int kRowChunk = 32; // k a wave takes at a time
+
+template <int WT>
+__device__ __forceinline__ float4v mfma16(u32x4 a, u32x4 b, float4v c)
+{
+    if constexpr (WT == kF16)
+        return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(half8, a), __builtin_bit_cast(half8, b), c, 0,
+                                                       0, 0);
+    else
+        return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c,
+                                                        0, 0, 0);
+}
+
+// One chunk's operands of a lane: eight k of MT rows and NT columns.
+template <int WT, int MT, int NT>
+struct RowChunk
+{
+    Run<kF32, 8, true> x[MT];
+    Run<WT, 8, true> w[NT];
+};
+
+template <int WT, int MT, int NT, bool SPLIT>
+__global__ void __launch_bounds__(kRowWaves * kWave) row_product_kernel(TileProduct a)
+{
+    static_assert(!SPLIT || WT != kF32, "parts go with 16-bit weights");
+    constexpr int P = WT == kF16 ? 2 : 3;
+    // Interleaved sums per tile: shorter chains of dependent products (a single
+    // one issues every 46 clocks instead of 32) and of roundings. With parts,
+    // the first part and the smaller ones are summed apart.
+    constexpr int SETS = SPLIT ? 2 : MT * NT >= 4 ? 1 : 4 / (MT * NT);
+    __shared__ float4v sums[kRowWaves][MT * NT][kWave];
+
+    const int tid = threadIdx.x, lane = tid % kWave, li = lane % 16, g = lane / 16;
+    const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
+    const int m_block = blockIdx.y * 16 * MT, n_block = blockIdx.x * 16 * NT;
+
+    size_t x_at[MT], w_at[NT];
+    const void* w_base[NT];
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt)
+        x_at[mt] = (size_t) min(m_block + 16 * mt + li, a.rows - 1) * a.inner;
+#pragma unroll
+    for (int nt = 0; nt < NT; ++nt)
+    {
+        const Column col = column_of(a, min(n_block + 16 * nt + li, a.out - 1));
+        w_base[nt] = col.w;
+        w_at[nt] = (size_t) col.c * a.inner;
+    }
+    float4v acc[SETS][MT][NT];
+#pragma unroll
+    for (int i = 0; i < SETS; ++i)
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+            for (int nt = 0; nt < NT; ++nt)
+                acc[i][mt][nt] = float4v {0.f, 0.f, 0.f, 0.f};
+
+    using Chunk = RowChunk<WT, MT, NT>;
+    auto load = [&](Chunk& ch, int chunk) {
+        const int k = kRowChunk * chunk + 8 * g, left = a.inner - k;
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt)
+            ch.x[mt].load(a.x, x_at[mt] + k, left);
+#pragma unroll
+        for (int nt = 0; nt < NT; ++nt)
+            ch.w[nt].load(w_base[nt], w_at[nt] + k, left);
+    };
+    auto multiply = [&](const Chunk& ch, int chunk) {
+        const int left = a.inner - kRowChunk * chunk - 8 * g;
+        float x[MT][8];
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt)
+            ch.x[mt].values(x[mt], left);
+        if constexpr (SPLIT) // (whole chunks: left is never short)
+        {
+            u32x4 xb[MT][3], wb[NT];
+#pragma unroll
+            for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+                for (int j = 0; j < 4; ++j)
+                {
+                    uint32_t b0[3], b1[3];
+                    exact_parts<WT>(x[mt][2 * j], b0);
+                    exact_parts<WT>(x[mt][2 * j + 1], b1);
+#pragma unroll
+                    for (int p = 0; p < 3; ++p)
+                        xb[mt][p][j] = b0[p] | (b1[p] << 16);
+                }
+#pragma unroll
+            for (int nt = 0; nt < NT; ++nt)
+                wb[nt] = u32x4 {ch.w[nt].raw[0], ch.w[nt].raw[1], ch.w[nt].raw[2], ch.w[nt].raw[3]};
+#pragma unroll
+            for (int p = 0; p < P; ++p)
+#pragma unroll
+                for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+                    for (int nt = 0; nt < NT; ++nt)
+                        {
+                        float4v& sum = acc[p == 0 ? 0 : 1][mt][nt];
+                        sum = mfma16<WT>(wb[nt], xb[mt][p], sum);
+                    }
+        }
+        else
+        {
+            float w[NT][8];
+#pragma unroll
+            for (int nt = 0; nt < NT; ++nt)
+                ch.w[nt].values(w[nt], left);
+#pragma unroll
+            for (int e = 0; e < 8; ++e)
+#pragma unroll
+                for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+                    for (int nt = 0; nt < NT; ++nt)
+                    {
+                        float4v& sum = acc[e % SETS][mt][nt];
+                        sum = __builtin_amdgcn_mfma_f32_16x16x4f32(w[nt][e], x[mt][e], sum, 0, 0, 0);
+                    }
+        }
+    };
+    // Chunks wave, wave + 8, ..., the next one's loads ahead of this one's products.
+    const int chunks = (a.inner + kRowChunk - 1) / kRowChunk;
+    Chunk c0, c1;
+    if (wave < chunks)
+        load(c0, wave);
+    for (int chunk = wave; chunk < chunks; chunk += 2 * kRowWaves)
+    {
+        const bool second = chunk + kRowWaves < chunks;
+        if (second)
+            load(c1, chunk + kRowWaves);
+        multiply(c0, chunk);
+        if (!second)
+            break;
+        if (chunk + 2 * kRowWaves < chunks)
+            load(c0, chunk + 2 * kRowWaves);
+        multiply(c1, chunk + kRowWaves);
+    }
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+        for (int nt = 0; nt < NT; ++nt)
+        {
+            float4v total = acc[SETS - 1][mt][nt];
+#pragma unroll
+            for (int i = SETS - 2; i >= 0; --i)
+                total += acc[i][mt][nt];
+            sums[wave][mt * NT + nt][lane] = total;
+        }
+    __syncthreads();
+    // Consecutive threads take consecutive columns of a row.
+    constexpr int kOutputs = MT * NT * 256;
+#pragma unroll
+    for (int i = 0; i < (kOutputs + kRowWaves * kWave - 1) / (kRowWaves * kWave); ++i)
+    {
+        const int at = tid + i * kRowWaves * kWave;
+        if (at >= kOutputs)
+            break;
+        const int n = at % (16 * NT), m = at / (16 * NT);
+        const int tile = m / 16 * NT + n / 16, from = m % 16 + 16 * (n % 16 / 4);
+        float v = 0.f;
+#pragma unroll
+        for (int w = 0; w < kRowWaves; ++w)
+            v += reinterpret_cast<const float*>(&sums[w][tile][from])[n % 4];
+        if (m_block + m < a.rows && n_block + n < a.out)
+            store_output(a, m_block + m, n_block + n, v);
+    }
+}
+
+int compute_units()
+{
+    static const int units = [] {
+        int device = 0, count = 0;
+        if (hipGetDevice(&device) == hipSuccess
+            && hipDeviceGetAttribute(&count, hipDeviceAttributeMultiprocessorCount, device) == hipSuccess && count > 0)
+            return count;
+        return 256;
+    }();
+    return units;
+}
+
+bool aligned(const void* p, size_t bytes)
+{
+    return reinterpret_cast<uintptr_t>(p) % bytes == 0;
+}
+
+// Whether X and every matrix take whole vector loads of `run` values.
+bool whole_vectors(const TileProduct& a, int run)
+{
+    const size_t bytes = a.wdtype == kF32 ? 16 : 2 * run;
+    return a.inner % run == 0 && aligned(a.x, 16) && aligned(a.w0, bytes) && (a.split >= a.out || aligned(a.w1, bytes))
+           && (a.split2 >= a.out || aligned(a.w2, bytes));
+}
+
+template <int WT, bool VEC>
+hipError_t launch_tile(hipStream_t stream, const TileProduct& a)
+{
+    hipLaunchKernelGGL((fp32_tile_kernel<WT, VEC>), dim3((a.out + kTileColumns - 1) / kTileColumns,
+                                                         (a.rows + kTileRows - 1) / kTileRows),
+                       dim3(kTileThreads), 0, stream, a);
+    return hipGetLastError();
+}
+
+template <int WT, int MT, int NT, bool SPLIT>
+hipError_t launch_row(hipStream_t stream, const TileProduct& a)
+{
+    hipLaunchKernelGGL((row_product_kernel<WT, MT, NT, SPLIT>),
+                       dim3((a.out + 16 * NT - 1) / (16 * NT), (a.rows + 16 * MT - 1) / (16 * MT)),
+                       dim3(kRowWaves * kWave), 0, stream, a);
+    return hipGetLastError();
+}
+
+// 16-bit weights with X in 16-bit parts: short products by row_product_kernel,
+// the others by tile_product. The line is at 2^17 outputs: 96 x 768 -> 768 ran
+// 5.3 us against 13.5 for tile_product, 96 x 3072 -> 768 13.2 against 41,
+// 200 x 1280 -> 5120 41 against 23.
+template <int WT>
+hipError_t parts_product(hipStream_t stream, const TileProduct& a)
+{
+    return (long long) a.rows * a.out <= 1 << 17 ? launch_row<WT, 1, 2, true>(stream, a) : tile_product(stream, a);
+}
+
+// fp32 arithmetic. Up to 16 rows, and while 32 x 32 tiles would not give each
+// CU one, row_product_kernel: 96 x 3072 -> 768 ran 19 us against 36 in such
+// tiles, 200 x 1280 -> 1280 (280 tiles) 20 against 17.6. fp32 weights
+// otherwise take split_product's direct-to-LDS form (1500 x 2048 -> 512 35 us
+// against 48 staged through registers), the rest fp32_tile_kernel.
+template <int WT>
+hipError_t fp32_product(hipStream_t stream, const TileProduct& a)
+{
+    const long long units = compute_units();
+    auto blocks = [&](int tm, int tn) { return (long long) ((a.rows + tm - 1) / tm) * ((a.out + tn - 1) / tn); };
+    if ((a.rows <= kSplitRowLimit || blocks(32, 32) < units) && whole_vectors(a, 8))
+    {
+        if (a.rows > 16)
+            return launch_row<WT, 2, 1, false>(stream, a);
+        // (16 x 1280 -> 5120: 9.8 us with 32 columns a block, 11.3 with 16; 8 x 768 -> 3072: 6.1 and 4.4)
+        return blocks(16, 16) > units ? launch_row<WT, 1, 2, false>(stream, a)
+                                      : launch_row<WT, 1, 1, false>(stream, a);
+    }
+    if (WT == kF32 && fp32_split_fits(a))
+        return fp32_split(stream, a);
+    return whole_vectors(a, 4) ? launch_tile<WT, true>(stream, a) : launch_tile<WT, false>(stream, a);
+}
+} // namespace
+
+bool row_product_fits(const TileProduct& product)
+{
+    return product.rows <= kSplitRowLimit && whole_vectors(product, 8);
+}
+
+hipError_t product(hipStream_t stream, const TileProduct& given)
+{
+    TileProduct a = given;
+    if (a.split2 <= 0 || a.split2 > a.out)
+        a.split2 = a.out;
+    if (a.split <= 0 || a.split > a.split2)
+        a.split = a.split2;
+    const bool parts = a.rows > kSplitRowLimit && tile_product_fits(a.wdtype, a.inner, a.out, a.split, a.x)
+                       && a.split2 % 128 == 0;
+    switch (a.wdtype)
+    {
+        case kF32: return fp32_product<kF32>(stream, a);
+        case kF16: return parts ? parts_product<kF16>(stream, a) : fp32_product<kF16>(stream, a);
+        default: return parts ? parts_product<kBF16>(stream, a) : fp32_product<kBF16>(stream, a);
+    }
+}
+} // namespace wsp::ops

@@ -47,6 +47,15 @@ struct TileProduct
     int split2;
 };
 
+// y = X·Wᵀ for any rows, extents and weight storage (linear_product.hip): what
+// tile_product fits, in its arithmetic (16-bit parts), else in fp32.
+hipError_t product(hipStream_t stream, const TileProduct& product);
+// Whether a product of at most kSplitRowLimit rows goes there in one launch.
+bool row_product_fits(const TileProduct& product);
+// fp32 weights in whole 16-byte runs (split_product.hip).
+bool fp32_split_fits(const TileProduct& product);
+hipError_t fp32_split(hipStream_t stream, const TileProduct& product);
+
 // 16-bit weights, inner % 32 == 0, out and split (and split2) multiples of
 // 128, X 16-byte aligned.
 bool tile_product_fits(int wdtype, int inner, int out, int split, const void* x);

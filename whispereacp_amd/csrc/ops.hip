@@ -119,171 +119,6 @@ __global__ void __launch_bounds__(kBlock) gemv_kernel(const float* __restrict__ 
 }
 
 // ---------------------------------------------------------------------------
-// Tiled product for many rows: 64x64 output tiles, 16-deep K slices staged in
-// LDS (weights widened to float on the way in), 4x4 outputs per thread, k
-// ascending within each thread's sum. Same epilogue as the GEMV. With VEC
-// (inner a multiple of 4, rows 16-byte aligned) each thread moves one row's
-// four consecutive k per operand per slice as one vector load, the next
-// slice's loads are in flight while the current one is multiplied, and the
-// fragments come out of LDS as float4 reads.
-// ---------------------------------------------------------------------------
-constexpr int kTile = 64;
-constexpr int kTileK = 16;
-
-// Four consecutive weights widened to float (VEC loads: 16 bytes for F32,
-// 8 for F16 and BF16).
-template <int WT>
-__device__ __forceinline__ float4v load4(const void* w, size_t index)
-{
-    if constexpr (WT == kF32)
-        return *reinterpret_cast<const float4v*>(static_cast<const float*>(w) + index);
-    else
-    {
-        const uint2 u = *reinterpret_cast<const uint2*>(static_cast<const uint16_t*>(w) + index);
-        const uint16_t h[4] = {(uint16_t) u.x, (uint16_t) (u.x >> 16), (uint16_t) u.y, (uint16_t) (u.y >> 16)};
-        float4v v;
-#pragma unroll
-        for (int i = 0; i < 4; ++i)
-        {
-            if constexpr (WT == kF16)
-                v[i] = (float) __builtin_bit_cast(_Float16, h[i]);
-            else
-                v[i] = bf16_to_float(h[i]);
-        }
-        return v;
-    }
-}
-
-// TM rows by 64 columns a block: RT = TM / 16 rows by 4 columns a thread
-// (TM 32, VEC only, when 64-row blocks leave CUs idle).
-template <int WT, bool VEC, int TM>
-__global__ void __launch_bounds__(kBlock) gemm_kernel(const float* __restrict__ x, int rows,
-                                                      int inner, const void* __restrict__ w,
-                                                      const float* __restrict__ bias,
-                                                      float* __restrict__ y, int out, int flags)
-{
-    constexpr int RT = TM / 16;
-    static_assert(TM == kTile || (VEC && TM == 32), "32-row blocks take vector loads");
-    __shared__ __attribute__((aligned(16))) float xs[kTileK][kTile + 4];
-    __shared__ __attribute__((aligned(16))) float ws[kTileK][kTile + 4];
-
-    const int row0 = blockIdx.y * TM;
-    const int col0 = blockIdx.x * kTile;
-    const int tx = threadIdx.x % 16, ty = threadIdx.x / 16;
-
-    float acc[RT][4] = {};
-
-    if constexpr (VEC)
-    {
-        // Thread t stages row (or weight row) t / 4, k = 4 (t % 4) .. + 3 of
-        // the slice.
-        const int sr = threadIdx.x / 4, sq = (threadIdx.x % 4) * 4;
-        const int gr = row0 + sr, gc = col0 + sr;
-        float4v xa = {0.f, 0.f, 0.f, 0.f}, wa = {0.f, 0.f, 0.f, 0.f};
-        auto fetch = [&](int k0) {
-            const int gk = k0 + sq;
-            xa = float4v {0.f, 0.f, 0.f, 0.f};
-            wa = float4v {0.f, 0.f, 0.f, 0.f};
-            if (sr < TM && gr < rows && gk < inner)
-                xa = *reinterpret_cast<const float4v*>(x + (size_t) gr * inner + gk);
-            if (gc < out && gk < inner)
-                wa = load4<WT>(w, (size_t) gc * inner + gk);
-        };
-        fetch(0);
-        for (int k0 = 0; k0 < inner; k0 += kTileK)
-        {
-#pragma unroll
-            for (int i = 0; i < 4; ++i)
-            {
-                if (sr < TM)
-                    xs[sq + i][sr] = xa[i];
-                ws[sq + i][sr] = wa[i];
-            }
-            __syncthreads();
-            if (k0 + kTileK < inner)
-                fetch(k0 + kTileK);
-#pragma unroll
-            for (int kk = 0; kk < kTileK; ++kk)
-            {
-                float a[RT];
-                if constexpr (RT == 4)
-                {
-                    const float4v v = *reinterpret_cast<const float4v*>(&xs[kk][ty * 4]);
-                    a[0] = v[0]; a[1] = v[1]; a[2] = v[2]; a[3] = v[3];
-                }
-                else
-                {
-                    const float2 v = *reinterpret_cast<const float2*>(&xs[kk][ty * 2]);
-                    a[0] = v.x; a[1] = v.y;
-                }
-                const float4v b = *reinterpret_cast<const float4v*>(&ws[kk][tx * 4]);
-#pragma unroll
-                for (int i = 0; i < RT; ++i)
-#pragma unroll
-                    for (int j = 0; j < 4; ++j)
-                        acc[i][j] += a[i] * b[j];
-            }
-            __syncthreads();
-        }
-    }
-    else if constexpr (TM == kTile)
-        for (int k0 = 0; k0 < inner; k0 += kTileK)
-        {
-            // 64 x 16 of each operand: 1024 elements, 4 per thread.
-#pragma unroll
-            for (int i = 0; i < 4; ++i)
-            {
-                const int e = threadIdx.x + i * kBlock;
-                const int r = e / kTileK, kk = e % kTileK;
-                const int gk = k0 + kk;
-                const int gr = row0 + r, gc = col0 + r;
-                xs[kk][r] = (gr < rows && gk < inner) ? x[(size_t) gr * inner + gk] : 0.f;
-                ws[kk][r] = (gc < out && gk < inner) ? load1<WT>(w, (size_t) gc * inner + gk) : 0.f;
-            }
-            __syncthreads();
-#pragma unroll
-            for (int kk = 0; kk < kTileK; ++kk)
-            {
-                float a[4], b[4];
-#pragma unroll
-                for (int i = 0; i < 4; ++i)
-                {
-                    a[i] = xs[kk][ty * 4 + i];
-                    b[i] = ws[kk][tx * 4 + i];
-                }
-#pragma unroll
-                for (int i = 0; i < 4; ++i)
-#pragma unroll
-                    for (int j = 0; j < 4; ++j)
-                        acc[i][j] += a[i] * b[j];
-            }
-            __syncthreads();
-        }
-
-#pragma unroll
-    for (int i = 0; i < RT; ++i)
-    {
-        const int r = row0 + ty * RT + i;
-        if (r >= rows)
-            continue;
-#pragma unroll
-        for (int j = 0; j < 4; ++j)
-        {
-            const int c = col0 + tx * 4 + j;
-            if (c >= out)
-                continue;
-            float v = acc[i][j] + (bias != nullptr ? bias[c] : 0.f);
-            if (flags & 1)
-                v = exact_gelu(v);
-            float* dst = y + (size_t) r * out + c;
-            if (flags & 2)
-                v += *dst;
-            *dst = v;
-        }
-    }
-}
-
-// ---------------------------------------------------------------------------
 // LayerNorm: one block per row; mean, then the centred variance, then
 // (x - mean) * rsqrt(var + eps) * gamma + beta (Kernels/LayerNorm.h:44-89).
 // ---------------------------------------------------------------------------
@@ -760,68 +595,33 @@ hipError_t launch_gemv(hipStream_t stream, const float* x, int rows, int inner, 
     return hipSuccess;
 }
 
-template <int WT>
-hipError_t launch_gemm(hipStream_t stream, const float* x, int rows, int inner, const void* w,
-                       const float* bias, float* y, int out, int flags)
-{
-    const dim3 grid((out + kTile - 1) / kTile, (rows + kTile - 1) / kTile);
-    const size_t w_align = WT == kF32 ? 16 : 8;
-    const bool vec = inner % 4 == 0 && reinterpret_cast<uintptr_t>(x) % 16 == 0
-                     && reinterpret_cast<uintptr_t>(w) % w_align == 0;
-    static const int units = [] {
-        int device = 0, count = 0;
-        if (hipGetDevice(&device) == hipSuccess
-            && hipDeviceGetAttribute(&count, hipDeviceAttributeMultiprocessorCount, device) == hipSuccess && count > 0)
-            return count;
-        return 256;
-    }();
-    if (vec && (long long) grid.x * grid.y < units) // 32-row blocks: twice the blocks
-        hipLaunchKernelGGL((gemm_kernel<WT, true, 32>), dim3(grid.x, (rows + 31) / 32), dim3(kBlock), 0, stream, x,
-                           rows, inner, w, bias, y, out, flags);
-    else if (vec)
-        hipLaunchKernelGGL((gemm_kernel<WT, true, kTile>), grid, dim3(kBlock), 0, stream, x, rows, inner, w, bias, y,
-                           out, flags);
-    else
-        hipLaunchKernelGGL((gemm_kernel<WT, false, kTile>), grid, dim3(kBlock), 0, stream, x, rows, inner, w, bias, y,
-                           out, flags);
-    return hipGetLastError();
-}
 } // namespace
 
 hipError_t linear(hipStream_t stream, const float* x, int rows, int inner, const void* weight,
                   int wdtype, const float* bias, float* y, int out, int flags)
 {
-    if (rows <= kSplitRowLimit)
-    {
-        switch (wdtype)
-        {
-            case kF32: return launch_gemv<kF32>(stream, x, rows, inner, weight, bias, y, out, flags);
-            case kF16: return launch_gemv<kF16>(stream, x, rows, inner, weight, bias, y, out, flags);
-            default: return launch_gemv<kBF16>(stream, x, rows, inner, weight, bias, y, out, flags);
-        }
-    }
-    if (tile_product_fits(wdtype, inner, out, out, x))
-    {
-        TileProduct p {};
-        p.x = x;
-        p.rows = rows;
-        p.inner = inner;
-        p.w0 = p.w1 = weight;
-        p.split = p.out = out;
-        p.bias0 = p.bias1 = bias;
-        p.y0 = p.y1 = y;
-        p.ldy = out;
-        p.rows_per_group = rows;
-        p.group_stride = 0;
-        p.flags = flags;
-        p.wdtype = wdtype;
-        return tile_product(stream, p);
-    }
+    TileProduct p {};
+    p.x = x;
+    p.rows = rows;
+    p.inner = inner;
+    p.w0 = p.w1 = weight;
+    p.split = p.out = out;
+    p.bias0 = p.bias1 = bias;
+    p.y0 = p.y1 = y;
+    p.ldy = out;
+    p.rows_per_group = rows;
+    p.flags = flags;
+    p.wdtype = wdtype;
+    // Up to four rows the GEMV (a wave per output, one read of W); from five
+    // on it would read W again for every four rows (16 x 768 -> 3072: four
+    // launches of 4 us against one of 5).
+    if (rows > kSplitRowLimit || (rows > 4 && row_product_fits(p)))
+        return product(stream, p);
     switch (wdtype)
     {
-        case kF32: return launch_gemm<kF32>(stream, x, rows, inner, weight, bias, y, out, flags);
-        case kF16: return launch_gemm<kF16>(stream, x, rows, inner, weight, bias, y, out, flags);
-        default: return launch_gemm<kBF16>(stream, x, rows, inner, weight, bias, y, out, flags);
+        case kF32: return launch_gemv<kF32>(stream, x, rows, inner, weight, bias, y, out, flags);
+        case kF16: return launch_gemv<kF16>(stream, x, rows, inner, weight, bias, y, out, flags);
+        default: return launch_gemv<kBF16>(stream, x, rows, inner, weight, bias, y, out, flags);
     }
 }
 

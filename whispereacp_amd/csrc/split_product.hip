@@ -37,6 +37,8 @@
 #include "device_common.h"
 #include "ops.h"
 
+#include <algorithm>
+
 namespace wsp::ops
 {
 namespace
@@ -46,21 +48,40 @@ typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 typedef __attribute__((address_space(3))) char lds_char;
 
-constexpr int kStep = 64;             // k per step: eight 16-byte chunks of 16-bit values per row
-constexpr int kChunks = kStep / 8;
-constexpr int kLoadRows = 1024 / (2 * kStep); // tile rows one wave load (1 KB) covers
+constexpr int kRowBytes = 128;              // of a tile row per step: 64 16-bit values or 32 fp32
+constexpr int kChunks = kRowBytes / 16;
+constexpr int kLoadRows = 1024 / kRowBytes; // tile rows one wave load (1 KB) covers
 constexpr int kSplitThreads = 256;
 
 template <int WT>
 constexpr int parts_of()
 {
-    return WT == kF16 ? 2 : 3;
+    return WT == kF32 ? 1 : WT == kF16 ? 2 : 3;
 }
 
 template <int WT>
-__device__ __forceinline__ float4v mfma16(u32x4 a, u32x4 b, float4v c)
+constexpr int value_bytes()
 {
-    if constexpr (WT == kF16)
+    return WT == kF32 ? 4 : 2;
+}
+
+// One 16-byte chunk of each operand: 32 k of 16-bit values, or 16 k of fp32 in
+// four products (a lane's element e of chunk c stands for k = 4c + e in both).
+// One sum in the order of k: even and odd elements summed apart would be a
+// shorter chain, but where X is a signal and W its spectrum's basis each half
+// is an aliased spectrum and the two cancel (the log-mel's error against 64
+// bits grew from 1.2e-7 to 2.8e-7).
+template <int WT>
+__device__ __forceinline__ float4v multiply(u32x4 a, u32x4 b, float4v c)
+{
+    if constexpr (WT == kF32)
+    {
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+            c = __builtin_amdgcn_mfma_f32_16x16x4f32(__uint_as_float(a[e]), __uint_as_float(b[e]), c, 0, 0, 0);
+        return c;
+    }
+    else if constexpr (WT == kF16)
         return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(half8, a), __builtin_bit_cast(half8, b), c, 0,
                                                        0, 0);
     else
@@ -201,8 +222,8 @@ struct Tile
     static constexpr int P = parts_of<WT>();
     static constexpr int TM = TM_, TN = TN_, WM = WM_, WN = WN_, S = S_;
     static constexpr int kWaves = WM * WN;
-    static constexpr int kABytes = TM * kStep * 2; // one part's rows
-    static constexpr int kStageBytes = P * kABytes + TN * kStep * 2;
+    static constexpr int kABytes = TM * kRowBytes; // one part's rows
+    static constexpr int kStageBytes = P * kABytes + TN * kRowBytes;
     static constexpr int kLoads = (P * TM + TN) / kLoadRows;
     static_assert(kLoads % kWaves == 0, "whole loads per wave");
     static constexpr int kPerWave = kLoads / kWaves;
@@ -213,7 +234,8 @@ struct Tile
 template <class T, int WT>
 __global__ void __launch_bounds__(T::kWaves * kWave) split_product_kernel(SplitProduct a)
 {
-    constexpr int P = T::P, MT = T::MT, NT = T::NT;
+    constexpr int P = T::P, MT = T::MT, NT = T::NT, B = value_bytes<WT>();
+    constexpr int kStep = kRowBytes / B; // k per step
     extern __shared__ __attribute__((aligned(16))) unsigned char stage_mem[];
 
     const int tid = threadIdx.x, lane = tid % kWave;
@@ -221,15 +243,17 @@ __global__ void __launch_bounds__(T::kWaves * kWave) split_product_kernel(SplitP
     const int li = lane % 16, g = lane / 16;
     const int wm = wave / T::WN, wn = wave % T::WN;
     const int n_block = blockIdx.x * T::TN, m_block = blockIdx.y * T::TM;
-    const int steps = a.inner / kStep;
+    const int steps = (a.inner + kStep - 1) / kStep;
     // The block's columns lie in one of the (up to three) matrices.
     const int seg = n_block < a.split ? 0 : n_block < a.split2 ? 1 : 2;
     const int seg_first = seg == 0 ? 0 : seg == 1 ? a.split : a.split2;
     const void* w = seg == 0 ? a.w0 : seg == 1 ? a.w1 : a.w2;
+    const int width = seg == 0 ? a.split : seg == 1 ? a.split2 - a.split : a.out - a.split2;
 
     // This wave's loads: load q = wave + waves·t of a stage covers 8 tile rows
     // (the parts' rows first, then W's); lane i moves row 8 q' + i / 8, chunk
-    // (i % 8) ^ (row & 7), so it lands in that chunk's slot.
+    // (i % 8) ^ (row & 7), so it lands in that chunk's slot. Rows past the end
+    // (and fp32 W's columns) re-read the last one.
     const void* src[T::kPerWave];
     uint32_t offset[T::kPerWave];
     uint32_t dst[T::kPerWave]; // byte offset in the stage
@@ -242,26 +266,29 @@ __global__ void __launch_bounds__(T::kWaves * kWave) split_product_kernel(SplitP
             const int p = q / (T::TM / kLoadRows), rq = q % (T::TM / kLoadRows);
             const int r = kLoadRows * rq + lane / kChunks;
             const int row = min(m_block + r, a.rows - 1);
-            const int c = (lane % kChunks) ^ (r & 7);
             src[t] = a.parts;
-            offset[t] = (uint32_t) (((size_t) p * a.part_stride + (size_t) row * a.inner + 8 * c) * 2);
+            offset[t] = (uint32_t) (((size_t) p * a.part_stride + (size_t) row * a.inner) * B);
             dst[t] = p * T::kABytes + 1024 * rq;
         }
         else
         {
             const int wq = q - P * T::TM / kLoadRows;
-            const int col = kLoadRows * wq + lane / kChunks;
-            const int c = (lane % kChunks) ^ (col & 7);
+            const int col = min(n_block - seg_first + kLoadRows * wq + lane / kChunks, width - 1);
             src[t] = w;
-            offset[t] = (uint32_t) (((size_t) (n_block - seg_first + col) * a.inner + 8 * c) * 2);
+            offset[t] = (uint32_t) ((size_t) col * a.inner * B);
             dst[t] = P * T::kABytes + 1024 * wq;
         }
     }
+    // (A load's first tile row is a multiple of 8, so every load of a lane
+    // moves the same chunk.)
+    const uint32_t chunk_bytes = 16 * ((lane % kChunks) ^ (lane / kChunks));
     const uint32_t stage0 = lds_address(stage_mem);
     // Issues step `step`'s loads into stage buffer `buf` (a step past the end
     // reloads the last one into a buffer no one reads again).
     auto issue = [&](int step, int buf) {
-        const uint32_t k_bytes = (uint32_t) min(step, steps - 1) * (kStep * 2);
+        uint32_t k_bytes = (uint32_t) min(step, steps - 1) * kRowBytes + chunk_bytes;
+        if constexpr (WT == kF32) // a last step past the row's end: its last chunk instead (zeroed before use)
+            k_bytes = min(k_bytes, (uint32_t) a.inner * B - 16);
 #pragma unroll
         for (int t = 0; t < T::kPerWave; ++t)
             load_lds16(src[t], offset[t] + k_bytes,
@@ -287,9 +314,18 @@ __global__ void __launch_bounds__(T::kWaves * kWave) split_product_kernel(SplitP
         wait_loads<(T::S - 2) * T::kPerWave>();
         __syncthreads();
         issue(s + T::S - 1, buf == 0 ? T::S - 1 : buf - 1);
-        const unsigned char* st = stage_mem + buf * T::kStageBytes;
+        unsigned char* const st = stage_mem + buf * T::kStageBytes;
+        if constexpr (WT == kF32)
+            if (s == steps - 1 && a.inner % kStep != 0) // the chunks past the rows' end
+            {
+                const int first = a.inner % kStep / 4; // (inner is a multiple of 4)
+                for (int i = tid; i < (T::TM + T::TN) * kChunks; i += T::kWaves * kWave)
+                    if (i % kChunks >= first)
+                        reinterpret_cast<u32x4*>(st)[slot(i / kChunks, i % kChunks)] = u32x4 {0, 0, 0, 0};
+                __syncthreads();
+            }
 #pragma unroll
-        for (int kk = 0; kk < kStep / 32; ++kk)
+        for (int kk = 0; kk < kChunks / 4; ++kk)
         {
             const int c = 4 * kk + g;
             u32x4 af[MT][P], bf[NT];
@@ -307,7 +343,7 @@ __global__ void __launch_bounds__(T::kWaves * kWave) split_product_kernel(SplitP
                 for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
                     for (int nt = 0; nt < NT; ++nt)
-                        acc[mt][nt] = mfma16<WT>(bf[nt], af[mt][p], acc[mt][nt]);
+                        acc[mt][nt] = multiply<WT>(bf[nt], af[mt][p], acc[mt][nt]);
         }
         buf = buf == T::S - 1 ? 0 : buf + 1;
     }
@@ -317,16 +353,19 @@ __global__ void __launch_bounds__(T::kWaves * kWave) split_product_kernel(SplitP
     float* y = seg == 0 ? a.y0 : seg == 1 ? a.y1 : a.y2;
     const float* bias = seg == 0 ? a.bias0 : seg == 1 ? a.bias1 : a.bias2;
     const float scale = seg == 0 ? a.scale0 : seg == 1 ? a.scale1 : a.scale2;
-    const int width = seg == 0 ? a.split : seg == 1 ? a.split2 - a.split : a.out - a.split2;
+    // Four columns a lane go out as one store; fp32 products may end inside them.
+    const bool quads = WT != kF32 || (width % 4 == 0 && a.ldy % 4 == 0 && reinterpret_cast<uintptr_t>(y) % 16 == 0);
 #pragma unroll
     for (int nt = 0; nt < NT; ++nt)
     {
         const int c = n_block - seg_first + 16 * (NT * wn + nt) + 4 * g;
+        if (WT == kF32 && c >= width)
+            continue;
         float b[4] = {0.f, 0.f, 0.f, 0.f};
         if (bias != nullptr)
 #pragma unroll
             for (int r = 0; r < 4; ++r)
-                b[r] = bias[c + r];
+                b[r] = bias[WT == kF32 ? min(c + r, width - 1) : c + r];
 #pragma unroll
         for (int mt = 0; mt < MT; ++mt)
         {
@@ -341,7 +380,7 @@ __global__ void __launch_bounds__(T::kWaves * kWave) split_product_kernel(SplitP
                 if (a.flags & kProductGelu)
                     v[r] = exact_gelu(v[r]);
             }
-            if (a.out_parts != nullptr)
+            if (WT != kF32 && a.out_parts != nullptr)
             {
                 uint32_t bits[4][3];
 #pragma unroll
@@ -353,7 +392,7 @@ __global__ void __launch_bounds__(T::kWaves * kWave) split_product_kernel(SplitP
                     *reinterpret_cast<uint2*>(o + p * a.out_part_stride)
                         = uint2 {bits[0][p] | (bits[1][p] << 16), bits[2][p] | (bits[3][p] << 16)};
             }
-            else if ((seg == 1 && a.y1_halves != nullptr) || (seg == 2 && a.y2_halves_t != nullptr))
+            else if (WT != kF32 && ((seg == 1 && a.y1_halves != nullptr) || (seg == 2 && a.y2_halves_t != nullptr)))
             {
                 uint32_t hi[4], lo[4];
 #pragma unroll
@@ -381,7 +420,7 @@ __global__ void __launch_bounds__(T::kWaves * kWave) split_product_kernel(SplitP
                     }
                 }
             }
-            else
+            else if (quads)
             {
                 float4v* o = reinterpret_cast<float4v*>(y + (size_t) row * a.ldy + c);
                 float4v sum = {v[0], v[1], v[2], v[3]};
@@ -389,6 +428,14 @@ __global__ void __launch_bounds__(T::kWaves * kWave) split_product_kernel(SplitP
                     sum = *o + sum;
                 *o = sum;
             }
+            else
+#pragma unroll
+                for (int r = 0; r < 4; ++r)
+                    if (c + r < width)
+                    {
+                        float* o = y + (size_t) row * a.ldy + c + r;
+                        *o = a.flags & kProductResidual ? *o + v[r] : v[r];
+                    }
         }
     }
 }
@@ -401,7 +448,7 @@ hipError_t launch(hipStream_t stream, const SplitProduct& a)
                                                           hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
     if (allowed != hipSuccess)
         return allowed;
-    hipLaunchKernelGGL((split_product_kernel<T, WT>), dim3(a.out / T::TN, (a.rows + T::TM - 1) / T::TM),
+    hipLaunchKernelGGL((split_product_kernel<T, WT>), dim3((a.out + T::TN - 1) / T::TN, (a.rows + T::TM - 1) / T::TM),
                        dim3(T::kWaves * kWave), bytes, stream, a);
     return hipGetLastError();
 }
@@ -445,7 +492,7 @@ hipError_t launch_tiles(hipStream_t stream, const SplitProduct& a)
 
 bool split_product_fits(int wdtype, int inner, int out, int split, int split2)
 {
-    return (wdtype == kF16 || wdtype == kBF16) && inner % kStep == 0 && out % 128 == 0 && split % 128 == 0
+    return (wdtype == kF16 || wdtype == kBF16) && inner % 64 == 0 && out % 128 == 0 && split % 128 == 0
            && split2 % 128 == 0 && split <= split2 && split2 <= out;
 }
 
@@ -481,6 +528,57 @@ hipError_t layernorm_parts(hipStream_t stream, const float* x, const float* gamm
         hipLaunchKernelGGL(layernorm_parts_kernel<kBF16>, grid, dim3(kNormRowsPerBlock * kWave), 0, stream, x,
                            gamma, beta, rows, width, eps, static_cast<u16*>(parts), part_stride);
     return hipGetLastError();
+}
+
+// fp32 X and W through the same kernel, one "part" of four-byte values:
+// v_mfma_f32_16x16x4_f32 in 32-wide steps.
+bool fp32_split_fits(const TileProduct& a)
+{
+    auto aligned = [](const void* p) { return reinterpret_cast<uintptr_t>(p) % 16 == 0; };
+    return a.wdtype == kF32 && a.inner % 4 == 0 && aligned(a.x) && aligned(a.w0) && a.rows_per_group >= a.rows
+           && (a.split >= a.out || (a.split % 64 == 0 && aligned(a.w1)))
+           && (a.split2 >= a.out || (a.split2 % 64 == 0 && aligned(a.w2)))
+           && (unsigned long long) std::max(a.rows, a.out) * a.inner < 1ull << 30; // 32-bit byte offsets
+}
+
+// 64 x 64 tiles, 32 x 64 or 32 x 32, whichever finishes first by its rounds
+// over the CUs: a smaller tile costs 1.07 or 1.2 of its share of a 64 x 64
+// one's time (more loads a product), so it wins where the larger leaves a
+// round part-filled. Measured at 1500 rows (us in that order): 512 -> 512
+// 13.2, 13.1, 11.7; 512 -> 1536 30.4, 28.7, 30.6; 512 -> 2048 31.9, 33.3,
+// 38.6; 2048 -> 512 41.4, 41.3, 35.4; 3840 -> 1280 129, 134, 153 (247 as 64 x
+// 64 tiles of vector multiply-adds).
+hipError_t fp32_split(hipStream_t stream, const TileProduct& t)
+{
+    SplitProduct a {};
+    a.parts = t.x;
+    a.rows = t.rows;
+    a.inner = t.inner;
+    a.w0 = t.w0;
+    a.w1 = t.w1;
+    a.w2 = t.w2;
+    a.split = t.split;
+    a.split2 = t.split2;
+    a.out = t.out;
+    a.bias0 = t.bias0;
+    a.bias1 = t.bias1;
+    a.bias2 = t.bias2;
+    a.y0 = t.y0;
+    a.y1 = t.y1;
+    a.y2 = t.y2;
+    a.ldy = t.ldy;
+    a.flags = t.flags;
+    a.wdtype = kF32;
+    const long long units = compute_units();
+    auto rounds = [&](int tm, int tn) {
+        return ((long long) ((a.rows + tm - 1) / tm) * ((a.out + tn - 1) / tn) + units - 1) / units;
+    };
+    const double whole = 1.0 * rounds(64, 64), half = 0.535 * rounds(32, 64), quarter = 0.3 * rounds(32, 32);
+    if (whole <= half && whole <= quarter)
+        return launch<Tile<kF32, 64, 64, 2, 2, 2>, kF32>(stream, a);
+    if (half <= quarter)
+        return launch<Tile<kF32, 32, 64, 2, 2, 2>, kF32>(stream, a);
+    return launch<Tile<kF32, 32, 32, 2, 2, 4>, kF32>(stream, a);
 }
 
 hipError_t split_product(hipStream_t stream, const SplitProduct& product)
