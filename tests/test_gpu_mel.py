@@ -35,6 +35,20 @@ def test_reduced_shape_matches_oracle(oracle):
     assert err <= 1e-4
 
 
+@pytest.mark.parametrize("samples,fft,hop,frames,mels", [
+    (4000, 400, 160, 17, 81),    # one frame past a block of sixteen, one band past a tile
+    (3000, 33, 7, 31, 5),        # an odd transform: no middle term
+    (40000, 2048, 512, 40, 24),  # too long for one block's memory: the product launches
+])
+def test_other_shapes_match_oracle(oracle, samples, fft, hop, frames, mels):
+    s = S.MelShape(samples, fft, hop, frames, mels)
+    x = S.tone_and_noise(s.sample_count)
+    f = S.triangular_filters(s.mel_count, s.bin_count)
+    got = gpu_mel(s, x, f)
+    expected = oracle.mel_spectrogram(x, f, s.fft_length, s.hop_length, s.frame_count)
+    assert float(np.max(np.abs(got - expected))) <= 1e-4
+
+
 def test_whisper_shape_spans_two_and_matches_oracle(oracle):
     s = S.MelShape()
     x = S.tone_and_noise(s.sample_count)
