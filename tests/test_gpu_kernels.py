@@ -191,7 +191,11 @@ def test_embed_refuses_positions_past_the_table(ctx):
     # encoder rows, at the decode configurations' head counts and narrower heads
     (2, 2, 768, 12, True), (4, 4, 768, 12, True), (7, 40, 512, 8, True), (16, 300, 1280, 20, True),
     (5, 448, 384, 6, True), (4, 1500, 768, 12, False), (16, 1500, 1280, 20, False), (9, 77, 768, 12, False),
-    (3, 65, 256, 4, False), (12, 129, 128, 4, True), (16, 1500, 128, 32, False), (8, 3, 64, 16, False)])
+    (3, 65, 256, 4, False), (12, 129, 128, 4, True), (16, 1500, 128, 32, False), (8, 3, 64, 16, False),
+    # long prompts: query tiles of 32 with a part-filled last one, one and
+    # several key splits, spans that end inside a wave's 32 keys
+    (17, 40, 512, 8, True), (33, 448, 384, 6, True), (40, 40, 64, 1, True), (224, 300, 1280, 20, True),
+    (96, 1500, 768, 12, False), (65, 257, 128, 2, False)])
 def test_attention_matches_oracle(ctx, oracle, q_count, k_count, width, heads, causal):
     q = S.normal_values(q_count * width, 1, 1.0).reshape(q_count, width)
     k = S.normal_values(k_count * width, 2, 1.0).reshape(k_count, width)
@@ -228,6 +232,27 @@ def test_attention_causal_future_keys_are_never_read(ctx):
     ctx.attention(dev(q), 3, dev(k), dev(v2), 3, 8, 2, True, 0.5, out_b)
     sync()
     assert np.array_equal(out_a.cpu().numpy()[:2], out_b.cpu().numpy()[:2])
+
+
+@pytest.mark.parametrize("q_count,k_count", [(3, 20), (40, 90)])
+def test_attention_hidden_values_may_be_non_finite(ctx, q_count, k_count):
+    # 64-channel heads: a later position's infinite or NaN value must not
+    # reach the queries before it, nor its NaN key their scores.
+    width = 128
+    q = S.normal_values(q_count * width, 1, 1.0).reshape(q_count, width)
+    k = S.normal_values(k_count * width, 2, 1.0).reshape(k_count, width)
+    v = S.normal_values(k_count * width, 3, 1.0).reshape(k_count, width)
+    first = k_count - 2
+    results = []
+    for key, value in ((0.0, 0.0), (np.nan, np.inf), (np.inf, np.nan)):
+        k[first:], v[first:] = key, value
+        out = dev(np.zeros((q_count, width), np.float32))
+        ctx.attention(dev(q), q_count, dev(k), dev(v), k_count, width, 2, True, 0.125, out)
+        sync()
+        results.append(out.cpu().numpy())
+    for odd in results[1:]:
+        assert np.allclose(odd[:-2], results[0][:-2], rtol=1e-5, atol=1e-6)
+        assert not np.any(np.isfinite(odd[-2:]))
 
 
 def test_attention_refuses_wide_heads(ctx):

@@ -27,6 +27,7 @@ namespace
 {
 constexpr size_t kStaticAttentionFloats = size_t(1) << 20;
 constexpr int kMaxDevices = 64;
+static_assert(kStaticAttentionFloats >= wsp::ops::kQueryAttentionFloats, "the multi-query attention fits");
 
 // On the host this name is a stand-in, not a device address: only the
 // pointer hipGetSymbolAddress returns for the current device may reach a

@@ -81,8 +81,8 @@ int wsp_hip_ctx_create(const wsp_decoder_shape* shape, int device, void* stream,
             floats = std::max(floats, wsp::ops::attention_workspace_floats(shape->heads, q, longest,
                                                                            head_width));
         ctx->attention_floats = std::max<size_t>(floats, 1);
-        status = hip_status(ctx, hipMalloc(&ctx->attention_workspace, ctx->attention_floats * sizeof(float)),
-                            "attention workspace");
+        const size_t held = std::max(ctx->attention_floats, wsp::ops::kQueryAttentionFloats);
+        status = hip_status(ctx, hipMalloc(&ctx->attention_workspace, held * sizeof(float)), "attention workspace");
         // The prompt attention's per-head counters start at zero (each launch
         // leaves them zero again).
         if (status == WSP_OK)

@@ -132,6 +132,12 @@ constexpr int kMaxPromptQueries = 16;
 // and whoever provides a workspace zeroes them once before its first use.
 constexpr int kAttentionCounters = 256;
 
+// Blocks a round of the multi-query attention of 64-channel heads takes, and
+// the workspace it may use whatever the call: a workspace handed to attention()
+// for such heads holds at least this many floats.
+constexpr int kQueryBlocks = 256;
+constexpr size_t kQueryAttentionFloats = kAttentionCounters + (size_t) kQueryBlocks * 32 * (64 + 2);
+
 // How many key chunks the split-key attention uses for this shape, and the
 // workspace (floats) it needs: the counters, then the partials —
 // chunks * (head_width + 2) per (head, query) for one query or more than

@@ -262,32 +262,273 @@ __global__ void __launch_bounds__(kBlock) attention_chunk_kernel(
     }
 }
 
-__global__ void attention_combine_kernel(const float* __restrict__ partials, int q_count,
-                                         int width, int head_width, int chunks,
-                                         float* __restrict__ out)
+// A wave for each fourth chunk, eight chunks' loads in flight: walking them
+// one after the other cost 18 us for 32 chunks of eight heads.
+__global__ void __launch_bounds__(kBlock) attention_combine_kernel(const float* __restrict__ partials, int q_count,
+                                                                   int width, int head_width, int chunks,
+                                                                   float* __restrict__ out)
 {
+    constexpr int kAhead = 8;
+    __shared__ float sums[kWavesPerBlock][2][kMaxHeadWidth];
     const int query = blockIdx.x % q_count;
     const int head = blockIdx.x / q_count;
-    const int c = threadIdx.x;
-    if (c >= head_width)
-        return;
-    const float* base = partials + (size_t) (head * q_count + query) * chunks * (head_width + 2);
+    const int c = threadIdx.x % kWave, wave = threadIdx.x / kWave;
+    const int pitch = head_width + 2;
+    const float* base = partials + (size_t) (head * q_count + query) * chunks * pitch;
 
     float largest = -INFINITY;
-    for (int k = 0; k < chunks; ++k)
-        largest = fmaxf(largest, base[(size_t) k * (head_width + 2)]);
+    for (int k = c; k < chunks; k += kWave)
+        largest = fmaxf(largest, base[(size_t) k * pitch]);
+    largest = wave_max(largest);
 
     float numerator = 0.f, denominator = 0.f;
-    for (int k = 0; k < chunks; ++k)
+    for (int k0 = wave; k0 < chunks; k0 += kAhead * kWavesPerBlock)
     {
-        const float* part = base + (size_t) k * (head_width + 2);
-        if (part[1] == 0.f)
-            continue;
-        const float factor = expf(part[0] - largest);
-        numerator += factor * part[2 + c];
-        denominator += factor * part[1];
+        float top[kAhead], sum[kAhead], row[kAhead];
+#pragma unroll
+        for (int i = 0; i < kAhead; ++i)
+        {
+            const float* part = base + (size_t) min(k0 + i * kWavesPerBlock, chunks - 1) * pitch;
+            top[i] = part[0];
+            sum[i] = part[1];
+            row[i] = part[2 + min(c, head_width - 1)];
+        }
+#pragma unroll
+        for (int i = 0; i < kAhead; ++i)
+            if (k0 + i * kWavesPerBlock < chunks && sum[i] != 0.f) // (a chunk with no visible key sums to zero)
+            {
+                const float factor = expf(top[i] - largest);
+                numerator += factor * row[i];
+                denominator += factor * sum[i];
+            }
     }
-    out[(size_t) query * width + head * head_width + c] = numerator / denominator;
+    sums[wave][0][c] = numerator;
+    sums[wave][1][c] = denominator;
+    __syncthreads();
+    if (threadIdx.x < head_width)
+    {
+        float n = 0.f, d = 0.f;
+#pragma unroll
+        for (int w = 0; w < kWavesPerBlock; ++w)
+        {
+            n += sums[w][0][c];
+            d += sums[w][1][c];
+        }
+        out[(size_t) query * width + head * head_width + c] = n / d;
+    }
+}
+
+// ---------------------------------------------------------------------------
+// Attention of two and more queries with heads of 64 channels, in fp32 on the
+// matrix cores (v_mfma_f32_16x16x4_f32), with the causal rule of
+// Kernels/Attention.h:34-47. Block (head, 16·QT queries, key split): its eight
+// waves take 32 keys at a time each, straight from memory into operand
+// registers (no barrier in the loop), every key serving all the block's
+// queries, and keep an online (max, sum, row) per query; the waves are merged
+// in order through LDS at the end.
+//
+// S^T = K·Q^T leaves lane (li, g) with keys 4g + r of query li, which is the
+// operand of O^T = V^T·P^T as it stands: product r takes key 4g + r from lane
+// group g, and V's float4 of channels 4li .. 4li + 3 feeds the four products
+// of channels 4·row + t. 96 queries over 1500 keys of 12 heads: 160 us as one
+// block per (query, head, chunk) of vector code, 17 here. Bound by the
+// K and V reads of each query tile from the L2s and, at these sizes, by the
+// chain load, score, softmax, merge.
+// ---------------------------------------------------------------------------
+constexpr int kQueryWaves = 8;
+constexpr int kQueryKeys = 32; // keys a wave takes at a time
+
+template <int QT>
+__global__ void __launch_bounds__(kQueryWaves * kWave) query_attention_kernel(
+    const float* __restrict__ q, int q_count, const float* __restrict__ keys, const float* __restrict__ values,
+    int k_count, int width, int causal, float scale, int splits, int span, float* __restrict__ out,
+    float* __restrict__ partials)
+{
+    __shared__ float tops[kQueryWaves][QT][16], totals[kQueryWaves][QT][16];
+    __shared__ float4v rows[kQueryWaves][16][16]; // [wave][query][channel run of four]
+
+    const int split = blockIdx.x % splits, head = blockIdx.x / splits, first_query = blockIdx.y * 16 * QT;
+    const int wave = threadIdx.x / kWave, lane = threadIdx.x % kWave, li = lane % 16, g = lane / 16;
+    const int column = head * 64;
+    const int past = k_count - q_count; // causal: query i sees keys 0 .. past + i
+    const int last_seen = causal ? past + min(first_query + 16 * QT, q_count) - 1 : k_count - 1;
+    const int end = min(min(split * span + span, k_count), last_seen + 1);
+
+    float4v qf[QT][4], o[QT][4];
+    float m[QT], l[QT];
+#pragma unroll
+    for (int t = 0; t < QT; ++t)
+    {
+        const float* row = q + (size_t) min(first_query + 16 * t + li, q_count - 1) * width + column + 4 * g;
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+        {
+            qf[t][j] = *reinterpret_cast<const float4v*>(row + 16 * j);
+            o[t][j] = float4v {0.f, 0.f, 0.f, 0.f};
+        }
+        m[t] = -INFINITY;
+        l[t] = 0.f;
+    }
+    for (int k0 = split * span + kQueryKeys * wave; k0 < end; k0 += kQueryKeys * kQueryWaves)
+    {
+        float4v kf[2][4], vf[2][4];
+#pragma unroll
+        for (int b = 0; b < 2; ++b)
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+            {
+                const int key = min(k0 + 16 * b + li, end - 1);
+                kf[b][j] = *reinterpret_cast<const float4v*>(keys + (size_t) key * width + column + 16 * j + 4 * g);
+            }
+#pragma unroll
+        for (int b = 0; b < 2; ++b)
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+            {
+                const int key = min(k0 + 16 * b + 4 * g + r, end - 1);
+                vf[b][r] = *reinterpret_cast<const float4v*>(values + (size_t) key * width + column + 4 * li);
+            }
+        // Keys that some of these queries do not see get weight zero in the
+        // products, which hides a value only while it is finite.
+        bool hidden_odd = false;
+        if (causal && k0 + kQueryKeys > past + first_query + 1)
+        {
+#pragma unroll
+            for (int b = 0; b < 2; ++b)
+#pragma unroll
+                for (int r = 0; r < 4; ++r)
+#pragma unroll
+                    for (int c = 0; c < 4; ++c)
+                        hidden_odd = hidden_odd || !isfinite(vf[b][r][c]);
+            hidden_odd = __any(hidden_odd);
+        }
+#pragma unroll
+        for (int t = 0; t < QT; ++t)
+        {
+            // Four partial sums a score, added in pairs: chains of four roundings
+            // instead of sixteen, and products that need not wait for each other.
+            float4v part[2][4], s[2];
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+#pragma unroll
+                for (int j = 0; j < 4; ++j)
+#pragma unroll
+                    for (int b = 0; b < 2; ++b)
+                        part[b][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(
+                            kf[b][j][e], qf[t][j][e], e == 0 ? float4v {0.f, 0.f, 0.f, 0.f} : part[b][j], 0, 0, 0);
+#pragma unroll
+            for (int b = 0; b < 2; ++b)
+                s[b] = (part[b][0] + part[b][1]) + (part[b][2] + part[b][3]);
+            const int seen = causal ? min(end, past + first_query + 16 * t + li + 1) : end; // keys before this one
+            float top = -INFINITY;
+#pragma unroll
+            for (int b = 0; b < 2; ++b)
+#pragma unroll
+                for (int r = 0; r < 4; ++r)
+                {
+                    s[b][r] = k0 + 16 * b + 4 * g + r < seen ? scale * s[b][r] : -INFINITY;
+                    top = fmaxf(top, s[b][r]);
+                }
+            top = fmaxf(top, __shfl_xor(top, 16));
+            top = fmaxf(top, __shfl_xor(top, 32));
+            const float m_new = fmaxf(m[t], top);
+            const float alpha = m_new == -INFINITY ? 1.f : expf(m[t] - m_new);
+            float own = 0.f;
+#pragma unroll
+            for (int b = 0; b < 2; ++b)
+#pragma unroll
+                for (int r = 0; r < 4; ++r)
+                {
+                    s[b][r] = k0 + 16 * b + 4 * g + r < seen ? expf(s[b][r] - m_new) : 0.f;
+                    own += s[b][r];
+                }
+            l[t] = l[t] * alpha + own;
+            m[t] = m_new;
+#pragma unroll
+            for (int c = 0; c < 4; ++c)
+                o[t][c] *= alpha;
+            if (hidden_odd) // each query's own keys alone
+            {
+#pragma unroll
+                for (int b = 0; b < 2; ++b)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r)
+                        for (int from = 0; from < 4; ++from)
+                        {
+                            const float weight = __shfl(s[b][r], li + 16 * from);
+                            const int key = k0 + 16 * b + 4 * from + r;
+                            if (key >= seen)
+                                continue;
+                            const float* row = values + (size_t) key * width + column;
+#pragma unroll
+                            for (int c = 0; c < 4; ++c)
+#pragma unroll
+                                for (int i = 0; i < 4; ++i)
+                                    o[t][c][i] += weight * row[4 * (4 * g + i) + c];
+                        }
+                continue;
+            }
+#pragma unroll
+            for (int b = 0; b < 2; ++b)
+#pragma unroll
+                for (int r = 0; r < 4; ++r)
+#pragma unroll
+                    for (int c = 0; c < 4; ++c)
+                        o[t][c] = __builtin_amdgcn_mfma_f32_16x16x4f32(vf[b][r][c], s[b][r], o[t][c], 0, 0, 0);
+        }
+    }
+#pragma unroll
+    for (int t = 0; t < QT; ++t)
+    {
+        l[t] += __shfl_xor(l[t], 16);
+        l[t] += __shfl_xor(l[t], 32);
+        if (g == 0)
+        {
+            tops[wave][t][li] = m[t];
+            totals[wave][t][li] = l[t];
+        }
+    }
+#pragma unroll
+    for (int t = 0; t < QT; ++t)
+    {
+        // o[t][c][r] is channel 4 (4g + r) + c of query li.
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+            rows[wave][li][4 * g + r] = float4v {o[t][0][r], o[t][1][r], o[t][2][r], o[t][3][r]};
+        __syncthreads();
+        for (int i = threadIdx.x; i < 16 * 64; i += kQueryWaves * kWave)
+        {
+            const int at = i / 64, c = i % 64, query = first_query + 16 * t + at;
+            float largest = -INFINITY;
+#pragma unroll
+            for (int w = 0; w < kQueryWaves; ++w)
+                largest = fmaxf(largest, tops[w][t][at]);
+            float numerator = 0.f, denominator = 0.f;
+#pragma unroll
+            for (int w = 0; w < kQueryWaves; ++w)
+                if (totals[w][t][at] != 0.f) // (a wave with no visible key)
+                {
+                    const float factor = expf(tops[w][t][at] - largest);
+                    numerator += factor * reinterpret_cast<const float*>(&rows[w][at][c / 4])[c % 4];
+                    denominator += factor * totals[w][t][at];
+                }
+            if (query >= q_count)
+                continue;
+            if (splits == 1)
+                out[(size_t) query * width + column + c] = numerator / denominator;
+            else
+            {
+                float* part = partials + ((size_t) (head * q_count + query) * splits + split) * (64 + 2);
+                part[2 + c] = numerator;
+                if (c == 0)
+                {
+                    part[0] = largest;
+                    part[1] = denominator;
+                }
+            }
+        }
+        __syncthreads(); // (the rows are written again for the next queries)
+    }
 }
 
 // ---------------------------------------------------------------------------
@@ -684,6 +925,34 @@ size_t attention_workspace_floats(int heads, int q_count, int k_count, int head_
     return kAttentionCounters + (chunks > 1 ? (size_t) heads * q_count * chunks * (head_width + 2) : 0);
 }
 
+// Two queries on, heads of 64 channels: query_attention_kernel over 16 queries
+// a block, or 32 (each key and value read for twice as many) where blocks of 16
+// over 256 keys each would not fit one round. As many key splits as leave each wave 32
+// keys, while the blocks fit one round of the CUs; what they leave stays within
+// kQueryAttentionFloats (at most 256·32 partial rows).
+hipError_t query_attention(hipStream_t stream, const float* q, int q_count, const float* keys, const float* values,
+                           int k_count, int width, int heads, int causal, float scale, float* out, float* partials)
+{
+    const int reach = kQueryKeys * kQueryWaves, reaches = (k_count + reach - 1) / reach;
+    const int tile = (long long) heads * ((q_count + 15) / 16) * reaches > kQueryBlocks ? 32 : 16;
+    const int tiles = (q_count + tile - 1) / tile;
+    const int splits = std::max(1, std::min(reaches, kQueryBlocks / (heads * tiles)));
+    const int span = ((k_count + splits - 1) / splits + kQueryKeys - 1) / kQueryKeys * kQueryKeys;
+    const dim3 grid(heads * splits, tiles), block(kQueryWaves * kWave);
+    if (tile == 32)
+        hipLaunchKernelGGL(query_attention_kernel<2>, grid, block, 0, stream, q, q_count, keys, values, k_count, width,
+                           causal, scale, splits, span, out, partials);
+    else
+        hipLaunchKernelGGL(query_attention_kernel<1>, grid, block, 0, stream, q, q_count, keys, values, k_count, width,
+                           causal, scale, splits, span, out, partials);
+    hipError_t e = hipGetLastError();
+    if (e != hipSuccess || splits == 1)
+        return e;
+    hipLaunchKernelGGL(attention_combine_kernel, dim3(heads * q_count), dim3(kBlock), 0, stream, partials, q_count,
+                       width, 64, splits, out);
+    return hipGetLastError();
+}
+
 hipError_t attention(hipStream_t stream, const float* q, int q_count, const float* keys,
                      const float* values, int k_count, int width, int heads, int causal,
                      float scale, float* out, float* workspace)
@@ -691,6 +960,8 @@ hipError_t attention(hipStream_t stream, const float* q, int q_count, const floa
     const int head_width = width / heads;
     unsigned int* const counters = reinterpret_cast<unsigned int*>(workspace);
     float* const partials = workspace + kAttentionCounters;
+    if (q_count > 1 && head_width == 64)
+        return query_attention(stream, q, q_count, keys, values, k_count, width, heads, causal, scale, out, partials);
     if (takes_prompt_attention(q_count, heads))
     {
         const int splits = prompt_attention_splits(heads, k_count);
@@ -708,7 +979,7 @@ hipError_t attention(hipStream_t stream, const float* q, int q_count, const floa
     hipError_t e = hipGetLastError();
     if (e != hipSuccess || chunks == 1)
         return e;
-    hipLaunchKernelGGL(attention_combine_kernel, dim3(heads * q_count), dim3(kMaxHeadWidth), 0, stream,
+    hipLaunchKernelGGL(attention_combine_kernel, dim3(heads * q_count), dim3(kBlock), 0, stream,
                        workspace, q_count, width, head_width, chunks, out);
     return hipGetLastError();
 }
