@@ -176,6 +176,7 @@ private:
     void touch(int value, int instruction);
 
     void place();
+    std::size_t issueShared(std::size_t first);
     void issue(const Instruction& instruction);
     void check(int status) const;
     void closeRecording();

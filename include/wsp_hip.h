@@ -91,6 +91,23 @@ void* wsp_hip_stream(const wsp_hip_ctx* ctx);
 int wsp_hip_linear(wsp_hip_ctx* ctx, const float* x, int rows, int inner, const void* weight,
                    int wdtype, const float* bias, float* y, int out, int flags);
 
+/* One of wsp_hip_linear_many's weights [out, inner], its bias [out] or null,
+ * and its output [rows, out]. */
+typedef struct wsp_linear_target
+{
+    const void* weight;
+    const float* bias;
+    float* y;
+} wsp_linear_target;
+
+/* wsp_hip_linear for several weights of one storage over the same rows, with
+ * no flags; the outputs must not overlap. More than 16 rows share launches:
+ * the consecutive projections of one input that a recording makes (a
+ * sequence's cross keys and values of every layer, Decoder/Decoder.cpp:121-146,
+ * a prompt's queries, keys and values). */
+int wsp_hip_linear_many(wsp_hip_ctx* ctx, const float* x, int rows, int inner, const wsp_linear_target* targets,
+                        int count, int wdtype, int out);
+
 /* y = (x - mean) * rsqrt(var + eps) * gamma + beta over rows of `width`
  * (biased variance of the centred values). Replaces LayerNorm
  * (Kernels/LayerNorm.h:19-90). */

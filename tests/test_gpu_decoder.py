@@ -266,3 +266,23 @@ def test_greedy_loop_honours_the_suppression_masks():
                                    later_mask=to_device(later_mask))
     assert masked[0] != full[0]
     assert full[1] not in masked[1:]
+
+
+@pytest.mark.parametrize("storage", ["F16", "F32"])
+def test_long_prompt_matches_oracle(oracle, storage):
+    # Past the fused launches: 40 tokens in one recorded step (multi-query
+    # attention over self and cross keys, the projections of one input sharing
+    # launches), then one more token.
+    from helpers import DecoderRun, oracle_tensors, worst_error
+    shape = S.DecoderShape(128, 2, 2, 512, 300, 64, 70)
+    decoder_file = S.workload_decoder_file(shape, storage, 1000)
+    encoded = S.normal_encoder_output(70, 128, 7)
+    tokens = [(7 * i) % 300 for i in range(41)]
+    run = DecoderRun(shape, decoder_file)
+    run.begin(encoded)
+    session = oracle.session(shape, oracle_tensors(decoder_file, shape))
+    session.begin(encoded)
+    for part in (tokens[:40], tokens[40:]):
+        _, logits, _ = run.step(part)
+        _, expected = session.step(part)
+        assert worst_error(logits, expected) <= 1e-4

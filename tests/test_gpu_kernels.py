@@ -101,6 +101,37 @@ def test_linear_paths(ctx, dtype, rows, inner, out):
         assert np.all(got[:, column] == np.inf)
 
 
+@pytest.mark.parametrize("dtype", ["F32", "F16", "BF16"])
+@pytest.mark.parametrize("rows,inner,out,count", [(3, 64, 128, 3), (17, 64, 128, 70), (300, 128, 256, 5),
+                                                  (300, 96, 64, 4), (40, 40, 24, 4)])
+def test_linear_many_equals_each_alone(ctx, dtype, rows, inner, out, count):
+    # Several weights over the same rows in shared launches: past a launch's 64
+    # matrices, over stored parts, in fp32 and three at a time.
+    import ctypes
+    from whispereacp_amd import _native as N
+    from whispereacp_amd.decoder import ptr, stored_to_device
+
+    class Target(ctypes.Structure):
+        _fields_ = [("weight", ctypes.c_void_p), ("bias", ctypes.c_void_p), ("y", ctypes.c_void_p)]
+
+    x = S.normal_values(rows * inner, 19, 1.0).reshape(rows, inner)
+    xd, keep, table = dev(x), [], (Target * count)()
+    for i in range(count):
+        stored, w = weights(out, inner, dtype, 100 + i)
+        wd, wdtype = stored_to_device(S.StoredTensor("w", dtype, (out, inner), stored))
+        bias = None if i % 2 else dev(S.normal_values(out, 300 + i, 0.1))
+        y = dev(np.full((rows, out), np.nan, np.float32))
+        keep.append((w, wd, bias, y))
+        table[i] = Target(ptr(wd), ptr(bias), ptr(y))
+    ctx._check(ctx.lib.wsp_hip_linear_many(ctx.handle, ptr(xd), rows, inner, ctypes.addressof(table), count, wdtype,
+                                           out))
+    sync()
+    for w, _, bias, y in keep:
+        expected = x.astype(np.float64) @ w.astype(np.float64).T
+        expected += 0 if bias is None else bias.cpu().numpy()
+        assert worst_error(y.cpu().numpy(), expected) <= 1e-5 + 2.4e-7 * inner
+
+
 def test_linear_without_bias(ctx, oracle):
     x = S.normal_values(2 * 64, 3, 1.0).reshape(2, 64)
     stored, w = weights(32, 64, "F32", 5)

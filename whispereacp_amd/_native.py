@@ -96,6 +96,7 @@ SIGNATURES = {
     "wsp_hip_last_error": (c_char_p, [c_void_p]),
     "wsp_hip_stream": (c_void_p, [c_void_p]),
     "wsp_hip_linear": (c_int, [c_void_p, c_void_p, c_int, c_int, c_void_p, c_int, c_void_p, c_void_p, c_int, c_int]),
+    "wsp_hip_linear_many": (c_int, [c_void_p, c_void_p, c_int, c_int, c_void_p, c_int, c_int, c_int]),
     "wsp_hip_layernorm": (c_int, [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int, c_float]),
     "wsp_hip_embed": (c_int, [c_void_p, c_void_p, c_int, c_void_p, c_void_p, c_int, c_void_p, c_int]),
     "wsp_hip_attention": (c_int, [c_void_p, c_void_p, c_int, c_void_p, c_void_p, c_int, c_int, c_int, c_int,

@@ -1590,6 +1590,11 @@ struct wsp_batch
     float* self_values = nullptr;
     float* cross_keys = nullptr;  // [layers][cross_positions][streams][width]
     float* cross_values = nullptr;
+    // begin's encoder rows as 16-bit parts, a few streams' at a time, and every
+    // layer's key and value matrices.
+    void* cross_parts = nullptr;
+    size_t cross_parts_bytes = 0;
+    std::vector<wsp::ops::ProductMatrix> cross_matrices;
     float* cross_scratch = nullptr; // [cross_positions][width], made by the first begin that needs it
     float* h = nullptr;           // [rows_padded][width] residual stream, fragment-major (residual_index)
     float* q = nullptr;           // [rows_padded][width] queries
@@ -2228,6 +2233,15 @@ int wsp_batch_create(const wsp_decoder_shape* shape, int streams, int max_step_t
     if (e == hipSuccess)
         e = allocate(b, &b->cross_values, (size_t) s.layers * cross_layer_stride(b));
     if (e == hipSuccess)
+    {
+        // Whole streams' rows, 64 MB of them (five streams of large-v3: 59 row
+        // tiles a launch) or one stream's.
+        const size_t stream_bytes = wsp::ops::parts_bytes((size_t) s.cross_positions * d);
+        const size_t streams_held = std::clamp<size_t>((size_t(64) << 20) / stream_bytes, 1, (size_t) streams);
+        b->cross_parts_bytes = streams_held * stream_bytes;
+        e = allocate(b, reinterpret_cast<char**>(&b->cross_parts), b->cross_parts_bytes);
+    }
+    if (e == hipSuccess)
         e = allocate(b, &b->h, (size_t) b->rows_padded * d);
     if (e == hipSuccess)
         e = allocate(b, &b->q, (size_t) b->rows_padded * d);
@@ -2342,35 +2356,49 @@ int wsp_batch_begin(wsp_batch* b, const wsp_cross_tensors* layers, int wdtype, c
         return fail(b, WSP_ERR_SHAPE, "wsp_batch_begin: more cross rows than the batch was sized for");
     const int d = b->shape.width;
     for (int l = 0; l < b->shape.layers; ++l)
-    {
-        const wsp_cross_tensors& L = layers[l];
-        if (L.key_w == nullptr || L.value_w == nullptr)
+        if (layers[l].key_w == nullptr || layers[l].value_w == nullptr)
             return fail(b, WSP_ERR_ARGUMENT, "wsp_batch_begin: a layer without cross key/value weights");
-        float* keys = b->cross_keys + (size_t) l * cross_layer_stride(b);
-        float* values = b->cross_values + (size_t) l * cross_layer_stride(b);
-        hipError_t e = hipSuccess;
-        if (wsp::ops::tile_product_fits(wdtype, d, 2 * d, d, encoder_rows))
+    if (wsp::ops::parts_fit(wdtype, d, d, encoder_rows) && b->streams * cross_rows > wsp::ops::kSplitRowLimit)
+    {
+        // A few streams' rows at a time, as many as the parts hold, for every
+        // layer's keys and values in one product (the rows are cut into parts
+        // once): row r of the encoder block is row r % cross_rows of stream
+        // r / cross_rows.
+        b->cross_matrices.resize((size_t) 2 * b->shape.layers);
+        const size_t rows_held = b->cross_parts_bytes / wsp::ops::parts_bytes((size_t) d);
+        const int at_once = (int) std::max<size_t>(1, rows_held / cross_rows);
+        for (int c = 0; c < b->streams; c += at_once)
         {
-            // Every stream's rows in one launch: row r of the encoder block is
-            // row r % cross_rows of stream r / cross_rows.
-            wsp::ops::TileProduct p {};
-            p.x = encoder_rows;
-            p.rows = b->streams * cross_rows;
+            const size_t at = (size_t) c * cross_stream_stride(b);
+            for (int l = 0; l < b->shape.layers; ++l)
+            {
+                const size_t layer = (size_t) l * cross_layer_stride(b) + at;
+                b->cross_matrices[2 * l] = {layers[l].key_w, nullptr, b->cross_keys + layer, 1.f};
+                b->cross_matrices[2 * l + 1] = {layers[l].value_w, layers[l].value_b, b->cross_values + layer, 1.f};
+            }
+            wsp::ops::Products p {};
+            p.x = encoder_rows + (size_t) c * cross_rows * d;
+            p.rows = std::min(at_once, b->streams - c) * cross_rows;
             p.inner = d;
-            p.w0 = L.key_w;
-            p.w1 = L.value_w;
-            p.split = d;
-            p.out = 2 * d;
-            p.bias1 = L.value_b;
-            p.y0 = keys;
-            p.y1 = values;
+            p.matrices = b->cross_matrices.data();
+            p.count = 2 * b->shape.layers;
+            p.columns = d;
             p.ldy = (int) cross_key_stride(b);
             p.rows_per_group = cross_rows;
             p.group_stride = cross_stream_stride(b);
             p.wdtype = wdtype;
-            e = wsp::ops::tile_product(b->stream, p);
+            const hipError_t e = wsp::ops::products(b->stream, p, {b->cross_parts, b->cross_parts_bytes});
+            if (e != hipSuccess)
+                return hip_fail(b, e, "cross key/value projection");
         }
-        else
+    }
+    else
+        for (int l = 0; l < b->shape.layers; ++l)
+        {
+            const wsp_cross_tensors& L = layers[l];
+            float* keys = b->cross_keys + (size_t) l * cross_layer_stride(b);
+            float* values = b->cross_values + (size_t) l * cross_layer_stride(b);
+            hipError_t e = hipSuccess;
             for (int c = 0; c < b->streams && e == hipSuccess; ++c)
             {
                 const float* x = encoder_rows + (size_t) c * cross_rows * d;

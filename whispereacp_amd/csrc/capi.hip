@@ -81,25 +81,30 @@ int wsp_hip_ctx_create(const wsp_decoder_shape* shape, int device, void* stream,
             floats = std::max(floats, wsp::ops::attention_workspace_floats(shape->heads, q, longest,
                                                                            head_width));
         ctx->attention_floats = std::max<size_t>(floats, 1);
-        const size_t held = std::max(ctx->attention_floats, wsp::ops::kQueryAttentionFloats);
-        status = hip_status(ctx, hipMalloc(&ctx->attention_workspace, held * sizeof(float)), "attention workspace");
-        // The prompt attention's per-head counters start at zero (each launch
-        // leaves them zero again).
+        ctx->argmax_candidates =
+            (size_t) shape->max_positions * wsp::ops::argmax_groups(shape->vocabulary_size);
+        ctx->parts_bytes = wsp::ops::parts_bytes(
+            std::max((size_t) shape->cross_positions * shape->width,
+                     (size_t) shape->max_positions * std::max(shape->width, shape->feed_forward_width)));
+        // One block: the attention workspace, the argmax candidates, the parts.
+        auto rounded = [](size_t bytes) { return (bytes + 255) / 256 * 256; };
+        const size_t attention = rounded(std::max(ctx->attention_floats, wsp::ops::kQueryAttentionFloats)
+                                         * sizeof(float));
+        const size_t candidates = rounded(ctx->argmax_candidates * sizeof(float));
+        char* block = nullptr;
+        status = hip_status(ctx, hipMalloc(&block, attention + 2 * candidates + ctx->parts_bytes), "workspace");
         if (status == WSP_OK)
+        {
+            ctx->attention_workspace = reinterpret_cast<float*>(block);
+            ctx->argmax_values = reinterpret_cast<float*>(block + attention);
+            ctx->argmax_indices = reinterpret_cast<uint32_t*>(block + attention + candidates);
+            ctx->parts = block + attention + 2 * candidates;
+            // The prompt attention's per-head counters start at zero (each launch
+            // leaves them zero again).
             status = hip_status(ctx, hipMemset(ctx->attention_workspace, 0,
                                                wsp::ops::kAttentionCounters * sizeof(unsigned int)),
                                 "attention workspace");
-    }
-    if (status == WSP_OK)
-    {
-        ctx->argmax_candidates =
-            (size_t) shape->max_positions * wsp::ops::argmax_groups(shape->vocabulary_size);
-        status = hip_status(ctx, hipMalloc(&ctx->argmax_values, ctx->argmax_candidates * sizeof(float)),
-                            "argmax workspace");
-        if (status == WSP_OK)
-            status = hip_status(ctx,
-                                hipMalloc(&ctx->argmax_indices, ctx->argmax_candidates * sizeof(uint32_t)),
-                                "argmax workspace");
+        }
     }
     if (status == WSP_OK)
         status = wsp::fused_prepare(ctx);
@@ -118,9 +123,7 @@ void wsp_hip_ctx_destroy(wsp_hip_ctx* ctx)
         return;
     hipSetDevice(ctx->device);
     wsp::fused_release(ctx);
-    hipFree(ctx->attention_workspace);
-    hipFree(ctx->argmax_values);
-    hipFree(ctx->argmax_indices);
+    hipFree(ctx->attention_workspace); // (the whole block)
     delete ctx;
 }
 
@@ -147,8 +150,53 @@ int wsp_hip_linear(wsp_hip_ctx* ctx, const float* x, int rows, int inner, const 
     if (!valid_dtype(wdtype) || (flags & ~(WSP_LINEAR_GELU | WSP_LINEAR_RESIDUAL)) != 0)
         return fail(ctx, WSP_ERR_ARGUMENT, "linear: unknown weight storage %d or flags %d", wdtype,
                     flags);
-    return hip_status(ctx, wsp::ops::linear(ctx->stream, x, rows, inner, weight, wdtype, bias, y, out, flags),
+    return hip_status(ctx,
+                      wsp::ops::linear(ctx->stream, x, rows, inner, weight, wdtype, bias, y, out, flags,
+                                       {ctx->parts, ctx->parts_bytes}),
                       "linear");
+}
+
+int wsp_hip_linear_many(wsp_hip_ctx* ctx, const float* x, int rows, int inner, const wsp_linear_target* targets,
+                        int count, int wdtype, int out)
+{
+    if (ctx == nullptr)
+        return WSP_ERR_ARGUMENT;
+    if (x == nullptr || targets == nullptr || count <= 0)
+        return fail(ctx, WSP_ERR_ARGUMENT, "linear: null input or no weights");
+    if (rows <= 0 || inner <= 0 || out <= 0)
+        return fail(ctx, WSP_ERR_ARGUMENT, "linear: extents %d x %d -> %d must be positive", rows,
+                    inner, out);
+    if (!valid_dtype(wdtype))
+        return fail(ctx, WSP_ERR_ARGUMENT, "linear: unknown weight storage %d", wdtype);
+    for (int i = 0; i < count; ++i)
+        if (targets[i].weight == nullptr || targets[i].y == nullptr)
+            return fail(ctx, WSP_ERR_ARGUMENT, "linear: null weight or output");
+    const wsp::ops::Scratch scratch {ctx->parts, ctx->parts_bytes};
+    hipError_t e = hipSuccess;
+    if (rows <= wsp::ops::kSplitRowLimit)
+    {
+        for (int i = 0; i < count && e == hipSuccess; ++i)
+            e = wsp::ops::linear(ctx->stream, x, rows, inner, targets[i].weight, wdtype, targets[i].bias, targets[i].y,
+                                 out, 0, scratch);
+        return hip_status(ctx, e, "linear");
+    }
+    wsp::ops::ProductMatrix matrices[wsp::ops::kMaxMatrices];
+    for (int first = 0; first < count && e == hipSuccess; first += wsp::ops::kMaxMatrices)
+    {
+        wsp::ops::Products p {};
+        p.x = x;
+        p.rows = rows;
+        p.inner = inner;
+        p.matrices = matrices;
+        p.count = std::min(count - first, wsp::ops::kMaxMatrices);
+        p.columns = out;
+        p.ldy = out;
+        p.wdtype = wdtype;
+        for (int i = 0; i < p.count; ++i)
+            matrices[i] = {targets[first + i].weight, targets[first + i].bias, targets[first + i].y, 1.f};
+        e = wsp::ops::products(ctx->stream, p, scratch);
+    }
+    return hip_status(ctx, e, "linear");
 }
 
 int wsp_hip_layernorm(wsp_hip_ctx* ctx, const float* x, const float* gamma, const float* beta,

@@ -21,6 +21,11 @@ struct wsp_hip_ctx
     uint32_t* argmax_indices = nullptr;
     size_t argmax_candidates = 0;
 
+    // A product's input as 16-bit parts (ops::Scratch): the cross projection's
+    // encoder rows, a prompt's rows of the widest layer.
+    void* parts = nullptr;
+    size_t parts_bytes = 0;
+
     void* fused = nullptr; // fused-step state (fused_step.hip)
 
     // wsp_hip_step_report_next: the host pair the next sampling step writes

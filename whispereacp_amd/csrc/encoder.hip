@@ -15,7 +15,7 @@
 // adds the bias, applies GELU and — for conv2 — adds the positional rows the
 // output buffer was filled with. The projections, LayerNorms and attention
 // are the library's per-op kernels; their 16-bit-weight products run on the
-// matrix cores (tile_product_kernel) over 1500-row operands.
+// matrix cores over 1500-row operands.
 #include "../../include/wsp_hip.h"
 #include "device_common.h"
 #include "ops.h"
@@ -500,8 +500,8 @@ int encoder_hip(wsp_encoder* e, hipError_t status, const char* what)
 bool pre_split_shape(int wdtype, int d, int f)
 {
     namespace ops = wsp::ops;
-    return d % 8 == 0 && ops::layernorm_parts_fits(d) && ops::split_product_fits(wdtype, d, 3 * d, d, 2 * d)
-           && ops::split_product_fits(wdtype, d, f, f, f) && ops::split_product_fits(wdtype, f, d, d, d);
+    return d % 8 == 0 && ops::layernorm_parts_fits(d) && ops::split_product_fits(wdtype, d, d)
+           && ops::split_product_fits(wdtype, d, f) && ops::split_product_fits(wdtype, f, d);
 }
 
 hipError_t encoder_allocate(wsp_encoder* e, float** out, size_t floats)
@@ -691,18 +691,19 @@ int wsp_encoder_encode(wsp_encoder* e, const wsp_encoder_tensors* T, const float
         p.part_stride = stride;
         p.rows = positions;
         p.inner = inner;
-        p.w0 = w;
-        p.out = out;
-        p.bias0 = bias;
-        p.y0 = y;
+        p.count = 1;
+        p.columns = out;
+        p.matrix[0] = {w, bias, y, unscale(stored_scale)};
         p.ldy = out;
         p.flags = flags;
         p.out_parts = out_parts;
         p.out_part_stride = ff_part_stride;
         p.wdtype = wt;
-        p.scale0 = unscale(stored_scale);
         return ops::split_product(st, p);
     };
+    // (Products that do not run over stored parts may store them there themselves.)
+    const size_t window_rows = (size_t) window_positions;
+    const ops::Scratch scratch {e->ff_parts, ops::parts_bytes(window_rows * f)};
     for (int l = 0; l < s.layers; ++l)
     {
         const wsp_encoder_layer_tensors& L = T->layers[l];
@@ -721,22 +722,13 @@ int wsp_encoder_encode(wsp_encoder* e, const wsp_encoder_tensors* T, const float
             p.part_stride = part_stride;
             p.rows = positions;
             p.inner = d;
-            p.w0 = L.q_w;
-            p.w1 = L.k_w;
-            p.w2 = L.v_w;
-            p.split = d;
-            p.split2 = 2 * d;
-            p.out = 3 * d;
-            p.bias0 = L.q_b;
-            p.bias2 = L.v_b;
-            p.y0 = e->q;
-            p.y1 = e->k;
-            p.y2 = e->v;
+            p.count = 3;
+            p.columns = d;
+            p.matrix[0] = {L.q_w, L.q_b, e->q, unscale(L.q_scale)};
+            p.matrix[1] = {L.k_w, nullptr, e->k, unscale(L.k_scale)};
+            p.matrix[2] = {L.v_w, L.v_b, e->v, unscale(L.v_scale)};
             p.ldy = d;
             p.wdtype = wt;
-            p.scale0 = unscale(L.q_scale);
-            p.scale1 = unscale(L.k_scale);
-            p.scale2 = unscale(L.v_scale);
             if (d / heads == kFlashWidth)
             {
                 // The attention takes k and v as fp16 halves.
@@ -749,25 +741,19 @@ int wsp_encoder_encode(wsp_encoder* e, const wsp_encoder_tensors* T, const float
         else
         {
             // q, k and v side by side in one launch: three times the blocks of one.
-            ops::TileProduct p {};
+            const ops::ProductMatrix matrices[] = {{L.q_w, L.q_b, e->q, 1.f},
+                                                   {L.k_w, nullptr, e->k, 1.f},
+                                                   {L.v_w, L.v_b, e->v, 1.f}};
+            ops::Products p {};
             p.x = e->normed;
             p.rows = positions;
             p.inner = d;
-            p.w0 = L.q_w;
-            p.w1 = L.k_w;
-            p.w2 = L.v_w;
-            p.split = d;
-            p.split2 = 2 * d;
-            p.out = 3 * d;
-            p.bias0 = L.q_b;
-            p.bias2 = L.v_b;
-            p.y0 = e->q;
-            p.y1 = e->k;
-            p.y2 = e->v;
+            p.matrices = matrices;
+            p.count = 3;
+            p.columns = d;
             p.ldy = d;
-            p.rows_per_group = positions;
             p.wdtype = wt;
-            status = ops::product(st, p);
+            status = ops::products(st, p, scratch);
         }
         if (status != hipSuccess)
             return encoder_hip(e, status, "self-attention projections");
@@ -843,7 +829,7 @@ int wsp_encoder_encode(wsp_encoder* e, const wsp_encoder_tensors* T, const float
                                        ops::kProductResidual, nullptr, L.out_scale);
         }
         else
-            status = ops::linear(st, e->att, positions, d, L.out_w, wt, L.out_b, e->hidden, d, 2);
+            status = ops::linear(st, e->att, positions, d, L.out_w, wt, L.out_b, e->hidden, d, 2, scratch);
         if (status != hipSuccess)
             return encoder_hip(e, status, "attention output");
         status = split ? ops::layernorm_parts(st, e->hidden, L.final_norm_w, L.final_norm_b, e->parts, part_stride,
@@ -859,8 +845,8 @@ int wsp_encoder_encode(wsp_encoder* e, const wsp_encoder_tensors* T, const float
                 status = split_product(e->ff_parts, ff_part_stride, f, L.fc2_w, L.fc2_b, e->hidden, d,
                                        ops::kProductResidual, nullptr, L.fc2_scale);
         }
-        else if ((status = ops::linear(st, e->normed, positions, d, L.fc1_w, wt, L.fc1_b, e->ff, f, 1)) == hipSuccess)
-            status = ops::linear(st, e->ff, positions, f, L.fc2_w, wt, L.fc2_b, e->hidden, d, 2);
+        else if ((status = ops::linear(st, e->normed, positions, d, L.fc1_w, wt, L.fc1_b, e->ff, f, 1, scratch)) == hipSuccess)
+            status = ops::linear(st, e->ff, positions, f, L.fc2_w, wt, L.fc2_b, e->hidden, d, 2, scratch);
         if (status != hipSuccess)
             return encoder_hip(e, status, "feed-forward");
     }

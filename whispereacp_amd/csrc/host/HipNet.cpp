@@ -5,7 +5,9 @@
 #include "../../../include/whispereacp/HipNet.h"
 #include "host_common.h"
 
+#include <array>
 #include <cmath>
+#include <functional>
 
 #include <stdexcept>
 #include <string>
@@ -399,8 +401,8 @@ void HipNet::end()
     try
     {
         place();
-        for (const Instruction& instruction : program)
-            issue(instruction);
+        for (std::size_t i = 0; i < program.size();)
+            i += issueShared(i);
     }
     catch (...)
     {
@@ -465,6 +467,51 @@ void HipNet::place()
             held[(std::size_t) (scratchClasses[(std::size_t) v.cls].first + v.buffer)] = 0;
         }
     }
+}
+
+// How many instructions from `first` on were issued: plain projections of one
+// input, one after the other, go out together where their weights agree in
+// storage and extents and their outputs lie apart.
+std::size_t HipNet::issueShared(std::size_t first)
+{
+    auto plain = [&](const Instruction& op) { return op.code == Opcode::project && !op.gelu; };
+    const Instruction& lead = program[first];
+    std::size_t end = first + 1;
+    if (plain(lead))
+    {
+        const Value& in = values[(std::size_t) lead.in[0]];
+        const int outputs = lead.weight->dimension(0);
+        const std::size_t span = (std::size_t) in.shape.rows() * (std::size_t) outputs;
+        std::array<wsp_linear_target, 64> targets;
+        std::size_t count = 0;
+        auto add = [&](const Instruction& op) {
+            if (count == targets.size())
+                return false;
+            float* y = static_cast<float*>(values[(std::size_t) op.dst].range.data())
+                       + (std::size_t) op.dstRow * (std::size_t) outputs;
+            for (std::size_t i = 0; i < count; ++i)
+                if (std::less<const float*>()(y, targets[i].y + span)
+                    && std::less<const float*>()(targets[i].y, y + span))
+                    return false;
+            targets[count++] = {op.weight->data(),
+                                op.bias != nullptr ? static_cast<const float*>(op.bias->data()) : nullptr, y};
+            return true;
+        };
+        add(lead);
+        while (end < program.size() && plain(program[end]) && program[end].in[0] == lead.in[0]
+               && program[end].weight->type == lead.weight->type && program[end].weight->dimension(0) == outputs
+               && add(program[end]))
+            ++end;
+        if (end - first > 1)
+        {
+            check(wsp_hip_linear_many(ctx, static_cast<const float*>(in.range.data()), in.shape.rows(),
+                                      in.shape.columns(), targets.data(), (int) count,
+                                      wsp_dtype_of(lead.weight->type), outputs));
+            return end - first;
+        }
+    }
+    issue(lead);
+    return 1;
 }
 
 void HipNet::issue(const Instruction& op)

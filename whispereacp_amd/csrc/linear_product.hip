@@ -22,12 +22,14 @@
 // as long as both operands share it), and the eight partial tiles are added in
 // wave order through LDS, so the result does not depend on timing. SPLIT takes
 // 16-bit weights in their own type with X cut into exact 16-bit parts (as
-// tile_product_kernel does), otherwise everything is fp32.
+// split_product's), otherwise everything is fp32.
 //
 // W is the matrix cores' row operand, X their column operand: a lane ends up
 // with four consecutive outputs of one row.
 #include "device_common.h"
 #include "ops.h"
+
+#include <algorithm>
 
 namespace wsp::ops
 {
@@ -36,6 +38,18 @@ namespace
 typedef uint16_t u16;
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+
+// Up to three matrices a launch here.
+constexpr int kMatrices = 3;
+struct RowProduct
+{
+    const float* x;
+    int rows, inner, columns, out; // out: every matrix's columns together
+    ProductMatrix matrix[kMatrices];
+    int ldy, rows_per_group;
+    size_t group_stride;
+    int flags;
+};
 
 // Output column n's matrix, and its column there.
 struct Column
@@ -46,16 +60,16 @@ struct Column
     int c;
 };
 
-__device__ __forceinline__ Column column_of(const TileProduct& a, int n)
+__device__ __forceinline__ Column column_of(const RowProduct& a, int n)
 {
-    if (n < a.split)
-        return {a.w0, a.bias0, a.y0, n};
-    if (n < a.split2)
-        return {a.w1, a.bias1, a.y1, n - a.split};
-    return {a.w2, a.bias2, a.y2, n - a.split2};
+    if (n < a.columns)
+        return {a.matrix[0].w, a.matrix[0].bias, a.matrix[0].y, n};
+    if (n < 2 * a.columns)
+        return {a.matrix[1].w, a.matrix[1].bias, a.matrix[1].y, n - a.columns};
+    return {a.matrix[2].w, a.matrix[2].bias, a.matrix[2].y, n - 2 * a.columns};
 }
 
-__device__ __forceinline__ void store_output(const TileProduct& a, int row, int n, float v)
+__device__ __forceinline__ void store_output(const RowProduct& a, int row, int n, float v)
 {
     const Column col = column_of(a, n);
     if (col.bias != nullptr)
@@ -135,7 +149,7 @@ __device__ __forceinline__ int slot(int r, int c)
 }
 
 template <int WT, bool VEC>
-__global__ void __launch_bounds__(kTileThreads, 2) fp32_tile_kernel(TileProduct a)
+__global__ void __launch_bounds__(kTileThreads, 2) fp32_tile_kernel(RowProduct a)
 {
     constexpr int TM = kTileRows, TN = kTileColumns, KS = kTileStep, CH = KS / 4;
     constexpr int MT = TM / 32, NT = TN / 32; // 16 x 16 tiles a wave, waves 2 x 2
@@ -281,7 +295,7 @@ struct RowChunk
 };
 
 template <int WT, int MT, int NT, bool SPLIT>
-__global__ void __launch_bounds__(kRowWaves * kWave) row_product_kernel(TileProduct a)
+__global__ void __launch_bounds__(kRowWaves * kWave) row_product_kernel(RowProduct a)
 {
     static_assert(!SPLIT || WT != kF32, "parts go with 16-bit weights");
     constexpr int P = WT == kF16 ? 2 : 3;
@@ -445,15 +459,16 @@ bool aligned(const void* p, size_t bytes)
 }
 
 // Whether X and every matrix take whole vector loads of `run` values.
-bool whole_vectors(const TileProduct& a, int run)
+bool whole_vectors(const Products& a, int run)
 {
-    const size_t bytes = a.wdtype == kF32 ? 16 : 2 * run;
-    return a.inner % run == 0 && aligned(a.x, 16) && aligned(a.w0, bytes) && (a.split >= a.out || aligned(a.w1, bytes))
-           && (a.split2 >= a.out || aligned(a.w2, bytes));
+    bool fits = a.inner % run == 0 && aligned(a.x, 16);
+    for (int i = 0; i < a.count; ++i)
+        fits = fits && aligned(a.matrices[i].w, a.wdtype == kF32 ? 16 : 2 * run);
+    return fits;
 }
 
 template <int WT, bool VEC>
-hipError_t launch_tile(hipStream_t stream, const TileProduct& a)
+hipError_t launch_tile(hipStream_t stream, const RowProduct& a)
 {
     hipLaunchKernelGGL((fp32_tile_kernel<WT, VEC>), dim3((a.out + kTileColumns - 1) / kTileColumns,
                                                          (a.rows + kTileRows - 1) / kTileRows),
@@ -462,7 +477,7 @@ hipError_t launch_tile(hipStream_t stream, const TileProduct& a)
 }
 
 template <int WT, int MT, int NT, bool SPLIT>
-hipError_t launch_row(hipStream_t stream, const TileProduct& a)
+hipError_t launch_row(hipStream_t stream, const RowProduct& a)
 {
     hipLaunchKernelGGL((row_product_kernel<WT, MT, NT, SPLIT>),
                        dim3((a.out + 16 * NT - 1) / (16 * NT), (a.rows + 16 * MT - 1) / (16 * MT)),
@@ -470,14 +485,67 @@ hipError_t launch_row(hipStream_t stream, const TileProduct& a)
     return hipGetLastError();
 }
 
-// 16-bit weights with X in 16-bit parts: short products by row_product_kernel,
-// the others by tile_product. The line is at 2^17 outputs: 96 x 768 -> 768 ran
-// 5.3 us against 13.5 for tile_product, 96 x 3072 -> 768 13.2 against 41,
-// 200 x 1280 -> 5120 41 against 23.
-template <int WT>
-hipError_t parts_product(hipStream_t stream, const TileProduct& a)
+RowProduct row_product(const Products& p, int first, int count)
 {
-    return (long long) a.rows * a.out <= 1 << 17 ? launch_row<WT, 1, 2, true>(stream, a) : tile_product(stream, a);
+    RowProduct a {};
+    a.x = p.x;
+    a.rows = p.rows;
+    a.inner = p.inner;
+    a.columns = p.columns;
+    a.out = count * p.columns;
+    for (int i = 0; i < count; ++i)
+        a.matrix[i] = p.matrices[first + i];
+    a.ldy = p.ldy;
+    a.rows_per_group = p.rows_per_group;
+    a.group_stride = p.group_stride;
+    a.flags = p.flags;
+    return a;
+}
+
+SplitProduct split_product_of(const Products& p, const void* parts, size_t part_stride, int first, int count)
+{
+    SplitProduct a {};
+    a.parts = parts;
+    a.part_stride = part_stride;
+    a.rows = p.rows;
+    a.inner = p.inner;
+    a.count = count;
+    a.columns = p.columns;
+    for (int i = 0; i < count; ++i)
+        a.matrix[i] = p.matrices[first + i];
+    a.ldy = p.ldy;
+    a.rows_per_group = p.rows_per_group;
+    a.group_stride = p.group_stride;
+    a.flags = p.flags;
+    a.wdtype = p.wdtype;
+    return a;
+}
+
+// 16-bit weights with X in 16-bit parts. From 2^17 outputs on (every matrix
+// together) X is stored as parts once and every matrix goes through
+// split_product in launches of up to 64; fewer, and what the scratch does not
+// hold, through row_product_kernel: 96 x 768 -> 768 runs 5.3 us there, 96 x 3072
+// -> 768 13; 200 x 5120 -> 1280 39, against 20 with the parts' launch.
+template <int WT>
+hipError_t parts_product(hipStream_t stream, const Products& p, const Scratch& scratch)
+{
+    const long long outputs = (long long) p.rows * p.columns * p.count;
+    const size_t values = (size_t) p.rows * p.inner;
+    hipError_t e = hipSuccess;
+    if (outputs > 1 << 17 && split_product_fits(p.wdtype, p.inner, p.columns) && parts_bytes(values) <= scratch.bytes
+        && values < 1u << 29 && (size_t) p.columns * p.inner < 1u << 30) // (32-bit byte offsets)
+    {
+        e = split_rows(stream, p.x, values, p.wdtype, scratch.data, values);
+        for (int i = 0; i < p.count && e == hipSuccess; i += kMaxMatrices)
+            e = split_product(stream, split_product_of(p, scratch.data, values, i, std::min(kMaxMatrices, p.count - i)));
+        return e;
+    }
+    for (int i = 0; i < p.count && e == hipSuccess; i += kMatrices)
+    {
+        const RowProduct a = row_product(p, i, std::min(kMatrices, p.count - i));
+        e = outputs <= 1 << 17 ? launch_row<WT, 1, 2, true>(stream, a) : launch_row<WT, 2, 4, true>(stream, a);
+    }
+    return e;
 }
 
 // fp32 arithmetic. Up to 16 rows, and while 32 x 32 tiles would not give each
@@ -486,43 +554,55 @@ hipError_t parts_product(hipStream_t stream, const TileProduct& a)
 // otherwise take split_product's direct-to-LDS form (1500 x 2048 -> 512 35 us
 // against 48 staged through registers), the rest fp32_tile_kernel.
 template <int WT>
-hipError_t fp32_product(hipStream_t stream, const TileProduct& a)
+hipError_t fp32_product(hipStream_t stream, const Products& p)
 {
     const long long units = compute_units();
-    auto blocks = [&](int tm, int tn) { return (long long) ((a.rows + tm - 1) / tm) * ((a.out + tn - 1) / tn); };
-    if ((a.rows <= kSplitRowLimit || blocks(32, 32) < units) && whole_vectors(a, 8))
+    const int out = p.count * p.columns;
+    auto blocks = [&](int tm, int tn) { return (long long) ((p.rows + tm - 1) / tm) * ((out + tn - 1) / tn); };
+    const bool few = (p.rows <= kSplitRowLimit || blocks(32, 32) < units) && whole_vectors(p, 8);
+    hipError_t e = hipSuccess;
+    if (!few && WT == kF32 && p.count <= kMaxMatrices)
     {
-        if (a.rows > 16)
-            return launch_row<WT, 2, 1, false>(stream, a);
-        // (16 x 1280 -> 5120: 9.8 us with 32 columns a block, 11.3 with 16; 8 x 768 -> 3072: 6.1 and 4.4)
-        return blocks(16, 16) > units ? launch_row<WT, 1, 2, false>(stream, a)
-                                      : launch_row<WT, 1, 1, false>(stream, a);
+        const SplitProduct a = split_product_of(p, p.x, 0, 0, p.count);
+        if (fp32_split_fits(a))
+            return fp32_split(stream, a);
     }
-    if (WT == kF32 && fp32_split_fits(a))
-        return fp32_split(stream, a);
-    return whole_vectors(a, 4) ? launch_tile<WT, true>(stream, a) : launch_tile<WT, false>(stream, a);
+    for (int i = 0; i < p.count && e == hipSuccess; i += kMatrices)
+    {
+        const RowProduct a = row_product(p, i, std::min(kMatrices, p.count - i));
+        if (few && p.rows > 16)
+            e = launch_row<WT, 2, 1, false>(stream, a);
+        else if (few) // (16 x 1280 -> 5120: 9.8 us with 32 columns a block, 11.3 with 16; 8 x 768 -> 3072: 6.1 and 4.4)
+            e = blocks(16, 16) > units ? launch_row<WT, 1, 2, false>(stream, a)
+                                       : launch_row<WT, 1, 1, false>(stream, a);
+        else
+            e = whole_vectors(p, 4) ? launch_tile<WT, true>(stream, a) : launch_tile<WT, false>(stream, a);
+    }
+    return e;
 }
 } // namespace
 
-bool row_product_fits(const TileProduct& product)
+bool parts_fit(int wdtype, int inner, int columns, const void* x)
+{
+    return (wdtype == kF16 || wdtype == kBF16) && inner % 32 == 0 && columns % 128 == 0 && aligned(x, 16);
+}
+
+bool row_product_fits(const Products& product)
 {
     return product.rows <= kSplitRowLimit && whole_vectors(product, 8);
 }
 
-hipError_t product(hipStream_t stream, const TileProduct& given)
+hipError_t products(hipStream_t stream, const Products& given, const Scratch& scratch)
 {
-    TileProduct a = given;
-    if (a.split2 <= 0 || a.split2 > a.out)
-        a.split2 = a.out;
-    if (a.split <= 0 || a.split > a.split2)
-        a.split = a.split2;
-    const bool parts = a.rows > kSplitRowLimit && tile_product_fits(a.wdtype, a.inner, a.out, a.split, a.x)
-                       && a.split2 % 128 == 0;
-    switch (a.wdtype)
+    Products p = given;
+    if (p.rows_per_group <= 0)
+        p.rows_per_group = p.rows;
+    const bool parts = p.rows > kSplitRowLimit && parts_fit(p.wdtype, p.inner, p.columns, p.x);
+    switch (p.wdtype)
     {
-        case kF32: return fp32_product<kF32>(stream, a);
-        case kF16: return parts ? parts_product<kF16>(stream, a) : fp32_product<kF16>(stream, a);
-        default: return parts ? parts_product<kBF16>(stream, a) : fp32_product<kBF16>(stream, a);
+        case kF32: return fp32_product<kF32>(stream, p);
+        case kF16: return parts ? parts_product<kF16>(stream, p, scratch) : fp32_product<kF16>(stream, p);
+        default: return parts ? parts_product<kBF16>(stream, p, scratch) : fp32_product<kBF16>(stream, p);
     }
 }
 } // namespace wsp::ops

@@ -13,65 +13,27 @@ constexpr int kSplitRowLimit = 16;
 constexpr int kMaxHeadWidth = 64;
 constexpr int kAttentionChunkKeys = 1024; // longest key chunk one workgroup scores
 
-hipError_t linear(hipStream_t stream, const float* x, int rows, int inner, const void* weight,
-                  int wdtype, const float* bias, float* y, int out, int flags);
-
-// The matrix-core tall product (mfma_product.hip): y = X·Wᵀ (+ bias, GELU,
-// residual as in `flags`) for fp32 X [rows, inner] and 16-bit W. Output
-// columns n < split read W rows from w0 and write y0 (bias0); the rest read
-// w1 row n - split and write y1 (bias1) — the key and value projections in one
-// launch. Output row r of column c lands at
-// (r / rows_per_group)·group_stride + (r % rows_per_group)·ldy + c.
-struct TileProduct
+// One of the matrices side by side in a product: W [columns][inner], its bias
+// (or null), its output, and the factor its sums are multiplied by before the
+// bias (the reciprocal of the power of two its stored weights carry, exact; 1
+// for weights stored as they are).
+struct ProductMatrix
 {
-    const float* x;
-    int rows, inner;
-    // Up to three weight matrices side by side: columns [0, split) read w0,
-    // [split, split2) w1 and [split2, out) w2, each with its bias and output
-    // (split2 0: two matrices, w1 running to out).
-    const void* w0;
-    const void* w1;
-    int split, out;
-    const float* bias0;
-    const float* bias1;
-    float* y0;
-    float* y1;
-    int ldy;
-    int rows_per_group;
-    size_t group_stride;
-    int flags;
-    int wdtype;
-    const void* w2;
-    const float* bias2;
-    float* y2;
-    int split2;
+    const void* w = nullptr;
+    const float* bias = nullptr;
+    float* y = nullptr;
+    float scale = 1.f;
 };
+constexpr int kMaxMatrices = 64;
 
-// y = X·Wᵀ for any rows, extents and weight storage (linear_product.hip): what
-// tile_product fits, in its arithmetic (16-bit parts), else in fp32.
-hipError_t product(hipStream_t stream, const TileProduct& product);
-// Whether a product of at most kSplitRowLimit rows goes there in one launch.
-bool row_product_fits(const TileProduct& product);
-// fp32 weights in whole 16-byte runs (split_product.hip).
-bool fp32_split_fits(const TileProduct& product);
-hipError_t fp32_split(hipStream_t stream, const TileProduct& product);
-
-// 16-bit weights, inner % 32 == 0, out and split (and split2) multiples of
-// 128, X 16-byte aligned.
-bool tile_product_fits(int wdtype, int inner, int out, int split, const void* x);
-hipError_t tile_product(hipStream_t stream, const TileProduct& product);
-
-hipError_t layernorm(hipStream_t stream, const float* x, const float* gamma, const float* beta,
-                     float* y, int rows, int width, float eps);
-
-// The encoder's products over pre-split activations (split_product.hip):
-// y = X·Wᵀ where X [rows, inner] is held as exact 16-bit parts (three bf16
-// parts for bf16 W, fp16 hi + lo for fp16 W), part p at
-// parts + p·part_stride + r·inner. Columns [0, split) read w0 (bias0, y0),
-// [split, split2) w1 and [split2, out) w2, each matrix's own column index c;
-// row r of a column lands at y·[r·ldy + c] (+= with kProductResidual, after
-// GELU with kProductGelu), or, with out_parts set, as the parts of the value
-// (one matrix only, rows of `out` values, part p at out_parts + p·out_part_stride).
+// The products over X as split_product's kernel reads it: exact 16-bit parts
+// for 16-bit W (three bf16 parts, or fp16 hi + lo), part p at
+// parts + p·part_stride + r·inner, or fp32 X for fp32 W. `count` matrices of
+// `columns` columns share the launch. Row r of a column lands at
+// y[(r / rows_per_group)·group_stride + (r % rows_per_group)·ldy + c]
+// (rows_per_group 0: one group; += with kProductResidual, after GELU with
+// kProductGelu), or, with out_parts set, as the parts of the value (one matrix
+// only, rows of `columns` values, part p at out_parts + p·out_part_stride).
 constexpr int kProductGelu = 1;
 constexpr int kProductResidual = 2;
 struct SplitProduct
@@ -79,47 +41,81 @@ struct SplitProduct
     const void* parts;
     size_t part_stride;
     int rows, inner;
-    const void* w0;
-    const void* w1;
-    const void* w2;
-    int split, split2, out;
-    const float* bias0;
-    const float* bias1;
-    const float* bias2;
-    float* y0;
-    float* y1;
-    float* y2;
+    int count, columns;
+    ProductMatrix matrix[kMaxMatrices];
     int ldy;
+    int rows_per_group;
+    size_t group_stride;
     int flags;
     void* out_parts;
     size_t out_part_stride;
     int wdtype;
-    // Columns [split, split2) (y1_halves) and [split2, out) (y2_halves_t), when
-    // set, go out as fp16 hi = fp16(v) and lo = fp16(v - hi) instead of fp32:
-    // hi of row r, column c at y1_halves[r·width + c], lo halves_pitch·width
-    // further; y2_halves_t transposed, hi at [c·halves_pitch + r]. (The
-    // encoder's keys and values for its attention.)
+    // Matrix 1 (y1_halves) and matrix 2 (y2_halves_t), when set, go out as fp16
+    // hi = fp16(v) and lo = fp16(v - hi) instead of fp32: hi of row r, column c
+    // at y1_halves[r·columns + c], lo halves_pitch·columns further; y2_halves_t
+    // transposed, hi at [c·halves_pitch + r]. (The encoder's keys and values
+    // for its attention.)
     void* y1_halves;
     void* y2_halves_t;
     int halves_pitch;
-    // Each matrix's sums are multiplied by its factor before the bias: the
-    // reciprocal of the power of two its stored weights carry (exact), 1 for
-    // weights stored as they are.
-    float scale0 = 1.f, scale1 = 1.f, scale2 = 1.f;
 };
 
-// 16-bit weights, inner % 64 == 0, out, split and split2 multiples of 128.
-bool split_product_fits(int wdtype, int inner, int out, int split, int split2);
+// 16-bit weights, inner a multiple of 64, columns of 128.
+bool split_product_fits(int wdtype, int inner, int columns);
 hipError_t split_product(hipStream_t stream, const SplitProduct& product);
+// fp32 weights: rows in whole 16-byte runs, several matrices in multiples of
+// 64 columns.
+bool fp32_split_fits(const SplitProduct& product);
+hipError_t fp32_split(hipStream_t stream, const SplitProduct& product);
+// count fp32 values (a multiple of 8) as parts for 16-bit weights of wdtype.
+hipError_t split_rows(hipStream_t stream, const float* x, size_t count, int wdtype, void* parts,
+                      size_t part_stride);
+
+// Memory for a product's input as 16-bit parts; products that would want more
+// read fp32 rows instead.
+struct Scratch
+{
+    void* data = nullptr;
+    size_t bytes = 0;
+};
+// Bytes for the parts of `values` fp32 values (three 16-bit parts at most).
+constexpr size_t parts_bytes(size_t values)
+{
+    return 6 * values;
+}
+
+// y = X·Wᵀ for any rows, extents and weight storage (linear_product.hip), any
+// number of matrices of `columns` columns over the same rows. More than
+// kSplitRowLimit rows of 16-bit weights in whole parts (parts_fit) are computed
+// in 16-bit parts, everything else in fp32.
+bool parts_fit(int wdtype, int inner, int columns, const void* x);
+struct Products
+{
+    const float* x;
+    int rows, inner;
+    const ProductMatrix* matrices;
+    int count, columns;
+    int ldy;
+    int rows_per_group;  // as SplitProduct's
+    size_t group_stride;
+    int flags;
+    int wdtype;
+};
+hipError_t products(hipStream_t stream, const Products& given, const Scratch& scratch);
+// Whether a product of at most kSplitRowLimit rows goes there in one launch.
+bool row_product_fits(const Products& product);
+
+hipError_t linear(hipStream_t stream, const float* x, int rows, int inner, const void* weight,
+                  int wdtype, const float* bias, float* y, int out, int flags, const Scratch& scratch = {});
+
+hipError_t layernorm(hipStream_t stream, const float* x, const float* gamma, const float* beta,
+                     float* y, int rows, int width, float eps);
+
 // LayerNorm rows (as layernorm) written as the parts of split_product's input;
 // widths that are multiples of 4 up to 2048 (layernorm_parts_fits).
 bool layernorm_parts_fits(int width);
 hipError_t layernorm_parts(hipStream_t stream, const float* x, const float* gamma, const float* beta, void* parts,
                            size_t part_stride, int rows, int width, float eps, int wdtype);
-// count fp32 values (a multiple of 8) as parts for 16-bit weights of wdtype.
-hipError_t split_rows(hipStream_t stream, const float* x, size_t count, int wdtype, void* parts,
-                      size_t part_stride);
-
 // Token ids at or past `vocabulary` poison their row with NaN.
 hipError_t embed(hipStream_t stream, const uint32_t* tokens, int count, const float* token_table,
                  const float* position_table, int first_position, float* y, int width,

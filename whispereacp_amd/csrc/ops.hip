@@ -839,25 +839,24 @@ hipError_t launch_gemv(hipStream_t stream, const float* x, int rows, int inner, 
 } // namespace
 
 hipError_t linear(hipStream_t stream, const float* x, int rows, int inner, const void* weight,
-                  int wdtype, const float* bias, float* y, int out, int flags)
+                  int wdtype, const float* bias, float* y, int out, int flags, const Scratch& scratch)
 {
-    TileProduct p {};
+    const ProductMatrix matrix {weight, bias, y, 1.f};
+    Products p {};
     p.x = x;
     p.rows = rows;
     p.inner = inner;
-    p.w0 = p.w1 = weight;
-    p.split = p.out = out;
-    p.bias0 = p.bias1 = bias;
-    p.y0 = p.y1 = y;
+    p.matrices = &matrix;
+    p.count = 1;
+    p.columns = out;
     p.ldy = out;
-    p.rows_per_group = rows;
     p.flags = flags;
     p.wdtype = wdtype;
     // Up to four rows the GEMV (a wave per output, one read of W); from five
     // on it would read W again for every four rows (16 x 768 -> 3072: four
     // launches of 4 us against one of 5).
     if (rows > kSplitRowLimit || (rows > 4 && row_product_fits(p)))
-        return product(stream, p);
+        return products(stream, p, scratch);
     switch (wdtype)
     {
         case kF32: return launch_gemv<kF32>(stream, x, rows, inner, weight, bias, y, out, flags);

@@ -244,11 +244,10 @@ __global__ void __launch_bounds__(T::kWaves * kWave) split_product_kernel(SplitP
     const int wm = wave / T::WN, wn = wave % T::WN;
     const int n_block = blockIdx.x * T::TN, m_block = blockIdx.y * T::TM;
     const int steps = (a.inner + kStep - 1) / kStep;
-    // The block's columns lie in one of the (up to three) matrices.
-    const int seg = n_block < a.split ? 0 : n_block < a.split2 ? 1 : 2;
-    const int seg_first = seg == 0 ? 0 : seg == 1 ? a.split : a.split2;
-    const void* w = seg == 0 ? a.w0 : seg == 1 ? a.w1 : a.w2;
-    const int width = seg == 0 ? a.split : seg == 1 ? a.split2 - a.split : a.out - a.split2;
+    // The block's columns lie in one of the matrices.
+    const int width = a.columns, seg = a.count > 1 ? n_block / width : 0, seg_first = seg * width;
+    const ProductMatrix& matrix = a.matrix[seg];
+    const void* w = matrix.w;
 
     // This wave's loads: load q = wave + waves·t of a stage covers 8 tile rows
     // (the parts' rows first, then W's); lane i moves row 8 q' + i / 8, chunk
@@ -350,11 +349,12 @@ __global__ void __launch_bounds__(T::kWaves * kWave) split_product_kernel(SplitP
     wait_loads<0>();
 
     // acc[mt][nt][r] of lane (g, li) is row li, column 4g + r of that 16 x 16 tile.
-    float* y = seg == 0 ? a.y0 : seg == 1 ? a.y1 : a.y2;
-    const float* bias = seg == 0 ? a.bias0 : seg == 1 ? a.bias1 : a.bias2;
-    const float scale = seg == 0 ? a.scale0 : seg == 1 ? a.scale1 : a.scale2;
+    float* y = matrix.y;
+    const float* bias = matrix.bias;
+    const float scale = matrix.scale;
     // Four columns a lane go out as one store; fp32 products may end inside them.
-    const bool quads = WT != kF32 || (width % 4 == 0 && a.ldy % 4 == 0 && reinterpret_cast<uintptr_t>(y) % 16 == 0);
+    const bool quads = width % 4 == 0 && a.ldy % 4 == 0 && a.group_stride % 4 == 0
+                       && reinterpret_cast<uintptr_t>(y) % 16 == 0;
 #pragma unroll
     for (int nt = 0; nt < NT; ++nt)
     {
@@ -420,9 +420,11 @@ __global__ void __launch_bounds__(T::kWaves * kWave) split_product_kernel(SplitP
                     }
                 }
             }
-            else if (quads)
+            else if (const size_t at = (size_t) (row / a.rows_per_group) * a.group_stride
+                                       + (size_t) (row % a.rows_per_group) * a.ldy + c;
+                     quads)
             {
-                float4v* o = reinterpret_cast<float4v*>(y + (size_t) row * a.ldy + c);
+                float4v* o = reinterpret_cast<float4v*>(y + at);
                 float4v sum = {v[0], v[1], v[2], v[3]};
                 if (a.flags & kProductResidual)
                     sum = *o + sum;
@@ -433,7 +435,7 @@ __global__ void __launch_bounds__(T::kWaves * kWave) split_product_kernel(SplitP
                 for (int r = 0; r < 4; ++r)
                     if (c + r < width)
                     {
-                        float* o = y + (size_t) row * a.ldy + c + r;
+                        float* o = y + at + r;
                         *o = a.flags & kProductResidual ? *o + v[r] : v[r];
                     }
         }
@@ -448,7 +450,7 @@ hipError_t launch(hipStream_t stream, const SplitProduct& a)
                                                           hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
     if (allowed != hipSuccess)
         return allowed;
-    hipLaunchKernelGGL((split_product_kernel<T, WT>), dim3((a.out + T::TN - 1) / T::TN, (a.rows + T::TM - 1) / T::TM),
+    hipLaunchKernelGGL((split_product_kernel<T, WT>), dim3((a.count * a.columns + T::TN - 1) / T::TN, (a.rows + T::TM - 1) / T::TM),
                        dim3(T::kWaves * kWave), bytes, stream, a);
     return hipGetLastError();
 }
@@ -477,8 +479,9 @@ template <int WT>
 hipError_t launch_tiles(hipStream_t stream, const SplitProduct& a)
 {
     const long long units = compute_units();
-    auto blocks = [&](int tm, int tn) { return (long long) ((a.rows + tm - 1) / tm) * (a.out / tn); };
-    if (a.out % 256 == 0 && a.split % 256 == 0 && a.split2 % 256 == 0 && 2 * blocks(128, 256) >= units)
+    const int out = a.count * a.columns;
+    auto blocks = [&](int tm, int tn) { return (long long) ((a.rows + tm - 1) / tm) * (out / tn); };
+    if (a.columns % 256 == 0 && 2 * blocks(128, 256) >= units)
         return launch<Tile<WT, 128, 256, 2, 4, 2>, WT>(stream, a);
     if (blocks(64, 128) > units)
         return launch<Tile<WT, 64, 128, 2, 4, 2>, WT>(stream, a);
@@ -490,10 +493,9 @@ hipError_t launch_tiles(hipStream_t stream, const SplitProduct& a)
 }
 } // namespace
 
-bool split_product_fits(int wdtype, int inner, int out, int split, int split2)
+bool split_product_fits(int wdtype, int inner, int columns)
 {
-    return (wdtype == kF16 || wdtype == kBF16) && inner % 64 == 0 && out % 128 == 0 && split % 128 == 0
-           && split2 % 128 == 0 && split <= split2 && split2 <= out;
+    return (wdtype == kF16 || wdtype == kBF16) && inner % 64 == 0 && columns % 128 == 0;
 }
 
 hipError_t split_rows(hipStream_t stream, const float* x, size_t count, int wdtype, void* parts, size_t part_stride)
@@ -532,13 +534,14 @@ hipError_t layernorm_parts(hipStream_t stream, const float* x, const float* gamm
 
 // fp32 X and W through the same kernel, one "part" of four-byte values:
 // v_mfma_f32_16x16x4_f32 in 32-wide steps.
-bool fp32_split_fits(const TileProduct& a)
+bool fp32_split_fits(const SplitProduct& a)
 {
     auto aligned = [](const void* p) { return reinterpret_cast<uintptr_t>(p) % 16 == 0; };
-    return a.wdtype == kF32 && a.inner % 4 == 0 && aligned(a.x) && aligned(a.w0) && a.rows_per_group >= a.rows
-           && (a.split >= a.out || (a.split % 64 == 0 && aligned(a.w1)))
-           && (a.split2 >= a.out || (a.split2 % 64 == 0 && aligned(a.w2)))
-           && (unsigned long long) std::max(a.rows, a.out) * a.inner < 1ull << 30; // 32-bit byte offsets
+    bool fits = a.wdtype == kF32 && a.inner % 4 == 0 && aligned(a.parts) && (a.count == 1 || a.columns % 64 == 0)
+                && (unsigned long long) std::max(a.rows, a.columns) * a.inner < 1ull << 30; // 32-bit byte offsets
+    for (int i = 0; i < a.count; ++i)
+        fits = fits && aligned(a.matrix[i].w);
+    return fits;
 }
 
 // 64 x 64 tiles, 32 x 64 or 32 x 32, whichever finishes first by its rounds
@@ -548,30 +551,16 @@ bool fp32_split_fits(const TileProduct& a)
 // 13.2, 13.1, 11.7; 512 -> 1536 30.4, 28.7, 30.6; 512 -> 2048 31.9, 33.3,
 // 38.6; 2048 -> 512 41.4, 41.3, 35.4; 3840 -> 1280 129, 134, 153 (247 as 64 x
 // 64 tiles of vector multiply-adds).
-hipError_t fp32_split(hipStream_t stream, const TileProduct& t)
+hipError_t fp32_split(hipStream_t stream, const SplitProduct& product)
 {
-    SplitProduct a {};
-    a.parts = t.x;
-    a.rows = t.rows;
-    a.inner = t.inner;
-    a.w0 = t.w0;
-    a.w1 = t.w1;
-    a.w2 = t.w2;
-    a.split = t.split;
-    a.split2 = t.split2;
-    a.out = t.out;
-    a.bias0 = t.bias0;
-    a.bias1 = t.bias1;
-    a.bias2 = t.bias2;
-    a.y0 = t.y0;
-    a.y1 = t.y1;
-    a.y2 = t.y2;
-    a.ldy = t.ldy;
-    a.flags = t.flags;
-    a.wdtype = kF32;
+    if (!fp32_split_fits(product))
+        return hipErrorInvalidValue;
+    SplitProduct a = product;
+    if (a.rows_per_group <= 0)
+        a.rows_per_group = a.rows;
     const long long units = compute_units();
     auto rounds = [&](int tm, int tn) {
-        return ((long long) ((a.rows + tm - 1) / tm) * ((a.out + tn - 1) / tn) + units - 1) / units;
+        return ((long long) ((a.rows + tm - 1) / tm) * ((a.count * a.columns + tn - 1) / tn) + units - 1) / units;
     };
     const double whole = 1.0 * rounds(64, 64), half = 0.535 * rounds(32, 64), quarter = 0.3 * rounds(32, 32);
     if (whole <= half && whole <= quarter)
@@ -583,13 +572,12 @@ hipError_t fp32_split(hipStream_t stream, const TileProduct& t)
 
 hipError_t split_product(hipStream_t stream, const SplitProduct& product)
 {
-    SplitProduct a = product;
-    if (a.split2 <= 0 || a.split2 > a.out)
-        a.split2 = a.out;
-    if (a.split <= 0 || a.split > a.split2)
-        a.split = a.split2;
-    if (!split_product_fits(a.wdtype, a.inner, a.out, a.split, a.split2))
+    if (!split_product_fits(product.wdtype, product.inner, product.columns) || product.count < 1
+        || product.count > kMaxMatrices)
         return hipErrorInvalidValue;
+    SplitProduct a = product;
+    if (a.rows_per_group <= 0)
+        a.rows_per_group = a.rows;
     return a.wdtype == kF16 ? launch_tiles<kF16>(stream, a) : launch_tiles<kBF16>(stream, a);
 }
 } // namespace wsp::ops
