@@ -199,6 +199,36 @@ __device__ __forceinline__ void exact_parts(float x, uint32_t (&bits)[3])
     }
 }
 
+// The LDS byte address of a shared-memory pointer.
+__device__ __forceinline__ uint32_t lds_address(const void* p)
+{
+    return (uint32_t) (uintptr_t) (__attribute__((address_space(3))) char*) (p);
+}
+
+// One direct-to-LDS load: this lane's 16 bytes at base + offset land at LDS
+// address lds + 16·lane (lds uniform over the wave).
+__device__ __forceinline__ void load_lds16(const void* base, uint32_t offset, uint32_t lds)
+{
+    asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds), "v"(offset), "s"(base)
+                 : "memory");
+}
+
+template <int N>
+__device__ __forceinline__ void wait_loads()
+{
+    static_assert(N >= 0 && N < 64, "vmcnt holds 0..63");
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
+}
+
+// Where the encoder attention's transposed values keep key `row`: inside each
+// 32 keys the eight that a lane group g of the score product's output holds
+// (4g .. 4g + 3 and 16 + 4g .. 16 + 4g + 3) lie together, so they are one
+// 16-byte operand read.
+__host__ __device__ constexpr int attention_place(int row)
+{
+    return (row & ~31) | ((row >> 2 & 3) << 3) | ((row >> 4 & 1) << 2) | (row & 3);
+}
+
 // x * 0.5 * (1 + erf(x / sqrt(2))), the exact form (Kernels/Gelu.h:16-21),
 // with the device library's erff.
 __device__ __forceinline__ float exact_gelu(float x)

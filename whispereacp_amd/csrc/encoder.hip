@@ -91,6 +91,7 @@ __global__ void __launch_bounds__(kColumnThreads) mel_columns_kernel(const float
 // ---------------------------------------------------------------------------
 constexpr int kFlashKeys = 64;
 constexpr int kFlashWidth = 64;
+constexpr int kFlashStages = 2; // 32 KB each
 typedef _Float16 f16x4 __attribute__((ext_vector_type(4)));
 typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
@@ -125,19 +126,20 @@ int compute_units()
     return units;
 }
 
+// K and V arrive cut into fp16 hi and lo (k_halves [2][pitch][width], vt_halves
+// transposed [2][width][pitch] with each 32 keys in attention_place order, pitch
+// a multiple of the key tile): the q/k/v product writes them, or halves_kernel.
+// Tiles go straight from there into LDS (direct-to-LDS loads, two stages, one
+// barrier a tile; chunk c of row r at slot 8r + (c ^ (r & 7)), so an operand
+// read's eight rows hit eight bank groups).
+//
 // Key splits: blockIdx.z takes keys [z·span, min((z + 1)·span, count)); with
 // one split the block writes the normalised rows to out (OUT = kF32) or as
 // the exact 16-bit parts of the output product's input (OUT = kF16, kBF16:
 // part p at out_parts + p·out_part_stride), with several it writes (max, sum,
 // row) partials [split][head][query][66] for flash_combine_kernel.
-// With PRESPLIT, K and V arrive already cut into fp16 hi and lo by the q/k/v
-// product (k_halves [2][pitch][width], vt_halves transposed [2][width][pitch],
-// pitch a multiple of the key tile and zero past count), so a tile's staging
-// is a copy; otherwise the fp32 k and v are cut here.
-template <int WAVES, bool PRESPLIT = false, int OUT = kF32>
-__global__ void __launch_bounds__(WAVES * 64) flash_attention_kernel(const float* __restrict__ q,
-                                                                    const float* __restrict__ k,
-                                                                    const float* __restrict__ v, int count,
+template <int WAVES, int OUT>
+__global__ void __launch_bounds__(WAVES * 64) flash_attention_kernel(const float* __restrict__ q, int count,
                                                                     int width, float scale2, float* __restrict__ out,
                                                                     int span, float* __restrict__ partials,
                                                                     const uint16_t* __restrict__ k_halves,
@@ -145,34 +147,55 @@ __global__ void __launch_bounds__(WAVES * 64) flash_attention_kernel(const float
                                                                     uint16_t* __restrict__ out_parts,
                                                                     size_t out_part_stride)
 {
-    constexpr int kThreadsHere = WAVES * 64;
-    constexpr int kUnits = kFlashKeys * kFlashWidth / 4; // float4 runs of a K (or V) tile
-    constexpr int kPerThread = (kUnits + kThreadsHere - 1) / kThreadsHere;
-    constexpr int kHalfChunks = 2 * kFlashKeys * kFlashWidth / 8; // 16-byte runs of a tile's K (or V) halves
-    constexpr int KB = kFlashKeys / 32;                           // 32-key blocks of a tile (P·V k-steps)
-    constexpr int kHalfPerThread = kHalfChunks / kThreadsHere;
-    static_assert(kHalfChunks % kThreadsHere == 0, "whole half runs per thread");
-    __shared__ __attribute__((aligned(16))) _Float16 ks[2][kFlashKeys][kFlashWidth + 8];
-    // V^T rows padded by four halves (a pitch of 34 words): the 8-byte operand
-    // reads of 16 lanes (rows li) then land on 16 distinct bank pairs; K's
-    // 16-byte reads of 8 lanes need a pitch of 4 words mod 32 (72 halves).
-    __shared__ __attribute__((aligned(16))) _Float16 vt[2][kFlashWidth][kFlashKeys + 4];
+    constexpr int KB = kFlashKeys / 32;            // 32-key blocks of a tile (P·V k-steps)
+    constexpr int kPartBytes = kFlashKeys * 128;   // one part of a tile of K, or of V^T
+    constexpr int kStageBytes = 4 * kPartBytes;    // K hi, K lo, V hi, V lo
+    constexpr int kPerWave = kStageBytes / 1024 / WAVES;
+    static_assert(kFlashKeys == 64 && kFlashWidth == 64, "rows of 64 halves, in both K and V^T");
+    __shared__ __attribute__((aligned(16))) unsigned char stages[kFlashStages][kStageBytes];
 
     const int head = blockIdx.y;
-    const int wave = threadIdx.x / 64, lane = threadIdx.x % 64, li = lane % 16, g = lane / 16;
+    const int lane = threadIdx.x % 64, li = lane % 16, g = lane / 16;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
     const int column = head * kFlashWidth;
     const int query = blockIdx.x * 16 * WAVES + 16 * wave + li;
     const bool query_in = query < count;
     const int k_begin = (int) blockIdx.z * span, k_end = min(count, k_begin + span);
+    const int tiles = max(0, k_end - k_begin + kFlashKeys - 1) / kFlashKeys;
+
+    // This wave's loads: load i moves eight rows (128 bytes each) of one part.
+    const void* src[kPerWave];
+    uint32_t offset[kPerWave], advance[kPerWave], dst[kPerWave];
+#pragma unroll
+    for (int t = 0; t < kPerWave; ++t)
+    {
+        const int i = wave + WAVES * t, part = i / 8 % 2, row = 8 * (i % 8) + lane / 8, chunk = (lane % 8) ^ (row & 7);
+        const bool is_key = i < 16;
+        src[t] = is_key ? k_halves : vt_halves;
+        offset[t] = 2 * (uint32_t) (part * (size_t) pitch * width
+                                    + (is_key ? (size_t) (k_begin + row) * width + column
+                                              : (size_t) (column + row) * pitch + k_begin)
+                                    + 8 * chunk);
+        advance[t] = is_key ? 2 * kFlashKeys * width : 2 * kFlashKeys;
+        dst[t] = 1024 * i;
+    }
+    const uint32_t stage0 = lds_address(stages);
+    // (a tile past the last reloads it, into a stage no one reads again)
+    auto issue = [&](int tile, int stage) {
+#pragma unroll
+        for (int t = 0; t < kPerWave; ++t)
+            load_lds16(src[t], offset[t] + (uint32_t) min(tile, tiles - 1) * advance[t],
+                       __builtin_amdgcn_readfirstlane(stage0 + stage * kStageBytes + dst[t]));
+    };
 
     // This lane's B fragments of Q^T: query `query`, dims 32 s + 8 g .. + 7.
     f16x8 qh[2], ql[2];
 #pragma unroll
     for (int s = 0; s < 2; ++s)
     {
-        const float* src = q + (size_t) min(query, count - 1) * width + column + 32 * s + 8 * g;
-        const f32x4 a = *reinterpret_cast<const f32x4*>(src);
-        const f32x4 b = *reinterpret_cast<const f32x4*>(src + 4);
+        const float* from = q + (size_t) min(query, count - 1) * width + column + 32 * s + 8 * g;
+        const f32x4 a = *reinterpret_cast<const f32x4*>(from);
+        const f32x4 b = *reinterpret_cast<const f32x4*>(from + 4);
 #pragma unroll
         for (int e = 0; e < 4; ++e)
         {
@@ -189,99 +212,23 @@ __global__ void __launch_bounds__(WAVES * 64) flash_attention_kernel(const float
     for (int t = 0; t < 4; ++t)
         o[t] = f32x4 {0.f, 0.f, 0.f, 0.f};
 
-    // K and V runs of a tile, loaded two tiles ahead of its use into one of
-    // two register stages (a tile past the end reloads the last keys, unused).
-    struct Stage
+    if (tiles > 0)
+#pragma unroll
+        for (int t = 0; t < kFlashStages - 1; ++t)
+            issue(t, t);
+    int stage = 0;
+    for (int tile = 0; tile < tiles; ++tile)
     {
-        f32x4 k[kPerThread], v[kPerThread];
-        u32x4 kh[kHalfPerThread], vh[kHalfPerThread];
-    };
-    // Run i of this thread in a tile of halves: part, then K row and 8-column
-    // block, or V^T row (channel) and 8-key block.
-    auto half_run = [&](int i, int& part, int& a, int& b, int& c, int& kb) {
-        const int unit = (int) threadIdx.x + i * kThreadsHere;
-        const int rest = unit % (kHalfChunks / 2);
-        part = unit / (kHalfChunks / 2);
-        a = rest / (kFlashWidth / 8);
-        b = rest % (kFlashWidth / 8);
-        c = rest / (kFlashKeys / 8);
-        kb = rest % (kFlashKeys / 8);
-    };
-    const int last_first = k_begin + (max(k_end - k_begin, 1) - 1) / kFlashKeys * kFlashKeys;
-    const size_t halves_part = (size_t) pitch * width;
-    auto load_tile = [&](Stage& st, int first) {
-        if constexpr (PRESPLIT)
-        {
-            const int f = min(first, last_first);
-#pragma unroll
-            for (int i = 0; i < kHalfPerThread; ++i)
-            {
-                int part, row, cb, c, kb;
-                half_run(i, part, row, cb, c, kb);
-                st.kh[i] = *reinterpret_cast<const u32x4*>(k_halves + part * halves_part + (size_t) (f + row) * width
-                                                           + column + 8 * cb);
-                st.vh[i] = *reinterpret_cast<const u32x4*>(vt_halves + part * halves_part
-                                                           + (size_t) (column + c) * pitch + f + 8 * kb);
-            }
-            return;
-        }
-#pragma unroll
-        for (int i = 0; i < kPerThread; ++i)
-        {
-            const int unit = (int) threadIdx.x + i * kThreadsHere;
-            const int key = first + (unit % kUnits) / 16, d4 = 4 * (unit % 16);
-            const size_t at = (size_t) min(key, k_end - 1) * width + column + d4;
-            st.k[i] = *reinterpret_cast<const f32x4*>(k + at);
-            st.v[i] = *reinterpret_cast<const f32x4*>(v + at);
-        }
-    };
-
-    // One tile: its stage into LDS (as fp16 parts), the stage refilled with
-    // the tile two ahead, then the scores, the online softmax and P·V.
-    auto tile = [&](int first, Stage& st) {
-        __syncthreads(); // the previous tile has been read
-        if constexpr (PRESPLIT)
-        {
-#pragma unroll
-            for (int i = 0; i < kHalfPerThread; ++i)
-            {
-                int part, row, cb, c, kb;
-                half_run(i, part, row, cb, c, kb);
-                *reinterpret_cast<u32x4*>(&ks[part][row][8 * cb]) = st.kh[i];
-                // (8-byte aligned rows: two 8-byte stores)
-                uint2* v2 = reinterpret_cast<uint2*>(&vt[part][c][8 * kb]);
-                v2[0] = uint2 {st.vh[i][0], st.vh[i][1]};
-                v2[1] = uint2 {st.vh[i][2], st.vh[i][3]};
-            }
-        }
-        else
-        {
-#pragma unroll
-            for (int i = 0; i < kPerThread; ++i)
-            {
-                const int unit = (int) threadIdx.x + i * kThreadsHere;
-                if (unit < kUnits)
-                {
-                    const int row = unit / 16, d4 = 4 * (unit % 16);
-                    const bool in = first + row < k_end;
-                    f16x4 kh, kl;
-#pragma unroll
-                    for (int e = 0; e < 4; ++e)
-                    {
-                        const float kv = in ? st.k[i][e] : 0.f, vv = in ? st.v[i][e] : 0.f;
-                        kh[e] = half_hi(kv);
-                        kl[e] = half_lo(kv);
-                        vt[0][d4 + e][row] = half_hi(vv);
-                        vt[1][d4 + e][row] = half_lo(vv);
-                    }
-                    *reinterpret_cast<f16x4*>(&ks[0][row][d4]) = kh;
-                    *reinterpret_cast<f16x4*>(&ks[1][row][d4]) = kl;
-                }
-            }
-        }
+        // This wave's loads of the tile are done once only the later stages'
+        // are in flight; the barrier makes every wave's visible and ends every
+        // read of the stage refilled next.
+        wait_loads<(kFlashStages - 2) * kPerWave>();
         __syncthreads();
-        if (k_begin < k_end)
-            load_tile(st, first + 2 * kFlashKeys);
+        issue(tile + kFlashStages - 1, stage == 0 ? kFlashStages - 1 : stage - 1);
+        const int first = k_begin + tile * kFlashKeys;
+        const f16x8* const ks = reinterpret_cast<const f16x8*>(stages[stage]);
+        const f16x8* const vs = ks + 2 * kPartBytes / 16;
+        auto at = [&](int row, int chunk) { return 8 * row + (chunk ^ (row & 7)); };
 
         // S^T for keys 16 mt + 4 g + r of the tile, query li.
         f32x4 st_[2 * KB];
@@ -292,9 +239,8 @@ __global__ void __launch_bounds__(WAVES * 64) flash_attention_kernel(const float
 #pragma unroll
             for (int s = 0; s < 2; ++s)
             {
-                const f16x8 kh = *reinterpret_cast<const f16x8*>(&ks[0][16 * mt + li][32 * s + 8 * g]);
-                const f16x8 kl = *reinterpret_cast<const f16x8*>(&ks[1][16 * mt + li][32 * s + 8 * g]);
-                st_[mt] = mfma3(kh, kl, qh[s], ql[s], st_[mt]);
+                const int from = at(16 * mt + li, 4 * s + g);
+                st_[mt] = mfma3(ks[from], ks[kPartBytes / 16 + from], qh[s], ql[s], st_[mt]);
             }
         }
         if (first + kFlashKeys > k_end) // the last tile: its keys past the end
@@ -348,33 +294,13 @@ __global__ void __launch_bounds__(WAVES * 64) flash_attention_kernel(const float
 #pragma unroll
             for (int b = 0; b < KB; ++b)
             {
-                const f16x4 a0 = *reinterpret_cast<const f16x4*>(&vt[0][16 * t + li][32 * b + 4 * g]);
-                const f16x4 a1 = *reinterpret_cast<const f16x4*>(&vt[0][16 * t + li][32 * b + 16 + 4 * g]);
-                const f16x4 b0 = *reinterpret_cast<const f16x4*>(&vt[1][16 * t + li][32 * b + 4 * g]);
-                const f16x4 b1 = *reinterpret_cast<const f16x4*>(&vt[1][16 * t + li][32 * b + 16 + 4 * g]);
-                const f16x8 vh = {a0[0], a0[1], a0[2], a0[3], a1[0], a1[1], a1[2], a1[3]};
-                const f16x8 vl = {b0[0], b0[1], b0[2], b0[3], b1[0], b1[1], b1[2], b1[3]};
-                o[t] = mfma3(vh, vl, ph[b], pl[b], o[t]);
+                const int from = at(16 * t + li, 4 * b + g);
+                o[t] = mfma3(vs[from], vs[kPartBytes / 16 + from], ph[b], pl[b], o[t]);
             }
         }
-    };
-
-    // Pairs of tiles, then an odd last one outside the loop, so the loop's
-    // back edge always follows the second tile of a pair.
-    Stage s0, s1;
-    if (k_begin < k_end)
-    {
-        load_tile(s0, k_begin);
-        load_tile(s1, k_begin + kFlashKeys);
+        stage = stage == kFlashStages - 1 ? 0 : stage + 1;
     }
-    int first = k_begin;
-    for (; first + kFlashKeys < k_end; first += 2 * kFlashKeys)
-    {
-        tile(first, s0);
-        tile(first + kFlashKeys, s1);
-    }
-    if (first < k_end)
-        tile(first, s0);
+    wait_loads<0>();
     // The row sum over the four lanes of query li, then O = O^T / l.
     l += __shfl_xor(l, 16);
     l += __shfl_xor(l, 32);
@@ -422,14 +348,40 @@ __global__ void __launch_bounds__(WAVES * 64) flash_attention_kernel(const float
     }
 }
 
+// fp32 k and v rows as the attention's halves, where their product does not
+// write them itself.
+__global__ void __launch_bounds__(kColumnThreads) halves_kernel(const float* __restrict__ k,
+                                                                const float* __restrict__ v, int width, int pitch,
+                                                                uint16_t* __restrict__ k_halves,
+                                                                uint16_t* __restrict__ vt_halves)
+{
+    const int row = blockIdx.x;
+    const size_t part = (size_t) pitch * width;
+    for (int c = threadIdx.x; c < width; c += kColumnThreads)
+    {
+        const float kv = k[(size_t) row * width + c], vv = v[(size_t) row * width + c];
+        const size_t at = (size_t) row * width + c, vat = (size_t) c * pitch + attention_place(row);
+        k_halves[at] = __builtin_bit_cast(uint16_t, half_hi(kv));
+        k_halves[part + at] = __builtin_bit_cast(uint16_t, half_lo(kv));
+        vt_halves[vat] = __builtin_bit_cast(uint16_t, half_hi(vv));
+        vt_halves[part + vat] = __builtin_bit_cast(uint16_t, half_lo(vv));
+    }
+}
+
 // The key splits of every (query, head) combined in split order, in base-2
 // units: out = Σ 2^(m_s - m)·row_s / Σ 2^(m_s - m)·l_s. One 64-lane wave per
-// (query, head), a lane per channel.
-__global__ void __launch_bounds__(kFlashWidth) flash_combine_kernel(const float* __restrict__ partials, int count,
-                                                                    int heads, int splits, int width,
-                                                                    float* __restrict__ out)
+// (query, head), a lane per channel, four waves a block; the rows go out in
+// fp32 or as the output product's parts, like the attention's.
+template <int OUT>
+__global__ void __launch_bounds__(4 * kFlashWidth) flash_combine_kernel(const float* __restrict__ partials, int count,
+                                                                        int heads, int splits, int width,
+                                                                        float* __restrict__ out,
+                                                                        uint16_t* __restrict__ out_parts,
+                                                                        size_t out_part_stride)
 {
-    const int query = blockIdx.x, head = blockIdx.y, c = threadIdx.x;
+    const int query = blockIdx.x * 4 + threadIdx.x / kFlashWidth, head = blockIdx.y, c = threadIdx.x % kFlashWidth;
+    if (query >= count)
+        return;
     const size_t stride = (size_t) heads * count * (kFlashWidth + 2);
     const float* base = partials + ((size_t) head * count + query) * (kFlashWidth + 2);
     float largest = -INFINITY;
@@ -445,7 +397,18 @@ __global__ void __launch_bounds__(kFlashWidth) flash_combine_kernel(const float*
         numerator += f * part[2 + c];
         denominator += f * part[1];
     }
-    out[(size_t) query * width + head * kFlashWidth + c] = numerator / denominator;
+    const size_t at = (size_t) query * width + head * kFlashWidth + c;
+    const float v = numerator / denominator;
+    if constexpr (OUT == kF32)
+        out[at] = v;
+    else
+    {
+        uint32_t bits[3];
+        exact_parts<OUT>(v, bits);
+#pragma unroll
+        for (int p = 0; p < (OUT == kF16 ? 2 : 3); ++p)
+            out_parts[p * out_part_stride + at] = (uint16_t) bits[p];
+    }
 }
 
 // Row p of the second convolution's columns over frame-major rows x
@@ -716,13 +679,35 @@ int wsp_encoder_encode(wsp_encoder* e, const wsp_encoder_tensors* T, const float
         p.wdtype = wt;
         return ops::split_product(st, p);
     };
+    // q, k and v of an fp32 layer side by side, k and v as the attention's halves.
+    auto fp32_projections = [&](const wsp_encoder_layer_tensors& L, bool as_halves) {
+        ops::SplitProduct p {};
+        p.parts = e->normed;
+        p.rows = positions;
+        p.inner = d;
+        p.count = 3;
+        p.columns = d;
+        p.matrix[0] = {L.q_w, L.q_b, e->q, 1.f};
+        p.matrix[1] = {L.k_w, nullptr, e->k, 1.f};
+        p.matrix[2] = {L.v_w, L.v_b, e->v, 1.f};
+        p.ldy = d;
+        p.wdtype = WSP_F32;
+        if (as_halves)
+        {
+            p.y1_halves = e->k_halves;
+            p.y2_halves_t = e->vt_halves;
+            p.halves_pitch = e->pitch;
+        }
+        return p;
+    };
     // (Products that do not run over stored parts may store them there themselves.)
     const size_t window_rows = (size_t) window_positions;
     const ops::Scratch scratch {e->ff_parts, ops::parts_bytes(window_rows * f)};
     for (int l = 0; l < s.layers; ++l)
     {
         const wsp_encoder_layer_tensors& L = T->layers[l];
-        bool att_parts = false; // the attention wrote its rows as the output product's parts
+        const bool flash = d / heads == kFlashWidth;
+        bool halves = false; // the projections left k and v as the attention's halves
         status = split ? ops::layernorm_parts(st, e->hidden, L.attention_norm_w, L.attention_norm_b, e->parts,
                                               part_stride, positions, d, eps, wt)
                        : ops::layernorm(st, e->hidden, L.attention_norm_w, L.attention_norm_b, e->normed, positions,
@@ -744,14 +729,21 @@ int wsp_encoder_encode(wsp_encoder* e, const wsp_encoder_tensors* T, const float
             p.matrix[2] = {L.v_w, L.v_b, e->v, unscale(L.v_scale)};
             p.ldy = d;
             p.wdtype = wt;
-            if (d / heads == kFlashWidth)
+            if (flash)
             {
                 // The attention takes k and v as fp16 halves.
                 p.y1_halves = e->k_halves;
                 p.y2_halves_t = e->vt_halves;
                 p.halves_pitch = e->pitch;
+                halves = true;
             }
             status = ops::split_product(st, p);
+        }
+        else if (const ops::SplitProduct three = fp32_projections(L, flash);
+                 wt == WSP_F32 && positions > 16 && ops::fp32_split_fits(three))
+        {
+            halves = flash;
+            status = ops::fp32_split(st, three);
         }
         else
         {
@@ -772,8 +764,15 @@ int wsp_encoder_encode(wsp_encoder* e, const wsp_encoder_tensors* T, const float
         }
         if (status != hipSuccess)
             return encoder_hip(e, status, "self-attention projections");
-        if (d / heads == kFlashWidth && d % 4 == 0)
+        if (flash)
         {
+            if (!halves)
+            {
+                hipLaunchKernelGGL(halves_kernel, dim3(positions), dim3(kColumnThreads), 0, st, e->k, e->v, d,
+                                   e->pitch, e->k_halves, e->vt_halves);
+                if ((status = hipGetLastError()) != hipSuccess)
+                    return encoder_hip(e, status, "self-attention keys and values");
+            }
             // 128 queries a block share each K/V tile when that still leaves
             // at most an eighth of the CUs idle (large-v3: 240 blocks,
             // 14.2 -> 13.4 ms a window); else 64 (tiny.en's 72 blocks of 128
@@ -791,45 +790,39 @@ int wsp_encoder_encode(wsp_encoder* e, const wsp_encoder_tensors* T, const float
             const int span = ((positions + splits - 1) / splits + kFlashKeys - 1) / kFlashKeys * kFlashKeys;
             float* partials = splits > 1 ? e->flash_partials : nullptr;
             const bool wide = 8 * wide_blocks >= 7 * compute_units();
-            // With the pre-split products, one split writes its rows straight
-            // as the output product's input parts.
-            att_parts = split && (wide || splits == 1);
             const dim3 grid = wide ? dim3((positions + 16 * kFlashWideWaves - 1) / (16 * kFlashWideWaves), heads)
                                    : dim3((positions + 16 * kFlashWaves - 1) / (16 * kFlashWaves), heads, splits);
             const int key_span = wide ? positions : span;
+            // With the pre-split products the rows (or their combination) go
+            // out as the output product's input parts.
             uint16_t* const out_parts = static_cast<uint16_t*>(e->parts);
             auto launch = [&](auto kernel, int waves) {
-                hipLaunchKernelGGL(kernel, grid, dim3(64 * waves), 0, st, e->q, e->k, e->v, positions, d, scale2,
-                                   e->att, key_span, wide ? nullptr : partials, e->k_halves, e->vt_halves, e->pitch,
-                                   out_parts, part_stride);
+                hipLaunchKernelGGL(kernel, grid, dim3(64 * waves), 0, st, e->q, positions, d, scale2, e->att, key_span,
+                                   wide ? nullptr : partials, e->k_halves, e->vt_halves, e->pitch, out_parts,
+                                   part_stride);
+            };
+            auto combine = [&](auto kernel) {
+                hipLaunchKernelGGL(kernel, dim3((positions + 3) / 4, heads), dim3(4 * kFlashWidth), 0, st,
+                                   e->flash_partials, positions, heads, splits, d, e->att, out_parts, part_stride);
+            };
+            auto attend = [&](auto wide_kernel, auto narrow_kernel, auto combine_kernel) {
+                if (wide)
+                    launch(wide_kernel, kFlashWideWaves);
+                else
+                    launch(narrow_kernel, kFlashWaves);
+                if (!wide && splits > 1)
+                    combine(combine_kernel);
             };
             if (!split)
-            {
-                if (wide)
-                    launch(flash_attention_kernel<kFlashWideWaves>, kFlashWideWaves);
-                else
-                    launch(flash_attention_kernel<kFlashWaves>, kFlashWaves);
-            }
-            else if (!att_parts)
-                launch(flash_attention_kernel<kFlashWaves, true>, kFlashWaves);
+                attend(flash_attention_kernel<kFlashWideWaves, wsp::kF32>, flash_attention_kernel<kFlashWaves, wsp::kF32>,
+                       flash_combine_kernel<wsp::kF32>);
             else if (wt == WSP_F16)
-            {
-                if (wide)
-                    launch(flash_attention_kernel<kFlashWideWaves, true, wsp::kF16>, kFlashWideWaves);
-                else
-                    launch(flash_attention_kernel<kFlashWaves, true, wsp::kF16>, kFlashWaves);
-            }
-            else if (wide)
-                launch(flash_attention_kernel<kFlashWideWaves, true, wsp::kBF16>, kFlashWideWaves);
+                attend(flash_attention_kernel<kFlashWideWaves, wsp::kF16>, flash_attention_kernel<kFlashWaves, wsp::kF16>,
+                       flash_combine_kernel<wsp::kF16>);
             else
-                launch(flash_attention_kernel<kFlashWaves, true, wsp::kBF16>, kFlashWaves);
+                attend(flash_attention_kernel<kFlashWideWaves, wsp::kBF16>,
+                       flash_attention_kernel<kFlashWaves, wsp::kBF16>, flash_combine_kernel<wsp::kBF16>);
             status = hipGetLastError();
-            if (status == hipSuccess && splits > 1)
-            {
-                hipLaunchKernelGGL(flash_combine_kernel, dim3(positions, heads), dim3(kFlashWidth), 0, st,
-                                   e->flash_partials, positions, heads, splits, d, e->att);
-                status = hipGetLastError();
-            }
         }
         else
             status = ops::attention(st, e->q, positions, e->k, e->v, positions, d, heads, 0, scale, e->att,
@@ -838,7 +831,7 @@ int wsp_encoder_encode(wsp_encoder* e, const wsp_encoder_tensors* T, const float
             return encoder_hip(e, status, "self attention");
         if (split)
         {
-            if (att_parts || (status = ops::split_rows(st, e->att, part_stride, wt, e->parts, part_stride))
+            if (flash || (status = ops::split_rows(st, e->att, part_stride, wt, e->parts, part_stride))
                                  == hipSuccess)
                 status = split_product(e->parts, part_stride, d, L.out_w, L.out_b, e->hidden, d,
                                        ops::kProductResidual, nullptr, L.out_scale);

@@ -53,8 +53,8 @@ struct SplitProduct
     // Matrix 1 (y1_halves) and matrix 2 (y2_halves_t), when set, go out as fp16
     // hi = fp16(v) and lo = fp16(v - hi) instead of fp32: hi of row r, column c
     // at y1_halves[r·columns + c], lo halves_pitch·columns further; y2_halves_t
-    // transposed, hi at [c·halves_pitch + r]. (The encoder's keys and values
-    // for its attention.)
+    // transposed, hi at [c·halves_pitch + attention_place(r)]. (The encoder's
+    // keys and values for its attention; fp32 products need columns in quads.)
     void* y1_halves;
     void* y2_halves_t;
     int halves_pitch;

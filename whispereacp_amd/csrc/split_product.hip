@@ -46,7 +46,6 @@ namespace
 typedef uint16_t u16;
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
-typedef __attribute__((address_space(3))) char lds_char;
 
 constexpr int kRowBytes = 128;              // of a tile row per step: 64 16-bit values or 32 fp32
 constexpr int kChunks = kRowBytes / 16;
@@ -186,27 +185,6 @@ __global__ void __launch_bounds__(kNormRowsPerBlock * kWave) layernorm_parts_ker
             *reinterpret_cast<uint2*>(parts + p * part_stride + (size_t) row * width + 4 * r)
                 = uint2 {bits[0][p] | (bits[1][p] << 16), bits[2][p] | (bits[3][p] << 16)};
     }
-}
-
-// The LDS byte address of a shared-memory pointer.
-__device__ __forceinline__ uint32_t lds_address(const void* p)
-{
-    return (uint32_t) (uintptr_t) (lds_char*) (p);
-}
-
-// One direct-to-LDS load: this lane's 16 bytes at base + offset land at LDS
-// address lds + 16·lane (lds uniform over the wave).
-__device__ __forceinline__ void load_lds16(const void* base, uint32_t offset, uint32_t lds)
-{
-    asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds), "v"(offset), "s"(base)
-                 : "memory");
-}
-
-template <int N>
-__device__ __forceinline__ void wait_loads()
-{
-    static_assert(N >= 0 && N < 64, "vmcnt holds 0..63");
-    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
 }
 
 // Slot of chunk c of tile row r (16-byte slots).
@@ -392,7 +370,7 @@ __global__ void __launch_bounds__(T::kWaves * kWave) split_product_kernel(SplitP
                     *reinterpret_cast<uint2*>(o + p * a.out_part_stride)
                         = uint2 {bits[0][p] | (bits[1][p] << 16), bits[2][p] | (bits[3][p] << 16)};
             }
-            else if (WT != kF32 && ((seg == 1 && a.y1_halves != nullptr) || (seg == 2 && a.y2_halves_t != nullptr)))
+            else if ((seg == 1 && a.y1_halves != nullptr) || (seg == 2 && a.y2_halves_t != nullptr))
             {
                 uint32_t hi[4], lo[4];
 #pragma unroll
@@ -411,7 +389,7 @@ __global__ void __launch_bounds__(T::kWaves * kWave) split_product_kernel(SplitP
                 }
                 else
                 {
-                    u16* o = static_cast<u16*>(a.y2_halves_t) + (size_t) c * a.halves_pitch + row;
+                    u16* o = static_cast<u16*>(a.y2_halves_t) + (size_t) c * a.halves_pitch + attention_place(row);
 #pragma unroll
                     for (int r = 0; r < 4; ++r)
                     {
