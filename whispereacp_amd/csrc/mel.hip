@@ -49,19 +49,27 @@ __global__ void __launch_bounds__(kThreads) frames_kernel(const float* __restric
 }
 
 // Sixteen frames a block, from samples to log10 of the bands, in LDS: the
-// windowed samples folded about the frame's middle (cos(2πbn/N) is even and
-// sin odd in n, so re needs x[n] + x[N-n] and im x[n] - x[N-n] for n up to N/2
-// only: half the products), the two half-length products on the matrix cores
-// (v_mfma_f32_16x16x4_f32: 16 bins by 16 frames), the power, the filterbank as
-// another such product, the logarithm and the block's largest value. A wave
-// takes 16-bin tiles, then 16-band tiles. Each product step sums four
+// windowed samples folded, the half- or quarter-length transforms on the
+// matrix cores (v_mfma_f32_16x16x4_f32: 16 bins by 16 frames), the power, the
+// filterbank as another such product, the logarithm and the block's largest
+// value.
+//
+// Folding: cos(2πbn/N) is even about n = N/2 and sin odd, so re needs
+// e[n] = x[n] + x[N-n] and im o[n] = x[n] - x[N-n] for n up to H = N/2 only.
+// With N a multiple of four both fold once more about H/2, differently for
+// even and odd bins: even ones take e[n] + e[H-n] and o[n] - o[H-n], odd ones
+// e[n] - e[H-n] and o[n] + o[H-n] (at H/2 itself the cosine of an odd bin and
+// the sine of an even one are zero). That leaves a quarter of the products of
+// the whole transform and of the basis to read (200 KB a block at 400 points).
+//
+// A wave takes tiles of 16 bins of one parity, then tiles of 16 bands; the
+// filterbank is copied to LDS meanwhile. Each product step sums four
 // consecutive n (and bins), in order: position 16j + 4g + e of an LDS row, and
 // of the basis, holds n = 16j + 4e + g. The basis is fragment-major, one
-// contiguous kilobyte a load; each block reads all of it (346 KB at 400
-// points), which with the 10.8 K matrix-core clocks of a CU's tiles is what
-// bounds the launch. The 30 s window went from 38.8 us as seven launches
-// (frames, spectrum 17, power, filterbank copy and product, log) and 53 with
-// the products on the vector units to 23.5.
+// contiguous kilobyte a load. The 30 s window: 53 us as seven launches with the
+// products on the vector units, 38.8 with them on the matrix cores, 23.9 in
+// this launch folded once with the filters read from memory, 17.3 now; two
+// launches that do nothing but move the data take about 9.
 constexpr int kSpectrogramThreads = 512;
 constexpr int kSpectrogramFrames = 16;
 constexpr int kRuns = 4;   // 16-value runs a wave loads at a time
@@ -75,6 +83,32 @@ __host__ __device__ constexpr int place(int n)
     return n / 16 * 16 + 4 * (n % 4) + n % 16 / 4;
 }
 
+// How a transform of `fft` points folds, and the tiles that leaves.
+struct Folds
+{
+    int parities; // 2: even and odd bins apart
+    int values;   // n of a folded row
+    int tiles;    // 16-value runs of a folded row, and 16-bin tiles of a parity
+    int bin_tiles; // 16-bin runs of a power row
+
+    __host__ __device__ explicit Folds(int fft)
+    {
+        const int half = fft / 2;
+        parities = fft % 4 == 0 ? 2 : 1;
+        values = parities == 2 ? half / 2 + 1 : half + 1;
+        tiles = (values + 15) / 16;
+        bin_tiles = (half + 16) / 16;
+    }
+    __host__ __device__ int folded_stride() const { return 16 * tiles + kRowPad; }
+    __host__ __device__ int power_stride() const { return 16 * bin_tiles + kRowPad; }
+    // Floats of the folded rows ([parity][cosine, sine][frame]) and the power rows.
+    __host__ __device__ int lds_floats() const
+    {
+        return kSpectrogramFrames * (2 * parities * folded_stride() + power_stride());
+    }
+};
+
+template <bool STAGED>
 __global__ void __launch_bounds__(kSpectrogramThreads) spectrogram_kernel(
     const float* __restrict__ samples, int count, const float* __restrict__ window, int fft, int hop, int frames,
     const float* __restrict__ basis, const float* __restrict__ filters, int mels, float* __restrict__ out,
@@ -82,49 +116,82 @@ __global__ void __launch_bounds__(kSpectrogramThreads) spectrogram_kernel(
 {
     extern __shared__ __attribute__((aligned(16))) float rows[];
     __shared__ float scratch[kSpectrogramThreads / kWave];
-    const int half = fft / 2, bins = half + 1, tiles = (bins + 15) / 16, stride = 16 * tiles + kRowPad;
-    float* const even = rows;                             // [frame][place(n)]
-    float* const odd = even + kSpectrogramFrames * stride;
-    float* const power = odd + kSpectrogramFrames * stride; // [frame][place(bin)]
+    const Folds folds(fft);
+    const int half = fft / 2, bins = half + 1, tiles = folds.tiles;
+    const int stride = folds.folded_stride(), power_stride = folds.power_stride();
+    float* const power = rows + 2 * folds.parities * kSpectrogramFrames * stride; // [frame][place(bin)]
+    float* const staged = rows + folds.lds_floats();                             // the filterbank as it is
     const int f0 = blockIdx.x * kSpectrogramFrames;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave), lane = threadIdx.x % kWave;
+    const int li = lane % 16, g = lane / 16;
 
-    // A thread folds value n of eight frames (all their loads in flight at
-    // once); values past the middle are the padding.
-    constexpr int kValues = 256, kFramesEach = kSpectrogramFrames * kValues / kSpectrogramThreads;
+    if constexpr (STAGED)
+    {
+        // In flight until the bands' tiles; the last few values by hand.
+        const int total = mels * bins, whole = total / 4 * 4;
+        const uint32_t base = lds_address(staged);
+        for (int i = 256 * wave; i < whole; i += 256 * (kSpectrogramThreads / kWave))
+            if (i + 4 * lane < whole)
+                load_lds16(filters, 4 * (i + 4 * lane), __builtin_amdgcn_readfirstlane(base + 4 * i));
+        if ((int) threadIdx.x < total - whole)
+            staged[whole + threadIdx.x] = filters[whole + threadIdx.x];
+    }
+
+    // A thread folds value n of four frames (all their loads in flight at
+    // once); values past the last are the padding.
+    constexpr int kValues = 128, kFramesEach = kSpectrogramFrames * kValues / kSpectrogramThreads;
     const int first = threadIdx.x / kValues * kFramesEach;
     for (int n = threadIdx.x % kValues; n < 16 * tiles; n += kValues)
     {
-        const bool in = n <= half, folded = in && n > 0 && 2 * n != fft;
-        const int t = in ? n : 0, u = folded ? fft - n : t;
-        const float wt = window[t], wu = window[u];
-        float a[kFramesEach], b[kFramesEach];
+        const bool in = n < folds.values, twice = folds.parities == 2;
+        // x[n], x[N-n] and, folding twice, x[H-n], x[H+n]; without a partner the value itself
+        const bool pair = in && n > 0 && 2 * n != fft;
+        const int t[4] = {in ? n : 0, pair ? fft - n : in ? n : 0, in && twice ? half - n : 0,
+                          pair && twice ? half + n : 0};
+        float w[4], x[kFramesEach][4];
+#pragma unroll
+        for (int k = 0; k < 4; ++k)
+            w[k] = window[t[k]];
+#pragma unroll
+        for (int i = 0; i < kFramesEach; ++i)
+#pragma unroll
+            for (int k = 0; k < 4; ++k)
+            {
+                const int at = abs(min(f0 + first + i, frames - 1) * hop - half + t[k]);
+                x[i][k] = samples[at >= count ? 2 * (count - 1) - at : at];
+            }
 #pragma unroll
         for (int i = 0; i < kFramesEach; ++i)
         {
-            const int start = min(f0 + first + i, frames - 1) * hop - half;
-            int x = abs(start + t), y = abs(start + u);
-            x = x >= count ? 2 * (count - 1) - x : x;
-            y = y >= count ? 2 * (count - 1) - y : y;
-            a[i] = samples[x];
-            b[i] = samples[y];
-        }
-#pragma unroll
-        for (int i = 0; i < kFramesEach; ++i)
-        {
-            const float left = a[i] * wt, right = b[i] * wu;
-            const int at = (first + i) * stride + place(n);
-            even[at] = folded ? left + right : in ? left : 0.f;
-            odd[at] = folded ? left - right : 0.f;
+            const float a = x[i][0] * w[0], b = x[i][1] * w[1], c = x[i][2] * w[2], d = x[i][3] * w[3];
+            const float en = !in ? 0.f : pair ? a + b : a, on = pair ? a - b : 0.f;
+            float* const row = rows + (first + i) * stride + place(n);
+            constexpr int kNext = kSpectrogramFrames; // rows between one folded row and the next kind
+            if (!twice)
+            {
+                row[0] = en;
+                row[kNext * stride] = on;
+                continue;
+            }
+            const bool middle = 2 * n == half;
+            const float em = !in ? 0.f : pair ? c + d : c, om = pair ? c - d : 0.f;
+            row[0] = middle ? en : en + em;
+            row[kNext * stride] = middle ? 0.f : on - om;
+            row[2 * kNext * stride] = middle ? 0.f : en - em;
+            row[3 * kNext * stride] = middle ? on : on + om;
         }
     }
     __syncthreads();
 
-    const int wave = threadIdx.x / kWave, lane = threadIdx.x % kWave, li = lane % 16, g = lane / 16;
     // Runs of the basis (and of the filters) are loaded kRuns ahead of their
     // products; runs past the last repeat it and are not multiplied.
-    for (int t = wave; t < tiles; t += kSpectrogramThreads / kWave)
+    for (int unit = wave; unit < folds.parities * tiles; unit += kSpectrogramThreads / kWave)
     {
-        const f32x4* b = reinterpret_cast<const f32x4*>(basis) + (size_t) t * tiles * 2 * kWave + lane;
+        const int parity = unit % folds.parities, t = unit / folds.parities;
+        const f32x4* from = reinterpret_cast<const f32x4*>(basis) + (size_t) (parity * tiles + t) * tiles * 2 * kWave
+                            + lane;
+        const float* even = rows + 2 * parity * kSpectrogramFrames * stride + li * stride + 4 * g;
+        const float* odd = even + kSpectrogramFrames * stride;
         f32x4 re = {0.f, 0.f, 0.f, 0.f}, im = {0.f, 0.f, 0.f, 0.f};
         f32x4 c[2][kRuns], s[2][kRuns];
         auto load = [&](int j0, int set) {
@@ -132,8 +199,8 @@ __global__ void __launch_bounds__(kSpectrogramThreads) spectrogram_kernel(
             for (int i = 0; i < kRuns; ++i)
             {
                 const int j = min(j0 + i, tiles - 1);
-                c[set][i] = b[(size_t) (2 * j) * kWave];
-                s[set][i] = b[(size_t) (2 * j + 1) * kWave];
+                c[set][i] = from[(size_t) (2 * j) * kWave];
+                s[set][i] = from[(size_t) (2 * j + 1) * kWave];
             }
         };
         auto multiply = [&](int j0, int set) {
@@ -142,8 +209,8 @@ __global__ void __launch_bounds__(kSpectrogramThreads) spectrogram_kernel(
             {
                 if (j0 + i >= tiles)
                     break;
-                const f32x4 e = *reinterpret_cast<const f32x4*>(even + li * stride + 16 * (j0 + i) + 4 * g);
-                const f32x4 o = *reinterpret_cast<const f32x4*>(odd + li * stride + 16 * (j0 + i) + 4 * g);
+                const f32x4 e = *reinterpret_cast<const f32x4*>(even + 16 * (j0 + i));
+                const f32x4 o = *reinterpret_cast<const f32x4*>(odd + 16 * (j0 + i));
 #pragma unroll
                 for (int k = 0; k < 4; ++k)
                 {
@@ -160,18 +227,24 @@ __global__ void __launch_bounds__(kSpectrogramThreads) spectrogram_kernel(
             load(j0 + 2 * kRuns, 0);
             multiply(j0 + kRuns, 1);
         }
-        // Lane (li, g) holds frame li's bins 16t + 4g + r.
+        // Lane (li, g) holds frame li's bins 16t + 4g + r of this parity.
 #pragma unroll
         for (int r = 0; r < 4; ++r)
-            power[li * stride + place(16 * t + 4 * g + r)] = re[r] * re[r] + im[r] * im[r];
+        {
+            const int bin = folds.parities * (16 * t + 4 * g + r) + parity;
+            if (bin < 16 * folds.bin_tiles)
+                power[li * power_stride + place(bin)] = re[r] * re[r] + im[r] * im[r];
+        }
     }
+    if constexpr (STAGED)
+        wait_loads<0>();
     __syncthreads();
 
     float best = -INFINITY;
     const int bands = (mels + 15) / 16;
     for (int t = wave; t < bands; t += kSpectrogramThreads / kWave)
     {
-        const float* row = filters + (size_t) min(16 * t + li, mels - 1) * bins;
+        const int from = min(16 * t + li, mels - 1) * bins;
         f32x4 sum = {0.f, 0.f, 0.f, 0.f};
         float w[2][kRuns][4];
         auto load = [&](int j0, int set) {
@@ -179,15 +252,18 @@ __global__ void __launch_bounds__(kSpectrogramThreads) spectrogram_kernel(
             for (int i = 0; i < kRuns; ++i)
 #pragma unroll
                 for (int k = 0; k < 4; ++k)
-                    w[set][i][k] = row[min(16 * (j0 + i) + 4 * k + g, bins - 1)];
+                {
+                    const int at = from + min(16 * (j0 + i) + 4 * k + g, bins - 1);
+                    w[set][i][k] = STAGED ? staged[at] : filters[at];
+                }
         };
         auto multiply = [&](int j0, int set) {
 #pragma unroll
             for (int i = 0; i < kRuns; ++i)
             {
-                if (j0 + i >= tiles)
+                if (j0 + i >= folds.bin_tiles)
                     break;
-                const f32x4 p = *reinterpret_cast<const f32x4*>(power + li * stride + 16 * (j0 + i) + 4 * g);
+                const f32x4 p = *reinterpret_cast<const f32x4*>(power + li * power_stride + 16 * (j0 + i) + 4 * g);
 #pragma unroll
                 for (int k = 0; k < 4; ++k)
                 {
@@ -197,7 +273,7 @@ __global__ void __launch_bounds__(kSpectrogramThreads) spectrogram_kernel(
             }
         };
         load(0, 0);
-        for (int j0 = 0; j0 < tiles; j0 += 2 * kRuns)
+        for (int j0 = 0; j0 < folds.bin_tiles; j0 += 2 * kRuns)
         {
             load(j0 + kRuns, 1);
             multiply(j0, 0);
@@ -221,9 +297,11 @@ __global__ void __launch_bounds__(kSpectrogramThreads) spectrogram_kernel(
         peaks[blockIdx.x] = best;
 }
 
+constexpr size_t kSpectrogramLds = 156 * 1024; // of a CU's 160 KB
+
 size_t spectrogram_lds(int fft)
 {
-    return (size_t) 3 * kSpectrogramFrames * (16 * ((fft / 2 + 16) / 16) + kRowPad) * sizeof(float);
+    return (size_t) Folds(fft).lds_floats() * sizeof(float);
 }
 
 // power rows have a stride of `padded` (bins rounded up to a multiple of 4,
@@ -349,16 +427,19 @@ int wsp_mel_create(const wsp_mel_shape* shape, int device, void* stream, wsp_mel
         status = mel_allocate(m, &m->peaks, std::max(wsp::mel::kLogBlocks, (s.frame_count + 15) / 16));
     if (status == hipSuccess)
         status = hipMemcpy(m->window, window.data(), window.size() * sizeof(float), hipMemcpyHostToDevice);
-    m->fused = wsp::mel::spectrogram_lds(fft) <= 152 * 1024; // of a CU's 160 KB
+    m->fused = wsp::mel::spectrogram_lds(fft) <= wsp::mel::kSpectrogramLds;
     if (m->fused)
     {
-        const int tiles = (bins + 15) / 16;
-        basis.assign((size_t) tiles * tiles * 2 * 256, 0.f);
+        const wsp::mel::Folds folds(fft);
+        const int tiles = folds.tiles;
+        basis.assign((size_t) folds.parities * tiles * tiles * 2 * 256, 0.f);
         for (int b = 0; b < bins; ++b)
-            for (int n = 0; n < bins; ++n)
+            for (int n = 0; n < folds.values; ++n)
             {
                 // lane (bin % 16, g), element e of run n / 16 stands for n = 16j + 4e + g
-                const size_t at = (((size_t) (b / 16) * tiles + n / 16) * 2 * 64 + 16 * (n % 4) + b % 16) * 4 + n % 16 / 4;
+                const int parity = b % folds.parities, i = b / folds.parities;
+                const size_t run = ((size_t) parity * tiles + i / 16) * tiles + n / 16;
+                const size_t at = (run * 2 * 64 + 16 * (n % 4) + i % 16) * 4 + n % 16 / 4;
                 basis[at] = (float) std::cos(angle(b, n));
                 basis[at + 256] = (float) -std::sin(angle(b, n));
             }
@@ -367,9 +448,11 @@ int wsp_mel_create(const wsp_mel_shape* shape, int device, void* stream, wsp_mel
         if (status == hipSuccess)
             status = hipMemcpy(m->folded, basis.data(), basis.size() * sizeof(float), hipMemcpyHostToDevice);
         if (status == hipSuccess)
-            status = hipFuncSetAttribute(reinterpret_cast<const void*>(&wsp::mel::spectrogram_kernel),
-                                         hipFuncAttributeMaxDynamicSharedMemorySize,
-                                         (int) wsp::mel::spectrogram_lds(fft));
+            status = hipFuncSetAttribute(reinterpret_cast<const void*>(&wsp::mel::spectrogram_kernel<true>),
+                                         hipFuncAttributeMaxDynamicSharedMemorySize, (int) wsp::mel::kSpectrogramLds);
+        if (status == hipSuccess)
+            status = hipFuncSetAttribute(reinterpret_cast<const void*>(&wsp::mel::spectrogram_kernel<false>),
+                                         hipFuncAttributeMaxDynamicSharedMemorySize, (int) wsp::mel::kSpectrogramLds);
     }
     else
     {
@@ -447,9 +530,17 @@ int wsp_mel_encode(wsp_mel* m, const float* samples, const float* filters, float
     if (m->fused)
     {
         const int blocks = (frames + kSpectrogramFrames - 1) / kSpectrogramFrames;
-        hipLaunchKernelGGL(spectrogram_kernel, dim3(blocks), dim3(kSpectrogramThreads), spectrogram_lds(fft), st,
-                           samples, s.sample_count, m->window, fft, s.hop_length, frames, m->folded, filters, mels,
-                           output, m->peaks);
+        // The filterbank goes through LDS where it fits and comes in whole 16-byte runs.
+        const size_t lds = spectrogram_lds(fft), with_filters = lds + ((size_t) mels * bins + 3) / 4 * 16;
+        const bool staged = with_filters <= kSpectrogramLds && reinterpret_cast<uintptr_t>(filters) % 16 == 0;
+        if (staged)
+            hipLaunchKernelGGL(spectrogram_kernel<true>, dim3(blocks), dim3(kSpectrogramThreads), with_filters, st,
+                               samples, s.sample_count, m->window, fft, s.hop_length, frames, m->folded, filters, mels,
+                               output, m->peaks);
+        else
+            hipLaunchKernelGGL(spectrogram_kernel<false>, dim3(blocks), dim3(kSpectrogramThreads), lds, st, samples,
+                               s.sample_count, m->window, fft, s.hop_length, frames, m->folded, filters, mels, output,
+                               m->peaks);
         if ((status = hipGetLastError()) != hipSuccess)
             return mel_hip(m, status, "spectrogram");
         hipLaunchKernelGGL(normalise_kernel, dim3(std::min(kLogBlocks, (total + kThreads - 1) / kThreads)),
