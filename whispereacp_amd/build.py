@@ -35,7 +35,7 @@ HOST_FLAGS = ["-O2", "-D__HIP_PLATFORM_AMD__", "-I" + os.path.join(ROCM, "includ
 # VGPRs (in AGPRs the compiler shuffles them between steps).
 SOURCE_FLAGS = {source: ["-mllvm", "-amdgpu-mfma-vgpr-form=1"] for source in (
     "split_product.hip", "linear_product.hip", "mel.hip", "ops.hip",
-    "encoder.hip")}
+    "encoder.hip", "batch.hip")}
 
 
 def hipcc() -> str:
