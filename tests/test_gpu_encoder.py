@@ -108,12 +108,13 @@ def test_whisper_width_encoder_matches_oracle(oracle, dtype, frames, scaled):
 
 @pytest.mark.parametrize("dtype,width,frames,scaled", [
     ("F16", 384, 2998, True), ("BF16", 384, 2998, False), ("F16", 384, 66, True), ("BF16", 384, 130, False),
-    ("F16", 768, 2050, True)])
+    ("F16", 768, 2050, True), ("F32", 384, 2999, True)])
 def test_product_tiles_match_oracle(oracle, dtype, width, frames, scaled):
     # The pre-split products choose their tile by the blocks it gives: 1499
     # rows at width 384 take 64 x 128 tiles with two and four stages and
     # 32 x 128, 33 and 65 rows take 32 x 64, 1025 rows at width 768 add
-    # 128 x 256 (fc1) — every one with a last row tile part-filled. Bar: 2^-22
+    # 128 x 256 (fc1) — every one with a last row tile part-filled; 2999 frames
+    # leave the second convolution's last tap outside. Bar: 2^-22
     # of each operand times sums of at most 3072 fp32 terms, as fp32 rounding
     # grows over them (measured up to 3e-6).
     shape = S.EncoderShape(16, width, width // 64, 1, 4 * width, frames)

@@ -433,7 +433,7 @@ struct wsp_encoder
     int device = 0;
     hipStream_t stream = nullptr;
     float* columns = nullptr; // both convolutions' gathered rows
-    float* conv = nullptr;    // [conv frames, width] frame-major
+    float* conv = nullptr;    // [conv frames, width] frame-major, or the second convolution's gathered rows
     float* hidden = nullptr;  // [positions, width]
     float* normed = nullptr;
     float* q = nullptr;
@@ -523,7 +523,7 @@ int wsp_encoder_create(const wsp_encoder_shape* shape, int device, void* stream,
     if (status == hipSuccess)
         status = encoder_allocate(e, &e->columns, std::max(frames * s.mel_bins * 3, positions * d * 3));
     if (status == hipSuccess)
-        status = encoder_allocate(e, &e->conv, frames * d);
+        status = encoder_allocate(e, &e->conv, std::max(frames, 3 * positions) * d);
     float** rows[] = {&e->hidden, &e->normed, &e->q, &e->k, &e->v, &e->att};
     for (float** r : rows)
         if (status == hipSuccess)
@@ -639,21 +639,54 @@ int wsp_encoder_encode(wsp_encoder* e, const wsp_encoder_tensors* T, const float
                        s.input_frames, frames, e->columns);
     if ((status = hipGetLastError()) != hipSuccess)
         return encoder_hip(e, status, "conv1 columns");
-    if ((status = ops::linear(st, e->columns, conv_frames, 3 * s.mel_bins, T->conv1_w, WSP_F32, T->conv1_b, e->conv,
-                              d, 1)) != hipSuccess)
-        return encoder_hip(e, status, "conv1");
-    hipLaunchKernelGGL(frame_columns_kernel, dim3(positions), dim3(kColumnThreads), 0, st, e->conv, d, conv_frames,
-                       e->columns);
-    if ((status = hipGetLastError()) != hipSuccess)
-        return encoder_hip(e, status, "conv2 columns");
-    // h = gelu(conv2) + embed_positions: the rows start as the positional
-    // table's first rows and the product adds to them (bias, GELU, residual).
-    if ((status = hipMemcpyAsync(e->hidden, T->positions, (size_t) positions * d * sizeof(float),
-                                 hipMemcpyDeviceToDevice, st)) != hipSuccess)
-        return encoder_hip(e, status, "positional rows");
-    if ((status = ops::linear(st, e->columns, positions, 3 * d, T->conv2_w, WSP_F32, T->conv2_b, e->hidden, d, 3))
-        != hipSuccess)
-        return encoder_hip(e, status, "conv2");
+    // Both convolutions as direct-to-LDS fp32 products where they fit and give
+    // each CU a tile: the first writes the second's columns itself, and the
+    // second adds to the positional table's rows.
+    auto convolution = [&](const float* x, int rows, int inner, const float* w, const float* bias, float* y, int flags) {
+        ops::SplitProduct p {};
+        p.parts = x;
+        p.rows = rows;
+        p.inner = inner;
+        p.count = 1;
+        p.columns = d;
+        p.matrix[0] = {w, bias, y, 1.f};
+        p.ldy = d;
+        p.flags = flags;
+        p.wdtype = WSP_F32;
+        return p;
+    };
+    auto tiles = [&](int rows) { return (rows + 31) / 32 * ((d + 31) / 32); };
+    ops::SplitProduct conv1 = convolution(e->columns, conv_frames, 3 * s.mel_bins, T->conv1_w, T->conv1_b, e->conv,
+                                          ops::kProductGelu | ops::kProductTaps);
+    conv1.taps = positions;
+    ops::SplitProduct conv2 = convolution(e->conv, positions, 3 * d, T->conv2_w, T->conv2_b, e->hidden,
+                                          ops::kProductGelu | ops::kProductResidual);
+    conv2.residual = T->positions;
+    if (tiles(positions) >= compute_units() && ops::fp32_split_fits(conv1) && ops::fp32_split_fits(conv2))
+    {
+        if ((status = ops::fp32_split(st, conv1)) != hipSuccess)
+            return encoder_hip(e, status, "conv1");
+        if ((status = ops::fp32_split(st, conv2)) != hipSuccess)
+            return encoder_hip(e, status, "conv2");
+    }
+    else
+    {
+        if ((status = ops::linear(st, e->columns, conv_frames, 3 * s.mel_bins, T->conv1_w, WSP_F32, T->conv1_b,
+                                  e->conv, d, 1)) != hipSuccess)
+            return encoder_hip(e, status, "conv1");
+        hipLaunchKernelGGL(frame_columns_kernel, dim3(positions), dim3(kColumnThreads), 0, st, e->conv, d, conv_frames,
+                           e->columns);
+        if ((status = hipGetLastError()) != hipSuccess)
+            return encoder_hip(e, status, "conv2 columns");
+        // h = gelu(conv2) + embed_positions: the rows start as the positional
+        // table's first rows and the product adds to them (bias, GELU, residual).
+        if ((status = hipMemcpyAsync(e->hidden, T->positions, (size_t) positions * d * sizeof(float),
+                                     hipMemcpyDeviceToDevice, st)) != hipSuccess)
+            return encoder_hip(e, status, "positional rows");
+        if ((status = ops::linear(st, e->columns, positions, 3 * d, T->conv2_w, WSP_F32, T->conv2_b, e->hidden, d, 3))
+            != hipSuccess)
+            return encoder_hip(e, status, "conv2");
+    }
 
     const int wt = T->wdtype;
     auto unscale = [](float c) { return c == 0.f ? 1.f : 1.f / c; };

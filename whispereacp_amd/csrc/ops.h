@@ -36,6 +36,10 @@ constexpr int kMaxMatrices = 64;
 // only, rows of `columns` values, part p at out_parts + p·out_part_stride).
 constexpr int kProductGelu = 1;
 constexpr int kProductResidual = 2;
+// fp32 products, one matrix: row f is frame f of a convolution and goes out as
+// the columns of the next, stride two: of output row p's three taps (channel·3 +
+// tap, rows of 3·columns) tap t is frame 2p + t - 1, zero outside the frames.
+constexpr int kProductTaps = 4;
 struct SplitProduct
 {
     const void* parts;
@@ -47,6 +51,8 @@ struct SplitProduct
     int rows_per_group;
     size_t group_stride;
     int flags;
+    const float* residual; // kProductResidual: what is added to, laid out as y (null: y)
+    int taps;              // kProductTaps: the next convolution's rows
     void* out_parts;
     size_t out_part_stride;
     int wdtype;

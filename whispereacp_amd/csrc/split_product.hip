@@ -332,7 +332,8 @@ __global__ void __launch_bounds__(T::kWaves * kWave) split_product_kernel(SplitP
     const float scale = matrix.scale;
     // Four columns a lane go out as one store; fp32 products may end inside them.
     const bool quads = width % 4 == 0 && a.ldy % 4 == 0 && a.group_stride % 4 == 0
-                       && reinterpret_cast<uintptr_t>(y) % 16 == 0;
+                       && reinterpret_cast<uintptr_t>(y) % 16 == 0
+                       && reinterpret_cast<uintptr_t>(a.residual) % 16 == 0;
 #pragma unroll
     for (int nt = 0; nt < NT; ++nt)
     {
@@ -398,6 +399,28 @@ __global__ void __launch_bounds__(T::kWaves * kWave) split_product_kernel(SplitP
                     }
                 }
             }
+            else if (WT == kF32 && (a.flags & kProductTaps))
+            {
+                const int p = row / 2;
+#pragma unroll
+                for (int r = 0; r < 4; ++r)
+                    if (c + r < width)
+                    {
+                        float* o = y + ((size_t) p * width + c + r) * 3;
+                        if (row % 2 != 0)
+                        {
+                            o[2] = v[r];
+                            if (p + 1 < a.taps)
+                                o[3 * (size_t) width] = v[r];
+                            continue;
+                        }
+                        o[1] = v[r];
+                        if (row == 0)
+                            o[0] = 0.f;
+                        if (row == a.rows - 1)
+                            o[2] = 0.f;
+                    }
+            }
             else if (const size_t at = (size_t) (row / a.rows_per_group) * a.group_stride
                                        + (size_t) (row % a.rows_per_group) * a.ldy + c;
                      quads)
@@ -405,7 +428,7 @@ __global__ void __launch_bounds__(T::kWaves * kWave) split_product_kernel(SplitP
                 float4v* o = reinterpret_cast<float4v*>(y + at);
                 float4v sum = {v[0], v[1], v[2], v[3]};
                 if (a.flags & kProductResidual)
-                    sum = *o + sum;
+                    sum = (a.residual != nullptr ? *reinterpret_cast<const float4v*>(a.residual + at) : *o) + sum;
                 *o = sum;
             }
             else
@@ -414,7 +437,8 @@ __global__ void __launch_bounds__(T::kWaves * kWave) split_product_kernel(SplitP
                     if (c + r < width)
                     {
                         float* o = y + at + r;
-                        *o = a.flags & kProductResidual ? *o + v[r] : v[r];
+                        const float from = a.residual != nullptr ? a.residual[at + r] : *o;
+                        *o = a.flags & kProductResidual ? from + v[r] : v[r];
                     }
         }
     }
