@@ -84,8 +84,10 @@ void* wsp_hip_stream(const wsp_hip_ctx* ctx);
 /* y[r, o] = act(Σ_k x[r,k]·W[o,k] + b[o]) (+ y[r,o] when RESIDUAL).
  * x [rows, inner] f32, W [out, inner] row-major in `wdtype`, bias [out] f32 or
  * null (zero, which replaces the zero-bias buffers at
- * Net/KernelNet.cpp:440-458), y [rows, out] f32. Rows up to 16 take the split
- * GEMV, more take the tiled product. Replaces KernelNet::dispatchProjection
+ * Net/KernelNet.cpp:440-458), y [rows, out] f32. Up to four rows take the split
+ * GEMV (as do 5 to 16 whose inner extent or addresses are not whole vectors),
+ * more the matrix cores: in exact 16-bit parts of x for more than 16 rows of
+ * 16-bit weights with inner % 32 == 0 and out % 128 == 0, else in fp32. Replaces KernelNet::dispatchProjection
  * (Net/KernelNet.cpp:817-859) over SplitLinear / HalfWeightSplitLinear
  * (Kernels/Linear.h:129-276) and LinearProduct (Kernels/SimdTiledMatMul.h:470-486). */
 int wsp_hip_linear(wsp_hip_ctx* ctx, const float* x, int rows, int inner, const void* weight,
@@ -124,7 +126,7 @@ int wsp_hip_embed(wsp_hip_ctx* ctx, const uint32_t* tokens, int count, const flo
  * width / heads columns. scale multiplies the summed dot product. One query
  * takes the split-key form (Kernels/SingleQueryAttention.h:505-556); several
  * take the causal multi-query form with the mask semantics of
- * Kernels/Attention.h:34-47. Replaces KernelNet::runCachedAttention
+ * Kernels/Attention.h:34-47, on the matrix cores for heads of 64 channels. Replaces KernelNet::runCachedAttention
  * (Net/KernelNet.cpp:951-1013). Head width must be a multiple of 4, at most 64
  * (the reference's own limit, Kernels/SingleQueryAttention.cpp:32-45). */
 int wsp_hip_attention(wsp_hip_ctx* ctx, const float* q, int q_count, const float* keys,

@@ -8,14 +8,14 @@
 //   per layer: h += out_proj(attention(LN(h)));  h += fc2(gelu(fc1(LN(h))))
 //   rows = LN(h)
 //
-// Both convolutions are products: a column kernel gathers, for every output
-// frame, the three taps of every input channel into one row (index
-// channel * 3 + tap, the order of a [out, in, 3] weight row), with zero past
-// the frames the run was given (Encoder/Encoder.h:46-56), and the product
-// adds the bias, applies GELU and — for conv2 — adds the positional rows the
-// output buffer was filled with. The projections, LayerNorms and attention
-// are the library's per-op kernels; their 16-bit-weight products run on the
-// matrix cores over 1500-row operands.
+// Both convolutions are products over rows that hold, for every output frame,
+// the three taps of every input channel (index channel * 3 + tap, the order of
+// a [out, in, 3] weight row), with zero past the frames the run was given
+// (Encoder/Encoder.h:46-56). A column kernel gathers the first's from the mel;
+// the first's product writes the second's itself, and the second's adds the
+// positional table. The projections are split_product's or the library's
+// products, the attention flash_attention_kernel for heads of 64 channels and
+// the library's otherwise.
 #include "../../include/wsp_hip.h"
 #include "device_common.h"
 #include "ops.h"

@@ -7,8 +7,9 @@
 
 namespace wsp::ops
 {
-// Rows up to this count take the split GEMV; more take the tiled product
-// (the reference's splitRowLimit, Net/KernelNet.h:144-149).
+// Up to this many rows the products stay in fp32 arithmetic, and those that
+// the matrix cores cannot load in whole vectors take the split GEMV (the
+// reference's splitRowLimit, Net/KernelNet.h:144-149).
 constexpr int kSplitRowLimit = 16;
 constexpr int kMaxHeadWidth = 64;
 constexpr int kAttentionChunkKeys = 1024; // longest key chunk one workgroup scores

@@ -1,5 +1,5 @@
-// Per-op gfx950 kernels behind the C ABI: the split GEMV and tiled product
-// (Kernels/Linear.h), LayerNorm (Kernels/LayerNorm.h), Embed
+// Per-op gfx950 kernels behind the C ABI: the split GEMV (Kernels/Linear.h;
+// linear_product.hip has the products of more rows), LayerNorm (Kernels/LayerNorm.h), Embed
 // (Kernels/Embed.h), split-key attention with its combine
 // (Kernels/SingleQueryAttention.h, Kernels/Attention.h) and the two-stage
 // argmax (Kernels/Argmax.h). Written for wave64 CDNA4; every reduction runs in

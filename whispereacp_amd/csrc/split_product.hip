@@ -1,8 +1,10 @@
-// The encoder's products on gfx950 matrix cores with pre-split activations:
-// y = X·Wᵀ for fp32 X of 1500 rows and a 16-bit W (Encoder/Encoder.cpp:82-174:
-// the q/k/v, attention-output, fc1 and fc2 products of every layer).
+// Products of many rows on gfx950 matrix cores: y = X·Wᵀ for fp32 X and a 16-bit
+// W with X in pre-split parts, or an fp32 W in fp32 arithmetic
+// (Encoder/Encoder.cpp:82-174: the q/k/v, attention-output, fc1 and fc2
+// products of every layer and the convolutions; the cross keys and values of
+// every layer, and long prompts, through linear_product.hip).
 //
-// X is stored once in exact 16-bit parts (three bf16 parts for bf16 weights,
+// For 16-bit W, X is stored once in exact 16-bit parts (three bf16 parts for bf16 weights,
 // fp16 hi + lo for fp16 weights, |x| < 65504), part-major: part p of row r at
 // parts + p·part_stride + r·inner. Every matrix-core product of a part with W
 // is exact, and the fp32 sums match an fp32 product with widened weights to
