@@ -163,6 +163,23 @@ def test_layernorm_widths(ctx, oracle, width):
     assert worst_error(y.cpu().numpy(), oracle.layernorm(x.astype(np.float64), w, b)) < 1e-4
 
 
+# The widths on either side of each register form (a wave holds 512, 1280 or
+# 2048 floats), rows that are not whole 16-byte runs, and terms at an odd float.
+# A lane's 32 terms and six rounds over the lanes: sums within 38 * 2^-24 =
+# 2.3e-6 of themselves, which moves values of up to five times the deviation
+# about a mean of three by less than 1e-5 together with the roundings behind.
+@pytest.mark.parametrize("width", [4, 252, 260, 512, 516, 1280, 1284, 2048, 2052, 770])
+def test_layernorm_forms(ctx, oracle, width):
+    rows = 5
+    x = (S.normal_values(rows * width, width, 1.0).reshape(rows, width) + 3.0).astype(np.float32)
+    w, b = S.spread_values(width + 1, 5, 1.5), S.spread_values(width + 1, 6, 0.75)
+    expected = oracle.layernorm(x.astype(np.float64), w[1:].copy(), b[1:].copy())
+    y = dev(np.zeros_like(x))
+    ctx.layernorm(dev(x), dev(w)[1:], dev(b)[1:], y, rows, width)
+    sync()
+    assert worst_error(y.cpu().numpy(), expected) < 1e-5
+
+
 def test_layernorm_constant_row_yields_bias(ctx):
     w = S.spread_values(32, 33, 2.0)
     b = S.spread_values(32, 44, 2.0)

@@ -149,6 +149,26 @@ __global__ void __launch_bounds__(kBlock) layernorm_kernel(const float* __restri
         dst[c] = (row[c] - mean) * scale * gamma[c] + beta[c];
 }
 
+// A wave for each row of up to 256·RUNS floats in whole 16-byte runs
+// (normalise_row); other rows take layernorm_kernel.
+template <int RUNS>
+__global__ void __launch_bounds__(kWave) layernorm_row_kernel(const float* __restrict__ x,
+                                                              const float* __restrict__ gamma,
+                                                              const float* __restrict__ beta, float* __restrict__ y,
+                                                              int width, float eps)
+{
+    const size_t row = (size_t) blockIdx.x * width;
+    float4v v[RUNS];
+    normalise_row<RUNS>(x + row, gamma, beta, width, eps, v);
+#pragma unroll
+    for (int i = 0; i < RUNS; ++i)
+    {
+        const int at = 4 * ((int) threadIdx.x + kWave * i);
+        if (at < width)
+            *reinterpret_cast<float4v*>(y + row + at) = v[i];
+    }
+}
+
 // ---------------------------------------------------------------------------
 // Embed: out[t, c] = tokens table row + position table row (Kernels/Embed.h).
 // ---------------------------------------------------------------------------
@@ -868,7 +888,18 @@ hipError_t linear(hipStream_t stream, const float* x, int rows, int inner, const
 hipError_t layernorm(hipStream_t stream, const float* x, const float* gamma, const float* beta,
                      float* y, int rows, int width, float eps)
 {
-    hipLaunchKernelGGL(layernorm_kernel, dim3(rows), dim3(kBlock), 0, stream, x, gamma, beta, y, width, eps);
+    auto whole = [](const void* p) { return reinterpret_cast<uintptr_t>(p) % 16 == 0; };
+    if (width % 4 != 0 || width > 2048 || !whole(x) || !whole(y))
+    {
+        hipLaunchKernelGGL(layernorm_kernel, dim3(rows), dim3(kBlock), 0, stream, x, gamma, beta, y, width, eps);
+        return hipGetLastError();
+    }
+    auto run = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, dim3(rows), dim3(kWave), 0, stream, x, gamma, beta, y, width, eps);
+    };
+    width <= 512    ? run(layernorm_row_kernel<2>)
+    : width <= 1280 ? run(layernorm_row_kernel<5>)
+                    : run(layernorm_row_kernel<8>);
     return hipGetLastError();
 }
 

@@ -132,59 +132,33 @@ __global__ void __launch_bounds__(kSplitThreads) split_rows_kernel(const float* 
         *reinterpret_cast<u32x4*>(parts + p * part_stride + i) = out[p];
 }
 
-// LayerNorm of one row per wave (ops::layernorm's arithmetic: the mean, the
-// centred squares' mean, then (x - mean)·rstd·gamma + beta), written as the
-// parts of split_product's input. A lane holds float4 runs lane, lane + 64,
-// ... of the row in registers (at most kNormRuns of them), so the row is read
-// once; each part's four values of a run go out as one 8-byte store.
-constexpr int kNormRowsPerBlock = 4;
-constexpr int kNormRuns = 8; // widths up to 2048
+// normalise_row written as the parts of split_product's input, each part's four
+// values of a run as one 8-byte store.
+constexpr int kNormWidth = 2048; // the widest
 
-template <int WT>
-__global__ void __launch_bounds__(kNormRowsPerBlock * kWave) layernorm_parts_kernel(
-    const float* __restrict__ x, const float* __restrict__ gamma, const float* __restrict__ beta, int rows,
-    int width, float eps, u16* __restrict__ parts, size_t part_stride)
+template <int WT, int RUNS>
+__global__ void __launch_bounds__(kWave) layernorm_parts_kernel(const float* __restrict__ x,
+                                                                const float* __restrict__ gamma,
+                                                                const float* __restrict__ beta, int width, float eps,
+                                                                u16* __restrict__ parts, size_t part_stride)
 {
     constexpr int P = parts_of<WT>();
-    const int row = blockIdx.x * kNormRowsPerBlock + (int) threadIdx.x / kWave, lane = threadIdx.x % kWave;
-    if (row >= rows)
-        return;
-    const int runs = width / 4;
-    const float* src = x + (size_t) row * width;
-    float4v v[kNormRuns];
-    float total = 0.f;
+    const size_t row = (size_t) blockIdx.x * width;
+    float4v v[RUNS];
+    normalise_row<RUNS>(x + row, gamma, beta, width, eps, v);
 #pragma unroll
-    for (int i = 0; i < kNormRuns; ++i)
+    for (int i = 0; i < RUNS; ++i)
     {
-        const int r = lane + kWave * i;
-        v[i] = r < runs ? *reinterpret_cast<const float4v*>(src + 4 * r) : float4v {0.f, 0.f, 0.f, 0.f};
-        total += (v[i][0] + v[i][1]) + (v[i][2] + v[i][3]);
-    }
-    const float mean = wave_sum(total) / (float) width;
-    float squares = 0.f;
-#pragma unroll
-    for (int i = 0; i < kNormRuns; ++i)
-        if (lane + kWave * i < runs)
-#pragma unroll
-            for (int e = 0; e < 4; ++e)
-            {
-                const float c = v[i][e] - mean;
-                squares += c * c;
-            }
-    const float scale = rsqrtf(wave_sum(squares) / (float) width + eps);
-#pragma unroll
-    for (int i = 0; i < kNormRuns; ++i)
-    {
-        const int r = lane + kWave * i;
-        if (r >= runs)
+        const int at = 4 * ((int) threadIdx.x + kWave * i);
+        if (at >= width)
             continue;
         uint32_t bits[4][3];
 #pragma unroll
         for (int e = 0; e < 4; ++e)
-            split<WT>((v[i][e] - mean) * scale * gamma[4 * r + e] + beta[4 * r + e], bits[e]);
+            split<WT>(v[i][e], bits[e]);
 #pragma unroll
         for (int p = 0; p < P; ++p)
-            *reinterpret_cast<uint2*>(parts + p * part_stride + (size_t) row * width + 4 * r)
+            *reinterpret_cast<uint2*>(parts + p * part_stride + row + at)
                 = uint2 {bits[0][p] | (bits[1][p] << 16), bits[2][p] | (bits[3][p] << 16)};
     }
 }
@@ -518,7 +492,7 @@ hipError_t split_rows(hipStream_t stream, const float* x, size_t count, int wdty
 
 bool layernorm_parts_fits(int width)
 {
-    return width > 0 && width % 4 == 0 && width <= 4 * kWave * kNormRuns;
+    return width > 0 && width % 4 == 0 && width <= kNormWidth;
 }
 
 hipError_t layernorm_parts(hipStream_t stream, const float* x, const float* gamma, const float* beta, void* parts,
@@ -526,13 +500,18 @@ hipError_t layernorm_parts(hipStream_t stream, const float* x, const float* gamm
 {
     if (!layernorm_parts_fits(width) || (wdtype != kF16 && wdtype != kBF16))
         return hipErrorInvalidValue;
-    const dim3 grid((rows + kNormRowsPerBlock - 1) / kNormRowsPerBlock);
+    auto run = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, dim3(rows), dim3(kWave), 0, stream, x, gamma, beta, width, eps,
+                           static_cast<u16*>(parts), part_stride);
+    };
     if (wdtype == kF16)
-        hipLaunchKernelGGL(layernorm_parts_kernel<kF16>, grid, dim3(kNormRowsPerBlock * kWave), 0, stream, x, gamma,
-                           beta, rows, width, eps, static_cast<u16*>(parts), part_stride);
+        width <= 512    ? run(layernorm_parts_kernel<kF16, 2>)
+        : width <= 1280 ? run(layernorm_parts_kernel<kF16, 5>)
+                        : run(layernorm_parts_kernel<kF16, 8>);
     else
-        hipLaunchKernelGGL(layernorm_parts_kernel<kBF16>, grid, dim3(kNormRowsPerBlock * kWave), 0, stream, x,
-                           gamma, beta, rows, width, eps, static_cast<u16*>(parts), part_stride);
+        width <= 512    ? run(layernorm_parts_kernel<kBF16, 2>)
+        : width <= 1280 ? run(layernorm_parts_kernel<kBF16, 5>)
+                        : run(layernorm_parts_kernel<kBF16, 8>);
     return hipGetLastError();
 }
 
