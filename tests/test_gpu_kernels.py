@@ -101,6 +101,27 @@ def test_linear_paths(ctx, dtype, rows, inner, out):
         assert np.all(got[:, column] == np.inf)
 
 
+@pytest.mark.parametrize("dtype", ["F16", "BF16"])
+@pytest.mark.parametrize("rows,inner,out", [(1100, 4096, 256), (2101, 4096, 128), (300, 16384, 512)])
+def test_linear_beyond_the_scratch(dtype, rows, inner, out):
+    # A context whose scratch (16 MB at least) does not hold the rows' parts:
+    # two or more slabs of rows, and rows too long even for those. The bound
+    # is test_linear_matches_oracle's.
+    from whispereacp_amd.decoder import KernelContext, stored_to_device
+    small = KernelContext(S.DecoderShape(64, 1, 1, 64, 64, 8, 8))
+    x = S.normal_values(rows * inner, 19, 1.0).reshape(rows, inner)
+    stored, w = weights(out, inner, dtype, 23)
+    bias = S.normal_values(out, 29, 0.1)
+    start = S.normal_values(rows * out, 17, 1.0).reshape(rows, out)
+    wdev, wdtype = stored_to_device(S.StoredTensor("w", dtype, (out, inner), stored))
+    y = dev(start.copy())
+    small.linear(dev(x), rows, inner, wdev, wdtype, dev(bias), y, out, 2)
+    sync()
+    expected = x.astype(np.float64) @ w.astype(np.float64).T + bias + start
+    assert worst_error(y.cpu().numpy(), expected) <= 1e-5 + 2.4e-7 * inner
+    small.close()
+
+
 @pytest.mark.parametrize("dtype", ["F32", "F16", "BF16"])
 @pytest.mark.parametrize("rows,inner,out,count", [(3, 64, 128, 3), (17, 64, 128, 70), (300, 128, 256, 5),
                                                   (300, 96, 64, 4), (40, 40, 24, 4)])

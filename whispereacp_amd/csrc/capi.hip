@@ -83,9 +83,11 @@ int wsp_hip_ctx_create(const wsp_decoder_shape* shape, int device, void* stream,
         ctx->attention_floats = std::max<size_t>(floats, 1);
         ctx->argmax_candidates =
             (size_t) shape->max_positions * wsp::ops::argmax_groups(shape->vocabulary_size);
-        ctx->parts_bytes = wsp::ops::parts_bytes(
-            std::max((size_t) shape->cross_positions * shape->width,
-                     (size_t) shape->max_positions * std::max(shape->width, shape->feed_forward_width)));
+        // Every product over a window's rows in one piece (46 MB at large-v3);
+        // longer ones go in slabs, of no less than 16 MB (546 rows of 5120 as
+        // three parts).
+        ctx->parts_bytes = std::max<size_t>(
+            16 << 20, wsp::ops::parts_bytes((size_t) longest * std::max(shape->width, shape->feed_forward_width)));
         // One block: the attention workspace, the argmax candidates, the parts.
         auto rounded = [](size_t bytes) { return (bytes + 255) / 256 * 256; };
         const size_t attention = rounded(std::max(ctx->attention_floats, wsp::ops::kQueryAttentionFloats)

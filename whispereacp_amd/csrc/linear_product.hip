@@ -521,23 +521,51 @@ SplitProduct split_product_of(const Products& p, const void* parts, size_t part_
     return a;
 }
 
+// Rows of X whose parts the scratch holds at a time: all of them, else equal
+// slabs in whole 32-row tiles; 0 where those would be of fewer than
+// kLeastSlab rows, or where the output's rows lie in groups.
+constexpr int kLeastSlab = 256;
+int slab_rows(const Products& p, const Scratch& scratch)
+{
+    const size_t row_bytes = (size_t) p.inner * 2 * (p.wdtype == kF16 ? 2 : 3);
+    const size_t held = std::min(scratch.bytes / row_bytes, ((size_t) (1u << 29) - 1) / p.inner); // (32-bit byte offsets)
+    if ((size_t) p.rows <= held)
+        return p.rows;
+    const int whole = (int) (held / 32 * 32);
+    if (whole < kLeastSlab || p.rows > p.rows_per_group)
+        return 0;
+    const int slabs = (p.rows + whole - 1) / whole;
+    return ((p.rows + slabs - 1) / slabs + 31) / 32 * 32;
+}
+
 // 16-bit weights with X in 16-bit parts. From 2^17 outputs on (every matrix
-// together) X is stored as parts once and every matrix goes through
-// split_product in launches of up to 64; fewer, and what the scratch does not
-// hold, through row_product_kernel: 96 x 768 -> 768 runs 5.3 us there, 96 x 3072
-// -> 768 13; 200 x 5120 -> 1280 39, against 20 with the parts' launch.
+// together) X is stored as parts, every matrix going through split_product in
+// launches of up to 64; fewer, and what the scratch does not hold, through
+// row_product_kernel: 96 x 768 -> 768 runs 5.3 us there, 96 x 3072 -> 768 13;
+// 200 x 5120 -> 1280 39, against 20 with the parts' launch.
 template <int WT>
 hipError_t parts_product(hipStream_t stream, const Products& p, const Scratch& scratch)
 {
     const long long outputs = (long long) p.rows * p.columns * p.count;
-    const size_t values = (size_t) p.rows * p.inner;
     hipError_t e = hipSuccess;
-    if (outputs > 1 << 17 && split_product_fits(p.wdtype, p.inner, p.columns) && parts_bytes(values) <= scratch.bytes
-        && values < 1u << 29 && (size_t) p.columns * p.inner < 1u << 30) // (32-bit byte offsets)
+    const int slab = slab_rows(p, scratch);
+    if (outputs > 1 << 17 && slab > 0 && split_product_fits(p.wdtype, p.inner, p.columns)
+        && (size_t) p.columns * p.inner < 1u << 30) // (32-bit byte offsets)
     {
-        e = split_rows(stream, p.x, values, p.wdtype, scratch.data, values);
-        for (int i = 0; i < p.count && e == hipSuccess; i += kMaxMatrices)
-            e = split_product(stream, split_product_of(p, scratch.data, values, i, std::min(kMaxMatrices, p.count - i)));
+        for (int first = 0; first < p.rows && e == hipSuccess; first += slab)
+        {
+            const int rows = std::min(slab, p.rows - first);
+            const size_t values = (size_t) rows * p.inner;
+            e = split_rows(stream, p.x + (size_t) first * p.inner, values, p.wdtype, scratch.data, values);
+            for (int i = 0; i < p.count && e == hipSuccess; i += kMaxMatrices)
+            {
+                SplitProduct a = split_product_of(p, scratch.data, values, i, std::min(kMaxMatrices, p.count - i));
+                a.rows = rows;
+                for (int m = 0; m < a.count; ++m)
+                    a.matrix[m].y += (size_t) first * p.ldy;
+                e = split_product(stream, a);
+            }
+        }
         return e;
     }
     for (int i = 0; i < p.count && e == hipSuccess; i += kMatrices)
