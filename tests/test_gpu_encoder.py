@@ -71,6 +71,33 @@ def test_reduced_context_matches_the_shorter_shape(oracle):
     assert worst_error(gpu_rows(shape, encoder_file, mel), oracle_rows(oracle, shape, encoder_file, mel)) <= 5e-6
 
 
+@pytest.mark.parametrize("dtype,width,scaled", [("F32", 128, True), ("F16", 128, True), ("BF16", 128, False),
+                                                ("BF16", 128, True), ("F16", 64, True), ("F32", 64, True)])
+@pytest.mark.parametrize("positions", [1, 37, 64, 95])
+def test_a_window_leaves_nothing_for_a_shorter_one(dtype, width, scaled, positions):
+    # One encoder, a whole window of NaN or of infinities, then a shorter clean
+    # one: the same bits as an encoder that ran nothing before. Widths 128 and
+    # 64: keys and values written by the projections (16-bit and fp32) and
+    # converted behind them.
+    from whispereacp_amd.encoder import Encoder, EncoderWeights
+    shape = S.EncoderShape(80, width, width // 64, 2, 4 * width, 200)
+    weights = EncoderWeights(shape, S.workload_encoder_file(shape, dtype, 3000), scaled)
+    mel = torch.from_numpy(np.ascontiguousarray(S.normal_mel(shape, 3500), dtype=np.float32)).cuda()
+
+    def rows(encoder, mel, positions):
+        out = torch.zeros((shape.positions(), shape.width), dtype=torch.float32, device="cuda")
+        encoder.encode(mel, weights, out, positions)
+        torch.cuda.synchronize()
+        return out[:positions].cpu()
+
+    expected = rows(Encoder(shape), mel, positions)
+    assert torch.isfinite(expected).all()
+    used = Encoder(shape)
+    for poison in (float("nan"), float("inf")):
+        assert not torch.isfinite(rows(used, torch.full_like(mel, poison), shape.positions())).any()
+        assert torch.equal(rows(used, mel, positions), expected)
+
+
 def test_too_long_a_context_is_a_model_error():
     from whispereacp_amd.decoder import ModelError
     shape = S.small_encoder_shape()

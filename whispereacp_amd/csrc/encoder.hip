@@ -47,11 +47,36 @@ int conv_length(int length, int stride)
 // Row t of the first convolution's columns: mel[s][t + tap - 1] at
 // s * 3 + tap. The mel is band-major with `stride` frames a band, of which
 // the run reads the first `frames`.
+//
+// The first `clearing` blocks set the attention's values to zero from the run's
+// `positions` to the end of their key tile: it reads them with weight zero,
+// which hides what an earlier, longer run left there only while it is finite. A
+// thread takes four keys of a channel, which attention_place keeps together.
+// (A launch of their own would cost an encode a few microseconds; stale keys
+// need no clearing, their scores are masked.)
+constexpr int kClearedQuads = 16; // of a 64-key tile
+
 __global__ void __launch_bounds__(kColumnThreads) mel_columns_kernel(const float* __restrict__ mel, int bins,
                                                                      int stride, int frames,
-                                                                     float* __restrict__ columns)
+                                                                     float* __restrict__ columns, int clearing,
+                                                                     int positions, int width, int pitch,
+                                                                     uint16_t* __restrict__ vt_halves)
 {
-    const int t = blockIdx.x;
+    const int t = (int) blockIdx.x - clearing;
+    if (t < 0)
+    {
+        const int i = blockIdx.x * kColumnThreads + threadIdx.x, row = i / kClearedQuads; // [part][channel]
+        const int key = (positions - 1) / (4 * kClearedQuads) * (4 * kClearedQuads) + 4 * (i % kClearedQuads);
+        if (row >= 2 * width || key + 4 <= positions)
+            return;
+        uint16_t* const at = vt_halves + (size_t) row * pitch + attention_place(key);
+        if (key >= positions)
+            *reinterpret_cast<uint2*>(at) = uint2 {0, 0};
+        else
+            for (int e = positions - key; e < 4; ++e)
+                at[e] = 0;
+        return;
+    }
     const int inner = bins * 3;
     for (int i = threadIdx.x; i < inner; i += kColumnThreads)
     {
@@ -447,7 +472,9 @@ struct wsp_encoder
     void* ff_parts = nullptr;
     // The attention's keys and values as fp16 hi and lo halves, written by the
     // q/k/v product: [2][pitch][width] and transposed [2][width][pitch], pitch
-    // the positions rounded up to the key tile, zero past the positions.
+    // the positions rounded up to the key tile. Past a run's positions the keys
+    // are whatever earlier runs left; the values of its last tile are zero
+    // (mel_columns_kernel).
     uint16_t* k_halves = nullptr;
     uint16_t* vt_halves = nullptr;
     int pitch = 0;
@@ -635,8 +662,11 @@ int wsp_encoder_encode(wsp_encoder* e, const wsp_encoder_tensors* T, const float
         return encoder_fail(e, WSP_ERR_SHAPE,
                             "wsp_encoder_encode: scaled projections need 16-bit storage and the pre-split products' "
                             "shapes");
-    hipLaunchKernelGGL(mel_columns_kernel, dim3(conv_frames), dim3(kColumnThreads), 0, st, mel, s.mel_bins,
-                       s.input_frames, frames, e->columns);
+    const bool flash = d / heads == kFlashWidth;
+    static_assert(kFlashKeys == 4 * kClearedQuads, "the key tile's values are cleared");
+    const int clearing = flash ? (2 * d * kClearedQuads + kColumnThreads - 1) / kColumnThreads : 0;
+    hipLaunchKernelGGL(mel_columns_kernel, dim3(clearing + conv_frames), dim3(kColumnThreads), 0, st, mel, s.mel_bins,
+                       s.input_frames, frames, e->columns, clearing, positions, d, e->pitch, e->vt_halves);
     if ((status = hipGetLastError()) != hipSuccess)
         return encoder_hip(e, status, "conv1 columns");
     // Both convolutions as direct-to-LDS fp32 products where they fit and give
@@ -739,7 +769,6 @@ int wsp_encoder_encode(wsp_encoder* e, const wsp_encoder_tensors* T, const float
     for (int l = 0; l < s.layers; ++l)
     {
         const wsp_encoder_layer_tensors& L = T->layers[l];
-        const bool flash = d / heads == kFlashWidth;
         bool halves = false; // the projections left k and v as the attention's halves
         status = split ? ops::layernorm_parts(st, e->hidden, L.attention_norm_w, L.attention_norm_b, e->parts,
                                               part_stride, positions, d, eps, wt)
