@@ -324,6 +324,27 @@ def test_attention_hidden_values_may_be_non_finite(ctx, q_count, k_count):
         assert not np.any(np.isfinite(odd[-2:]))
 
 
+@pytest.mark.parametrize("q_count,k_count,causal", [(3, 40, False), (20, 40, False), (40, 300, False), (3, 64, False),
+                                                    (20, 1500, False), (2, 33, True), (17, 40, True)])
+def test_attention_seen_values_may_be_infinite(ctx, q_count, k_count, causal):
+    # 64-channel heads: the last key's infinite value reaches the queries that
+    # see it as an infinity of its sign (a softmax weight above zero times it),
+    # also where its tile of keys has room for more.
+    width = 128
+    q = S.normal_values(q_count * width, 1, 1.0).reshape(q_count, width)
+    k = S.normal_values(k_count * width, 2, 1.0).reshape(k_count, width)
+    v = S.normal_values(k_count * width, 3, 1.0).reshape(k_count, width)
+    v[-1] = np.where(np.arange(width) % 2 == 0, np.inf, -np.inf)
+    out = dev(np.zeros((q_count, width), np.float32))
+    ctx.attention(dev(q), q_count, dev(k), dev(v), k_count, width, 2, causal, 0.125, out)
+    sync()
+    got = out.cpu().numpy()
+    if causal:
+        assert np.all(np.isfinite(got[:-1]))
+        got = got[-1:]
+    assert np.array_equal(got, np.broadcast_to(v[-1], got.shape))
+
+
 def test_attention_refuses_wide_heads(ctx):
     from whispereacp_amd.decoder import LogicError
     q = dev(np.zeros((1, 128), np.float32))

@@ -408,10 +408,11 @@ __global__ void __launch_bounds__(kQueryWaves * kWave) query_attention_kernel(
                 const int key = min(k0 + 16 * b + 4 * g + r, end - 1);
                 vf[b][r] = *reinterpret_cast<const float4v*>(values + (size_t) key * width + column + 4 * li);
             }
-        // Keys that some of these queries do not see get weight zero in the
-        // products, which hides a value only while it is finite.
+        // Keys that some of these queries do not see, and the last key again in
+        // place of those past the end, get weight zero in the products, which
+        // hides a value only while it is finite.
         bool hidden_odd = false;
-        if (causal && k0 + kQueryKeys > past + first_query + 1)
+        if (k0 + kQueryKeys > (causal ? min(end, past + first_query + 1) : end))
         {
 #pragma unroll
             for (int b = 0; b < 2; ++b)
