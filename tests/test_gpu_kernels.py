@@ -345,6 +345,19 @@ def test_attention_seen_values_may_be_infinite(ctx, q_count, k_count, causal):
     assert np.array_equal(got, np.broadcast_to(v[-1], got.shape))
 
 
+@pytest.mark.parametrize("q_count,k_count", [(3, 40), (20, 200)])
+def test_attention_rows_may_start_at_any_float(ctx, oracle, q_count, k_count):
+    width = 128
+    q, k, v = (S.normal_values(n * width + 1, seed, 1.0) for seed, n in ((1, q_count), (2, k_count), (3, k_count)))
+    out = dev(np.zeros(q_count * width + 1, np.float32))
+    ctx.attention(dev(q)[1:], q_count, dev(k)[1:], dev(v)[1:], k_count, width, 2, True, 0.125, out[1:])
+    sync()
+    expected = oracle.attention(*(a[1:].reshape(-1, width).copy() for a in (q, k, v)), 2, True,
+                                first_query=k_count - q_count)
+    got = out.cpu().numpy()
+    assert got[0] == 0.0 and worst_error(got[1:].reshape(q_count, width), expected) < 1e-5
+
+
 def test_attention_refuses_wide_heads(ctx):
     from whispereacp_amd.decoder import LogicError
     q = dev(np.zeros((1, 128), np.float32))

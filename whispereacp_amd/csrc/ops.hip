@@ -353,7 +353,8 @@ __global__ void __launch_bounds__(kBlock) attention_combine_kernel(const float* 
 // of channels 4·row + t. 96 queries over 1500 keys of 12 heads: 160 us as one
 // block per (query, head, chunk) of vector code, 17 here. Bound by the
 // K and V reads of each query tile from the L2s and, at these sizes, by the
-// chain load, score, softmax, merge.
+// chain load, score, softmax, merge. The rows may start at any float (the loads
+// are 16 bytes wide all the same).
 // ---------------------------------------------------------------------------
 constexpr int kQueryWaves = 8;
 constexpr int kQueryKeys = 32; // keys a wave takes at a time
@@ -383,7 +384,7 @@ __global__ void __launch_bounds__(kQueryWaves * kWave) query_attention_kernel(
 #pragma unroll
         for (int j = 0; j < 4; ++j)
         {
-            qf[t][j] = *reinterpret_cast<const float4v*>(row + 16 * j);
+            qf[t][j] = *reinterpret_cast<const float4u*>(row + 16 * j);
             o[t][j] = float4v {0.f, 0.f, 0.f, 0.f};
         }
         m[t] = -INFINITY;
@@ -398,7 +399,7 @@ __global__ void __launch_bounds__(kQueryWaves * kWave) query_attention_kernel(
             for (int j = 0; j < 4; ++j)
             {
                 const int key = min(k0 + 16 * b + li, end - 1);
-                kf[b][j] = *reinterpret_cast<const float4v*>(keys + (size_t) key * width + column + 16 * j + 4 * g);
+                kf[b][j] = *reinterpret_cast<const float4u*>(keys + (size_t) key * width + column + 16 * j + 4 * g);
             }
 #pragma unroll
         for (int b = 0; b < 2; ++b)
@@ -406,7 +407,7 @@ __global__ void __launch_bounds__(kQueryWaves * kWave) query_attention_kernel(
             for (int r = 0; r < 4; ++r)
             {
                 const int key = min(k0 + 16 * b + 4 * g + r, end - 1);
-                vf[b][r] = *reinterpret_cast<const float4v*>(values + (size_t) key * width + column + 4 * li);
+                vf[b][r] = *reinterpret_cast<const float4u*>(values + (size_t) key * width + column + 4 * li);
             }
         // Keys that some of these queries do not see, and the last key again in
         // place of those past the end, get weight zero in the products, which
