@@ -102,6 +102,31 @@ def test_linear_paths(ctx, dtype, rows, inner, out):
 
 
 @pytest.mark.parametrize("dtype", ["F16", "BF16"])
+@pytest.mark.parametrize("rows,inner,out,flags", [
+    (1500, 96, 384, 0), (1500, 160, 1536, 3), (3001, 32, 5632, 2),  # K in odd 32s: tiles of 32, 64 and 128 rows
+    (1500, 96, 128, 3), (500, 96, 640, 0), (513, 1056, 1152, 0)])   # few tiles, on either side of the rules
+def test_linear_of_parts_cut_on_the_way(ctx, dtype, rows, inner, out, flags):
+    # Many rows of 16-bit weights that do not go through stored parts, against
+    # float64; the bound is test_linear_matches_oracle's.
+    from whispereacp_amd.decoder import stored_to_device
+    x = S.normal_values(rows * inner, 19, 1.0).reshape(rows, inner)
+    stored, w = weights(out, inner, dtype, 23)
+    bias = S.normal_values(out, 29, 0.1)
+    start = S.normal_values(rows * out, 17, 1.0).reshape(rows, out)
+    wdev, wdtype = stored_to_device(S.StoredTensor("w", dtype, (out, inner), stored))
+    y = dev(start.copy())
+    ctx.linear(dev(x), rows, inner, wdev, wdtype, dev(bias), y, out, flags)
+    sync()
+    expected = x.astype(np.float64) @ w.astype(np.float64).T + bias
+    if flags & 1:
+        import torch
+        expected = torch.nn.functional.gelu(torch.from_numpy(expected)).numpy()
+    if flags & 2:
+        expected = expected + start
+    assert worst_error(y.cpu().numpy(), expected) <= 1e-5 + 2.4e-7 * inner
+
+
+@pytest.mark.parametrize("dtype", ["F16", "BF16"])
 @pytest.mark.parametrize("rows,inner,out", [(1100, 4096, 256), (2101, 4096, 128), (300, 16384, 512)])
 def test_linear_beyond_the_scratch(dtype, rows, inner, out):
     # A context whose scratch (16 MB at least) does not hold the rows' parts:
@@ -124,7 +149,7 @@ def test_linear_beyond_the_scratch(dtype, rows, inner, out):
 
 @pytest.mark.parametrize("dtype", ["F32", "F16", "BF16"])
 @pytest.mark.parametrize("rows,inner,out,count", [(3, 64, 128, 3), (17, 64, 128, 70), (300, 128, 256, 5),
-                                                  (300, 96, 64, 4), (40, 40, 24, 4)])
+                                                  (300, 96, 64, 4), (40, 40, 24, 4), (1500, 96, 256, 4)])
 def test_linear_many_equals_each_alone(ctx, dtype, rows, inner, out, count):
     # Several weights over the same rows in shared launches: past a launch's 64
     # matrices, over stored parts, in fp32 and three at a time.

@@ -24,8 +24,12 @@
 // 16-bit weights in their own type with X cut into exact 16-bit parts (as
 // split_product's), otherwise everything is fp32.
 //
-// W is the matrix cores' row operand, X their column operand: a lane ends up
-// with four consecutive outputs of one row.
+// In these two W is the matrix cores' row operand, X their column operand: a
+// lane ends up with four consecutive outputs of one row.
+//
+// cut_product_kernel: many rows of 16-bit weights that split_product does not
+// take (K in odd multiples of 32, or parts that the scratch does not hold). X is
+// cut into its 16-bit parts on its way through registers into LDS, 32 k a step.
 #include "device_common.h"
 #include "ops.h"
 
@@ -441,6 +445,129 @@ __global__ void __launch_bounds__(kRowWaves * kWave) row_product_kernel(RowProdu
     }
 }
 
+// ---------------------------------------------------------------------------
+// Many rows, parts cut on the way
+// ---------------------------------------------------------------------------
+constexpr int kCutThreads = 256;
+constexpr int kCutColumns = 128;
+constexpr int kCutStep = 32;
+constexpr int kCutRow = kCutStep + 16; // 16-bit values an LDS row: at 96 bytes its reads conflict half as often as at 80
+
+// TM rows by 128 columns of one matrix a block, its four waves 2 x 2; the next
+// step's loads are in flight over this one's products.
+template <int WT, int TM>
+__global__ void __launch_bounds__(kCutThreads) cut_product_kernel(RowProduct a)
+{
+    constexpr int P = WT == kF16 ? 2 : 3, NT = 4;
+    constexpr int MT = TM / 32;                       // 16-row tiles a wave
+    constexpr int kValues = TM * kCutStep / kCutThreads; // of X a thread moves a step: 16, 8 or 4
+    constexpr int kRowThreads = kCutStep / kValues;
+    __shared__ __attribute__((aligned(16))) u16 xs[P][TM][kCutRow];
+    __shared__ __attribute__((aligned(16))) u16 ws[kCutColumns][kCutRow];
+
+    const int tid = threadIdx.x, wave = tid / kWave, lane = tid % kWave, li = lane % 16, g = lane / 16;
+    const int wm = wave / 2, wn = wave % 2;
+    const int m_block = blockIdx.y * TM, n_block = blockIdx.x * kCutColumns;
+    const Column first = column_of(a, n_block);
+
+    // Rows past the end re-read the last one; their outputs are not stored.
+    const int xr = tid / kRowThreads, xk = tid % kRowThreads * kValues;
+    constexpr int kRuns = kValues / 4;
+    const int wr = tid / 2, wk = tid % 2 * 16;
+    const float* const x = a.x + (size_t) min(m_block + xr, a.rows - 1) * a.inner + xk;
+    const u16* const w = static_cast<const u16*>(first.w) + (size_t) (first.c + wr) * a.inner + wk;
+    float4v xv[kRuns];
+    u32x4 wv[2];
+    auto fetch = [&](int k0) {
+#pragma unroll
+        for (int i = 0; i < kRuns; ++i)
+            xv[i] = *reinterpret_cast<const float4v*>(x + k0 + 4 * i);
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+            wv[i] = *reinterpret_cast<const u32x4*>(w + k0 + 8 * i);
+    };
+
+    float4v acc[MT][NT];
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+        for (int nt = 0; nt < NT; ++nt)
+            acc[mt][nt] = float4v {0.f, 0.f, 0.f, 0.f};
+
+    fetch(0);
+    for (int k0 = 0; k0 < a.inner; k0 += kCutStep)
+    {
+        __syncthreads(); // the previous step has been read
+        uint2 cut[kRuns][P];
+#pragma unroll
+        for (int i = 0; i < kRuns; ++i)
+        {
+            uint32_t bits[4][3];
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+                exact_parts<WT>(xv[i][e], bits[e]);
+#pragma unroll
+            for (int p = 0; p < P; ++p)
+                cut[i][p] = uint2 {bits[0][p] | (bits[1][p] << 16), bits[2][p] | (bits[3][p] << 16)};
+        }
+#pragma unroll
+        for (int p = 0; p < P; ++p)
+            if constexpr (kRuns == 1)
+                *reinterpret_cast<uint2*>(&xs[p][xr][xk]) = cut[0][p];
+            else
+#pragma unroll
+                for (int i = 0; i < kRuns; i += 2)
+                    *reinterpret_cast<u32x4*>(&xs[p][xr][xk + 4 * i])
+                        = u32x4 {cut[i][p].x, cut[i][p].y, cut[i + 1][p].x, cut[i + 1][p].y};
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+            *reinterpret_cast<u32x4*>(&ws[wr][wk + 8 * i]) = wv[i];
+        __syncthreads();
+        if (k0 + kCutStep < a.inner)
+            fetch(k0 + kCutStep);
+        u32x4 xf[MT][P], wf[NT];
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+            for (int p = 0; p < P; ++p)
+                xf[mt][p] = *reinterpret_cast<const u32x4*>(&xs[p][16 * (MT * wm + mt) + li][8 * g]);
+#pragma unroll
+        for (int nt = 0; nt < NT; ++nt)
+            wf[nt] = *reinterpret_cast<const u32x4*>(&ws[16 * (NT * wn + nt) + li][8 * g]);
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+            for (int nt = 0; nt < NT; ++nt)
+#pragma unroll
+                for (int p = 0; p < P; ++p)
+                    acc[mt][nt] = mfma16<WT>(xf[mt][p], wf[nt], acc[mt][nt]);
+    }
+
+    // acc[mt][nt][r] of lane (g, li) is row 4g + r, column li of that tile.
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+        {
+            const int row = m_block + 16 * (MT * wm + mt) + 4 * g + r;
+            if (row >= a.rows)
+                continue;
+            float* const y = first.y + (size_t) (row / a.rows_per_group) * a.group_stride
+                             + (size_t) (row % a.rows_per_group) * a.ldy;
+#pragma unroll
+            for (int nt = 0; nt < NT; ++nt)
+            {
+                const int c = first.c + 16 * (NT * wn + nt) + li;
+                float v = acc[mt][nt][r];
+                if (first.bias != nullptr)
+                    v += first.bias[c];
+                if (a.flags & 1)
+                    v = exact_gelu(v);
+                y[c] = a.flags & 2 ? y[c] + v : v;
+            }
+        }
+}
+
 int compute_units()
 {
     static const int units = [] {
@@ -485,6 +612,14 @@ hipError_t launch_row(hipStream_t stream, const RowProduct& a)
     return hipGetLastError();
 }
 
+template <int WT, int TM>
+hipError_t launch_cut(hipStream_t stream, const RowProduct& a)
+{
+    hipLaunchKernelGGL((cut_product_kernel<WT, TM>), dim3(a.out / kCutColumns, (a.rows + TM - 1) / TM),
+                       dim3(kCutThreads), 0, stream, a);
+    return hipGetLastError();
+}
+
 RowProduct row_product(const Products& p, int first, int count)
 {
     RowProduct a {};
@@ -521,10 +656,13 @@ SplitProduct split_product_of(const Products& p, const void* parts, size_t part_
     return a;
 }
 
-// Rows of X whose parts the scratch holds at a time: all of them, else equal
-// slabs in whole 32-row tiles; 0 where those would be of fewer than
-// kLeastSlab rows, or where the output's rows lie in groups.
-constexpr int kLeastSlab = 256;
+// Rows of X whose parts the scratch holds at a time: all of them, else half of
+// them in whole 32-row tiles; 0 where it holds less or fewer than kLeastSlab
+// rows, or where the output's rows lie in groups. (In shorter slabs each launch
+// leaves CUs idle: 1500 x 16384 -> 1280 in six of 256 rows 365 us, 306 in
+// cut_product_kernel, 3000 x 5120 -> 384 in four 110 against 102; 1000 x 8192 ->
+// 512 in two 72 against 144.)
+constexpr int kLeastSlab = 512;
 int slab_rows(const Products& p, const Scratch& scratch)
 {
     const size_t row_bytes = (size_t) p.inner * 2 * (p.wdtype == kF16 ? 2 : 3);
@@ -532,46 +670,63 @@ int slab_rows(const Products& p, const Scratch& scratch)
     if ((size_t) p.rows <= held)
         return p.rows;
     const int whole = (int) (held / 32 * 32);
-    if (whole < kLeastSlab || p.rows > p.rows_per_group)
-        return 0;
-    const int slabs = (p.rows + whole - 1) / whole;
-    return ((p.rows + slabs - 1) / slabs + 31) / 32 * 32;
+    const int half = ((p.rows + 1) / 2 + 31) / 32 * 32;
+    return whole < kLeastSlab || half > whole || p.rows > p.rows_per_group ? 0 : half;
+}
+
+// Parts without storing them, two or three matrices at a time. Up to 2^17 outputs
+// row_product_kernel in 16 x 32 tiles; more, in 32 x 64 tiles while those do not
+// give each CU one, or two where K is long (a tile's eight waves share it):
+// 300 x 1056 -> 1152 10.5 us against 18.5 in cut_product_kernel's tiles, 700 x
+// 3104 -> 768 40 against 59, but 300 x 96 -> 5120 14 against 8.5 and 1500 x
+// 2080 -> 5120 215 against 94. Those tiles are of 128 rows, halved while they
+// give fewer than four blocks a CU, and again below one.
+template <int WT>
+hipError_t unstored_parts_product(hipStream_t stream, const Products& p)
+{
+    const long long units = compute_units(), out = (long long) p.columns * p.count;
+    auto blocks = [&](int tm, int tn) { return (p.rows + tm - 1) / tm * (out / tn); };
+    const bool few = p.rows * out <= 1 << 17, some = blocks(32, 64) <= (p.inner < 1024 ? units : 2 * units);
+    hipError_t e = hipSuccess;
+    for (int i = 0; i < p.count && e == hipSuccess; i += kMatrices)
+    {
+        const RowProduct a = row_product(p, i, std::min(kMatrices, p.count - i));
+        e = few                               ? launch_row<WT, 1, 2, true>(stream, a)
+            : some                            ? launch_row<WT, 2, 4, true>(stream, a)
+            : blocks(64, 128) < units         ? launch_cut<WT, 32>(stream, a)
+            : blocks(128, 128) < 4 * units    ? launch_cut<WT, 64>(stream, a)
+                                              : launch_cut<WT, 128>(stream, a);
+    }
+    return e;
 }
 
 // 16-bit weights with X in 16-bit parts. From 2^17 outputs on (every matrix
 // together) X is stored as parts, every matrix going through split_product in
-// launches of up to 64; fewer, and what the scratch does not hold, through
-// row_product_kernel: 96 x 768 -> 768 runs 5.3 us there, 96 x 3072 -> 768 13;
-// 200 x 5120 -> 1280 39, against 20 with the parts' launch.
+// launches of up to 64; fewer, and what split_product or the scratch does not
+// take, without (96 x 768 -> 768 runs 5.3 us there, 96 x 3072 -> 768 13; 200 x
+// 5120 -> 1280 39, against 20 with the parts' launch).
 template <int WT>
 hipError_t parts_product(hipStream_t stream, const Products& p, const Scratch& scratch)
 {
     const long long outputs = (long long) p.rows * p.columns * p.count;
-    hipError_t e = hipSuccess;
     const int slab = slab_rows(p, scratch);
-    if (outputs > 1 << 17 && slab > 0 && split_product_fits(p.wdtype, p.inner, p.columns)
-        && (size_t) p.columns * p.inner < 1u << 30) // (32-bit byte offsets)
+    if (outputs <= 1 << 17 || slab == 0 || !split_product_fits(p.wdtype, p.inner, p.columns)
+        || (size_t) p.columns * p.inner >= 1u << 30) // (32-bit byte offsets)
+        return unstored_parts_product<WT>(stream, p);
+    hipError_t e = hipSuccess;
+    for (int first = 0; first < p.rows && e == hipSuccess; first += slab)
     {
-        for (int first = 0; first < p.rows && e == hipSuccess; first += slab)
+        const int rows = std::min(slab, p.rows - first);
+        const size_t values = (size_t) rows * p.inner;
+        e = split_rows(stream, p.x + (size_t) first * p.inner, values, p.wdtype, scratch.data, values);
+        for (int i = 0; i < p.count && e == hipSuccess; i += kMaxMatrices)
         {
-            const int rows = std::min(slab, p.rows - first);
-            const size_t values = (size_t) rows * p.inner;
-            e = split_rows(stream, p.x + (size_t) first * p.inner, values, p.wdtype, scratch.data, values);
-            for (int i = 0; i < p.count && e == hipSuccess; i += kMaxMatrices)
-            {
-                SplitProduct a = split_product_of(p, scratch.data, values, i, std::min(kMaxMatrices, p.count - i));
-                a.rows = rows;
-                for (int m = 0; m < a.count; ++m)
-                    a.matrix[m].y += (size_t) first * p.ldy;
-                e = split_product(stream, a);
-            }
+            SplitProduct a = split_product_of(p, scratch.data, values, i, std::min(kMaxMatrices, p.count - i));
+            a.rows = rows;
+            for (int m = 0; m < a.count; ++m)
+                a.matrix[m].y += (size_t) first * p.ldy;
+            e = split_product(stream, a);
         }
-        return e;
-    }
-    for (int i = 0; i < p.count && e == hipSuccess; i += kMatrices)
-    {
-        const RowProduct a = row_product(p, i, std::min(kMatrices, p.count - i));
-        e = outputs <= 1 << 17 ? launch_row<WT, 1, 2, true>(stream, a) : launch_row<WT, 2, 4, true>(stream, a);
     }
     return e;
 }
