@@ -28,8 +28,8 @@
 // lane ends up with four consecutive outputs of one row.
 //
 // cut_product_kernel: many rows of 16-bit weights that split_product does not
-// take (K in odd multiples of 32, or parts that the scratch does not hold). X is
-// cut into its 16-bit parts on its way through registers into LDS, 32 k a step.
+// take (K in odd multiples of 32, or parts that the scratch does not hold) and
+// of short K, where storing the parts costs more than it gives. X is cut into its 16-bit parts on its way through registers into LDS, 32 k a step.
 #include "device_common.h"
 #include "ops.h"
 
@@ -704,13 +704,20 @@ hipError_t unstored_parts_product(hipStream_t stream, const Products& p)
 // together) X is stored as parts, every matrix going through split_product in
 // launches of up to 64; fewer, and what split_product or the scratch does not
 // take, without (96 x 768 -> 768 runs 5.3 us there, 96 x 3072 -> 768 13; 200 x
-// 5120 -> 1280 39, against 20 with the parts' launch).
+// 5120 -> 1280 39, against 20 with the parts' launch). So do short K over many
+// rows where split_product's tiles make one round at most: the launch that stores
+// the parts is then not made up for (1500 x 384 -> 768 in three parts 14.5 us,
+// 11.5 without; 3000 x 384 -> 384 in two 12.9 and 10.6; but 448 x 384 -> 1152
+// 6.8 and 8.5, 1500 x 512 -> 1152 in two 13.0 and 13.7).
 template <int WT>
 hipError_t parts_product(hipStream_t stream, const Products& p, const Scratch& scratch)
 {
-    const long long outputs = (long long) p.rows * p.columns * p.count;
+    const long long units = compute_units(), out = (long long) p.columns * p.count, outputs = p.rows * out;
+    auto blocks = [&](int tm, int tn) { return (p.rows + tm - 1) / tm * (out / tn); };
     const int slab = slab_rows(p, scratch);
-    if (outputs <= 1 << 17 || slab == 0 || !split_product_fits(p.wdtype, p.inner, p.columns)
+    const bool short_inner = p.inner <= (WT == kF16 ? 384 : 512) && p.rows >= 700 && blocks(64, 128) <= units
+                             && 2 * blocks(WT == kF16 ? 64 : 32, 128) >= units;
+    if (outputs <= 1 << 17 || short_inner || slab == 0 || !split_product_fits(p.wdtype, p.inner, p.columns)
         || (size_t) p.columns * p.inner >= 1u << 30) // (32-bit byte offsets)
         return unstored_parts_product<WT>(stream, p);
     hipError_t e = hipSuccess;
