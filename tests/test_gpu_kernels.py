@@ -127,6 +127,27 @@ def test_linear_of_parts_cut_on_the_way(ctx, dtype, rows, inner, out, flags):
     assert worst_error(y.cpu().numpy(), expected) <= 1e-5 + 2.4e-7 * inner
 
 
+@pytest.mark.parametrize("dtype", ["F32", "F16", "BF16"])
+@pytest.mark.parametrize("rows,inner,out", [(4, 256, 128), (16, 256, 128), (17, 256, 128), (300, 1280, 1280),
+                                            (1500, 768, 768), (1500, 384, 768), (40, 64, 96)])
+def test_linear_weights_may_start_at_any_value(ctx, dtype, rows, inner, out):
+    # A weight one value past a 16-byte boundary, on every route; the bound is
+    # test_linear_matches_oracle's.
+    import torch
+    from whispereacp_amd.decoder import stored_to_device
+    x = S.normal_values(rows * inner, 19, 1.0).reshape(rows, inner)
+    stored, w = weights(out, inner, dtype, 23)
+    wdev, wdtype = stored_to_device(S.StoredTensor("w", dtype, (out, inner), stored))
+    moved = torch.empty(out * inner + 1, dtype=wdev.dtype, device="cuda")[1:]
+    moved.copy_(wdev.reshape(-1))
+    assert moved.data_ptr() % 16 != 0
+    y = dev(np.full((rows, out), np.nan, np.float32))
+    ctx.linear(dev(x), rows, inner, moved, wdtype, None, y, out, 0)
+    sync()
+    expected = x.astype(np.float64) @ w.astype(np.float64).T
+    assert worst_error(y.cpu().numpy(), expected) <= 1e-5 + 2.4e-7 * inner
+
+
 @pytest.mark.parametrize("dtype", ["F16", "BF16"])
 @pytest.mark.parametrize("rows,inner,out", [(1100, 4096, 256), (2101, 4096, 128), (300, 16384, 512)])
 def test_linear_beyond_the_scratch(dtype, rows, inner, out):

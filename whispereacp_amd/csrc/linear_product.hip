@@ -28,8 +28,8 @@
 // lane ends up with four consecutive outputs of one row.
 //
 // cut_product_kernel: many rows of 16-bit weights that split_product does not
-// take (K in odd multiples of 32, or parts that the scratch does not hold) and
-// of short K, where storing the parts costs more than it gives. X is cut into its 16-bit parts on its way through registers into LDS, 32 k a step.
+// take (K in odd multiples of 32, W not at 16 bytes, or parts that the scratch
+// does not hold) and of short K, where storing the parts costs more than it gives. X is cut into its 16-bit parts on its way through registers into LDS, 32 k a step.
 #include "device_common.h"
 #include "ops.h"
 
@@ -42,6 +42,7 @@ namespace
 typedef uint16_t u16;
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+typedef uint32_t u32x4u __attribute__((ext_vector_type(4), aligned(2))); // the same at any 16-bit value
 
 // Up to three matrices a launch here.
 constexpr int kMatrices = 3;
@@ -90,8 +91,9 @@ __device__ __forceinline__ void store_output(const RowProduct& a, int row, int n
 // COUNT consecutive values of a row from element `index` on, as loaded: kept
 // raw until values() so that nothing waits for the load before its use. Past
 // the row's end (`left` elements from `index` on) they read as zero. VEC:
-// 16-byte loads (8 for four 16-bit values), the row's end a multiple of COUNT;
-// a run past it loads the matrix's first values instead.
+// 16-byte loads (8 for four 16-bit values, which may lie at any of them), the
+// row's end a multiple of COUNT; a run past it loads the matrix's first values
+// instead.
 template <int WT, int COUNT, bool VEC>
 struct Run
 {
@@ -104,7 +106,7 @@ struct Run
         {
             const size_t at = left > 0 ? index : 0;
             constexpr int kPiece = kWords >= 4 ? 4 : 2;
-            typedef uint32_t piece __attribute__((ext_vector_type(kPiece)));
+            typedef uint32_t piece __attribute__((ext_vector_type(kPiece), aligned(WT == kF32 ? 4 * kPiece : 2)));
             const piece* p = reinterpret_cast<const piece*>(static_cast<const char*>(base) + at * (WT == kF32 ? 4 : 2));
 #pragma unroll
             for (int i = 0; i < kWords / kPiece; ++i)
@@ -484,7 +486,7 @@ __global__ void __launch_bounds__(kCutThreads) cut_product_kernel(RowProduct a)
             xv[i] = *reinterpret_cast<const float4v*>(x + k0 + 4 * i);
 #pragma unroll
         for (int i = 0; i < 2; ++i)
-            wv[i] = *reinterpret_cast<const u32x4*>(w + k0 + 8 * i);
+            wv[i] = *reinterpret_cast<const u32x4u*>(w + k0 + 8 * i);
     };
 
     float4v acc[MT][NT];
@@ -678,8 +680,8 @@ int slab_rows(const Products& p, const Scratch& scratch)
 // row_product_kernel in 16 x 32 tiles; more, in 32 x 64 tiles while those do not
 // give each CU one, or two where K is long (a tile's eight waves share it):
 // 300 x 1056 -> 1152 10.5 us against 18.5 in cut_product_kernel's tiles, 700 x
-// 3104 -> 768 40 against 59, but 300 x 96 -> 5120 14 against 8.5 and 1500 x
-// 2080 -> 5120 215 against 94. Those tiles are of 128 rows, halved while they
+// 3104 -> 768 40 against 59, but 300 x 96 -> 5120 14 against 7.2 and 1500 x
+// 2080 -> 5120 215 against 92. Those tiles are of 128 rows, halved while they
 // give fewer than four blocks a CU, and again below one.
 template <int WT>
 hipError_t unstored_parts_product(hipStream_t stream, const Products& p)
@@ -706,9 +708,9 @@ hipError_t unstored_parts_product(hipStream_t stream, const Products& p)
 // take, without (96 x 768 -> 768 runs 5.3 us there, 96 x 3072 -> 768 13; 200 x
 // 5120 -> 1280 39, against 20 with the parts' launch). So do short K over many
 // rows where split_product's tiles make one round at most: the launch that stores
-// the parts is then not made up for (1500 x 384 -> 768 in three parts 14.5 us,
-// 11.5 without; 3000 x 384 -> 384 in two 12.9 and 10.6; but 448 x 384 -> 1152
-// 6.8 and 8.5, 1500 x 512 -> 1152 in two 13.0 and 13.7).
+// the parts is then not made up for (1500 x 384 -> 768 in three parts 14.3 us,
+// 11.3 without; 3000 x 384 -> 384 in two 12.7 and 10.7; but 448 x 384 -> 1152
+// 7.5 and 9.7, 1500 x 512 -> 1152 in two 14.8 and 15.6).
 template <int WT>
 hipError_t parts_product(hipStream_t stream, const Products& p, const Scratch& scratch)
 {
@@ -717,8 +719,8 @@ hipError_t parts_product(hipStream_t stream, const Products& p, const Scratch& s
     const int slab = slab_rows(p, scratch);
     const bool short_inner = p.inner <= (WT == kF16 ? 384 : 512) && p.rows >= 700 && blocks(64, 128) <= units
                              && 2 * blocks(WT == kF16 ? 64 : 32, 128) >= units;
-    if (outputs <= 1 << 17 || short_inner || slab == 0 || !split_product_fits(p.wdtype, p.inner, p.columns)
-        || (size_t) p.columns * p.inner >= 1u << 30) // (32-bit byte offsets)
+    if (outputs <= 1 << 17 || short_inner || slab == 0 || !whole_vectors(p, 8)
+        || !split_product_fits(p.wdtype, p.inner, p.columns) || (size_t) p.columns * p.inner >= 1u << 30) // (32-bit byte offsets)
         return unstored_parts_product<WT>(stream, p);
     hipError_t e = hipSuccess;
     for (int first = 0; first < p.rows && e == hipSuccess; first += slab)

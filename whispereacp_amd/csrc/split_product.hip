@@ -451,8 +451,8 @@ int compute_units()
 // rows 1536 -> 384 ran 9.8 us as 141 blocks of 32 x 128, 13.6 as 72 of 64 x 128
 // and 14.5 as 282 of 32 x 64; 768 -> 2304 17.3 as 432 of 64 x 128, 19.9 in 64 x
 // 64 and 23 as 108 of 128 x 256. Up to 512 of K, 128 x 256 tiles also have to
-// give every CU a block (3000 x 256 -> 2048, fp16: 19.0 us as 752 blocks of 64 x
-// 128, 22.1 as 192 of 128 x 256; 1500 x 512 -> 5120 27.1 and 27.7; 768 of K 34.1
+// give every CU a block (3000 x 256 -> 2048, fp16: 18.3 us as 752 blocks of 64 x
+// 128, 21.6 as 192 of 128 x 256; 1500 x 512 -> 5120 27.1 and 27.7; 768 of K 34.1
 // and 34.0). With at most one 64 x 128 block a CU, four
 // stages hide the loads (5120 -> 1280: 45 us against 60 with two); with more,
 // two let the blocks share a CU (768 -> 2304: 17.3 against 19.6 with four).
