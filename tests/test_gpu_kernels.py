@@ -148,6 +148,25 @@ def test_linear_weights_may_start_at_any_value(ctx, dtype, rows, inner, out):
     assert worst_error(y.cpu().numpy(), expected) <= 1e-5 + 2.4e-7 * inner
 
 
+@pytest.mark.parametrize("dtype,inner,out", [("F32", 4, 8), ("F32", 5, 3), ("F16", 8, 8), ("F16", 32, 128)])
+def test_linear_of_more_rows_than_a_launch_takes(ctx, dtype, inner, out):
+    # Past 65535 tiles of 32 rows. The bound is test_linear_matches_oracle's.
+    import torch
+    from whispereacp_amd.decoder import stored_to_device
+    rows = 65535 * 32 + 77
+    x = torch.randn((rows, inner), device="cuda")
+    stored, w = weights(out, inner, dtype, 23)
+    wdev, wdtype = stored_to_device(S.StoredTensor("w", dtype, (out, inner), stored))
+    bias = torch.randn(out, device="cuda")
+    y = torch.full((rows, out), 0.5, device="cuda")
+    ctx.linear(x, rows, inner, wdev, wdtype, bias, y, out, 2)
+    w = torch.from_numpy(w).cuda()
+    for first in range(0, rows, 1 << 19):
+        expected = 0.5 + (x[first:first + (1 << 19)].double() @ w.double().T + bias.double())
+        error = (y[first:first + (1 << 19)].double() - expected).abs() / (1 + expected.abs())
+        assert float(error.max()) <= 1e-5 + 2.4e-7 * inner
+
+
 @pytest.mark.parametrize("dtype", ["F16", "BF16"])
 @pytest.mark.parametrize("rows,inner,out", [(1100, 4096, 256), (2101, 4096, 128), (300, 16384, 512)])
 def test_linear_beyond_the_scratch(dtype, rows, inner, out):

@@ -784,11 +784,44 @@ bool row_product_fits(const Products& product)
     return product.rows <= kSplitRowLimit && whole_vectors(product, 8);
 }
 
+namespace
+{
+// Rows of one call at most: their tiles (of 16 at least) are a launch's y extent,
+// which ends at 65535.
+constexpr int kMostRows = 1 << 19;
+
+// Longer products of one group of rows, in equal calls.
+hipError_t products_in_calls(hipStream_t stream, const Products& p, const Scratch& scratch)
+{
+    const int calls = (p.rows + kMostRows - 1) / kMostRows, most = (p.rows + calls - 1) / calls;
+    hipError_t e = hipSuccess;
+    for (int first = 0; first < p.rows && e == hipSuccess; first += most)
+        for (int i = 0; i < p.count && e == hipSuccess; i += kMaxMatrices)
+        {
+            ProductMatrix matrices[kMaxMatrices];
+            Products part = p;
+            part.x += (size_t) first * p.inner;
+            part.rows = part.rows_per_group = std::min(most, p.rows - first);
+            part.matrices = matrices;
+            part.count = std::min(kMaxMatrices, p.count - i);
+            for (int m = 0; m < part.count; ++m)
+            {
+                matrices[m] = p.matrices[i + m];
+                matrices[m].y += (size_t) first * p.ldy;
+            }
+            e = products(stream, part, scratch);
+        }
+    return e;
+}
+} // namespace
+
 hipError_t products(hipStream_t stream, const Products& given, const Scratch& scratch)
 {
     Products p = given;
     if (p.rows_per_group <= 0)
         p.rows_per_group = p.rows;
+    if (p.rows > kMostRows && p.rows_per_group >= p.rows)
+        return products_in_calls(stream, p, scratch);
     const bool parts = p.rows > kSplitRowLimit && parts_fit(p.wdtype, p.inner, p.columns, p.x);
     switch (p.wdtype)
     {
