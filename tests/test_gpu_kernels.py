@@ -424,6 +424,20 @@ def test_attention_rows_may_start_at_any_float(ctx, oracle, q_count, k_count):
     assert got[0] == 0.0 and worst_error(got[1:].reshape(q_count, width), expected) < 1e-5
 
 
+def test_attention_of_more_queries_than_a_launch_has_tiles(ctx):
+    # Past 65535 tiles of 32 queries, one head over four keys.
+    import torch
+    q_count, k_count = 65535 * 32 + 33, 4
+    q, k, v = (torch.randn((n, 64), device="cuda") for n in (q_count, k_count, k_count))
+    out = torch.zeros((q_count, 64), device="cuda")
+    ctx.attention(q, q_count, k, v, k_count, 64, 1, False, 0.125, out)
+    for first in range(0, q_count, 1 << 19):
+        scores = q[first:first + (1 << 19)].double() @ k.double().T * 0.125
+        expected = torch.softmax(scores, -1) @ v.double()
+        error = (out[first:first + (1 << 19)].double() - expected).abs() / (1 + expected.abs())
+        assert float(error.max()) < 1e-5
+
+
 def test_attention_refuses_wide_heads(ctx):
     from whispereacp_amd.decoder import LogicError
     q = dev(np.zeros((1, 128), np.float32))

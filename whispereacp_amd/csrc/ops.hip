@@ -362,13 +362,14 @@ constexpr int kQueryKeys = 32; // keys a wave takes at a time
 template <int QT>
 __global__ void __launch_bounds__(kQueryWaves * kWave) query_attention_kernel(
     const float* __restrict__ q, int q_count, const float* __restrict__ keys, const float* __restrict__ values,
-    int k_count, int width, int causal, float scale, int splits, int span, float* __restrict__ out,
+    int k_count, int width, int causal, float scale, int splits, int span, int first_tile, float* __restrict__ out,
     float* __restrict__ partials)
 {
     __shared__ float tops[kQueryWaves][QT][16], totals[kQueryWaves][QT][16];
     __shared__ float4v rows[kQueryWaves][16][16]; // [wave][query][channel run of four]
 
-    const int split = blockIdx.x % splits, head = blockIdx.x / splits, first_query = blockIdx.y * 16 * QT;
+    const int split = blockIdx.x % splits, head = blockIdx.x / splits;
+    const int first_query = (first_tile + (int) blockIdx.y) * 16 * QT;
     const int wave = threadIdx.x / kWave, lane = threadIdx.x % kWave, li = lane % 16, g = lane / 16;
     const int column = head * 64;
     const int past = k_count - q_count; // causal: query i sees keys 0 .. past + i
@@ -979,14 +980,20 @@ hipError_t query_attention(hipStream_t stream, const float* q, int q_count, cons
     const int tiles = (q_count + tile - 1) / tile;
     const int splits = std::max(1, std::min(reaches, kQueryBlocks / (heads * tiles)));
     const int span = ((k_count + splits - 1) / splits + kQueryKeys - 1) / kQueryKeys * kQueryKeys;
-    const dim3 grid(heads * splits, tiles), block(kQueryWaves * kWave);
-    if (tile == 32)
-        hipLaunchKernelGGL(query_attention_kernel<2>, grid, block, 0, stream, q, q_count, keys, values, k_count, width,
-                           causal, scale, splits, span, out, partials);
-    else
-        hipLaunchKernelGGL(query_attention_kernel<1>, grid, block, 0, stream, q, q_count, keys, values, k_count, width,
-                           causal, scale, splits, span, out, partials);
-    hipError_t e = hipGetLastError();
+    const dim3 block(kQueryWaves * kWave);
+    constexpr int kMostTiles = 65535; // a launch's y extent
+    hipError_t e = hipSuccess;
+    for (int first = 0; first < tiles && e == hipSuccess; first += kMostTiles)
+    {
+        const dim3 grid(heads * splits, std::min(tiles - first, kMostTiles));
+        if (tile == 32)
+            hipLaunchKernelGGL(query_attention_kernel<2>, grid, block, 0, stream, q, q_count, keys, values, k_count,
+                               width, causal, scale, splits, span, first, out, partials);
+        else
+            hipLaunchKernelGGL(query_attention_kernel<1>, grid, block, 0, stream, q, q_count, keys, values, k_count,
+                               width, causal, scale, splits, span, first, out, partials);
+        e = hipGetLastError();
+    }
     if (e != hipSuccess || splits == 1)
         return e;
     hipLaunchKernelGGL(attention_combine_kernel, dim3(heads * q_count), dim3(kBlock), 0, stream, partials, q_count,
