@@ -411,7 +411,23 @@ def test_attention_seen_values_may_be_infinite(ctx, q_count, k_count, causal):
     assert np.array_equal(got, np.broadcast_to(v[-1], got.shape))
 
 
-@pytest.mark.parametrize("q_count,k_count", [(3, 40), (20, 200)])
+@pytest.mark.parametrize("q_count,k_count,heads,causal", [
+    (17, 17, 12, True), (17, 32, 12, False), (17, 40, 20, True), (17, 41, 20, True), (224, 1, 6, False),
+    (100, 20, 12, False), (30, 33, 8, False)])
+def test_attention_of_many_queries_over_few_keys(ctx, oracle, q_count, k_count, heads, causal):
+    # On either side of the rule that gives each (query, head) a block; the bound
+    # is test_attention_matches_oracle's.
+    width = 64 * heads
+    q, k, v = (S.normal_values(n * width, seed, 1.0).reshape(n, width)
+               for seed, n in ((1, q_count), (2, k_count), (3, k_count)))
+    out = dev(np.zeros((q_count, width), np.float32))
+    ctx.attention(dev(q), q_count, dev(k), dev(v), k_count, width, heads, causal, 0.125, out)
+    sync()
+    expected = oracle.attention(q, k, v, heads, causal, first_query=k_count - q_count)
+    assert worst_error(out.cpu().numpy(), expected) < 1e-5
+
+
+@pytest.mark.parametrize("q_count,k_count", [(3, 40), (20, 200), (20, 20)])
 def test_attention_rows_may_start_at_any_float(ctx, oracle, q_count, k_count):
     width = 128
     q, k, v = (S.normal_values(n * width + 1, seed, 1.0) for seed, n in ((1, q_count), (2, k_count), (3, k_count)))

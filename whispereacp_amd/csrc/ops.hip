@@ -224,7 +224,7 @@ __global__ void __launch_bounds__(kBlock) attention_chunk_kernel(
     const float* qrow = q + (size_t) query * width + column;
     float4v qv = {0.f, 0.f, 0.f, 0.f};
     if (4 * sub < head_width)
-        qv = *reinterpret_cast<const float4v*>(qrow + 4 * sub);
+        qv = *reinterpret_cast<const float4u*>(qrow + 4 * sub);
 
     float local_max = -INFINITY;
     for (int j = group; j < count; j += 16)
@@ -233,7 +233,7 @@ __global__ void __launch_bounds__(kBlock) attention_chunk_kernel(
         if (4 * sub < head_width)
         {
             const float4v kv =
-                *reinterpret_cast<const float4v*>(keys + (size_t) (first + j) * width + column + 4 * sub);
+                *reinterpret_cast<const float4u*>(keys + (size_t) (first + j) * width + column + 4 * sub);
             part = qv[0] * kv[0] + qv[1] * kv[1] + qv[2] * kv[2] + qv[3] * kv[3];
         }
 #pragma unroll
@@ -1008,7 +1008,15 @@ hipError_t attention(hipStream_t stream, const float* q, int q_count, const floa
     const int head_width = width / heads;
     unsigned int* const counters = reinterpret_cast<unsigned int*>(workspace);
     float* const partials = workspace + kAttentionCounters;
-    if (q_count > 1 && head_width == 64)
+    // More queries than a prompt step's over few keys: one launch of a block for
+    // each (query, head), while those fit one round (eight a CU) and their scores
+    // are few. 17 queries of 12 heads over 20 keys: 4.4 us, 5.0 in
+    // query_attention_kernel; 40 of 20 heads over 20 keys 4.7 and 4.9, over 33
+    // 5.5 and 5.3; 100 of 12 heads over 20 5.1 and 5.0.
+    const long long units = (long long) heads * q_count;
+    const bool few_keys = q_count > kMaxPromptQueries && k_count <= 40 && units <= 2048 && units * k_count <= 20000
+                          && attention_chunks(heads, q_count, k_count) == 1;
+    if (q_count > 1 && head_width == 64 && !few_keys)
         return query_attention(stream, q, q_count, keys, values, k_count, width, heads, causal, scale, out, partials);
     if (takes_prompt_attention(q_count, heads))
     {
