@@ -427,6 +427,16 @@ def test_attention_of_many_queries_over_few_keys(ctx, oracle, q_count, k_count, 
     assert worst_error(out.cpu().numpy(), expected) < 1e-5
 
 
+@pytest.mark.parametrize("k_count", [33, 100, 128, 129, 256, 257, 448])
+def test_attention_combines_any_number_of_chunks(ctx, oracle, k_count):
+    # One query of six heads: two chunks, and either side of four and eight.
+    q, k, v = (S.normal_values(n * 384, seed, 1.0).reshape(n, 384) for seed, n in ((1, 1), (2, k_count), (3, k_count)))
+    out = dev(np.zeros((1, 384), np.float32))
+    ctx.attention(dev(q), 1, dev(k), dev(v), k_count, 384, 6, True, 0.125, out)
+    sync()
+    assert worst_error(out.cpu().numpy(), oracle.attention(q, k, v, 6, True, first_query=k_count - 1)) < 1e-5
+
+
 @pytest.mark.parametrize("q_count,k_count", [(3, 40), (20, 200), (20, 20)])
 def test_attention_rows_may_start_at_any_float(ctx, oracle, q_count, k_count):
     width = 128

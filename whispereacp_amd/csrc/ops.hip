@@ -282,13 +282,14 @@ __global__ void __launch_bounds__(kBlock) attention_chunk_kernel(
     }
 }
 
-// A wave for each fourth chunk, eight chunks' loads in flight: walking them
-// one after the other cost 18 us for 32 chunks of eight heads.
+// A wave for each fourth chunk, AHEAD chunks' loads in flight: walking them one
+// after the other cost 18 us for 32 chunks of eight heads. (As many as there are
+// four or eight: the loads of eight cost two chunks of 12 heads 0.4 us of 7.5.)
+template <int AHEAD>
 __global__ void __launch_bounds__(kBlock) attention_combine_kernel(const float* __restrict__ partials, int q_count,
                                                                    int width, int head_width, int chunks,
                                                                    float* __restrict__ out)
 {
-    constexpr int kAhead = 8;
     __shared__ float sums[kWavesPerBlock][2][kMaxHeadWidth];
     const int query = blockIdx.x % q_count;
     const int head = blockIdx.x / q_count;
@@ -302,11 +303,11 @@ __global__ void __launch_bounds__(kBlock) attention_combine_kernel(const float* 
     largest = wave_max(largest);
 
     float numerator = 0.f, denominator = 0.f;
-    for (int k0 = wave; k0 < chunks; k0 += kAhead * kWavesPerBlock)
+    for (int k0 = wave; k0 < chunks; k0 += AHEAD * kWavesPerBlock)
     {
-        float top[kAhead], sum[kAhead], row[kAhead];
+        float top[AHEAD], sum[AHEAD], row[AHEAD];
 #pragma unroll
-        for (int i = 0; i < kAhead; ++i)
+        for (int i = 0; i < AHEAD; ++i)
         {
             const float* part = base + (size_t) min(k0 + i * kWavesPerBlock, chunks - 1) * pitch;
             top[i] = part[0];
@@ -314,7 +315,7 @@ __global__ void __launch_bounds__(kBlock) attention_combine_kernel(const float* 
             row[i] = part[2 + min(c, head_width - 1)];
         }
 #pragma unroll
-        for (int i = 0; i < kAhead; ++i)
+        for (int i = 0; i < AHEAD; ++i)
             if (k0 + i * kWavesPerBlock < chunks && sum[i] != 0.f) // (a chunk with no visible key sums to zero)
             {
                 const float factor = expf(top[i] - largest);
@@ -955,6 +956,18 @@ bool takes_prompt_attention(int q_count, int heads)
     return q_count >= 2 && q_count <= kMaxPromptQueries && heads <= kAttentionCounters;
 }
 
+hipError_t combine(hipStream_t stream, const float* partials, int q_count, int width, int heads, int chunks, float* out)
+{
+    auto run = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, dim3(heads * q_count), dim3(kBlock), 0, stream, partials, q_count, width,
+                           width / heads, chunks, out);
+    };
+    chunks <= kWavesPerBlock       ? run(attention_combine_kernel<1>)
+    : chunks <= 2 * kWavesPerBlock ? run(attention_combine_kernel<2>)
+                                   : run(attention_combine_kernel<8>);
+    return hipGetLastError();
+}
+
 size_t attention_workspace_floats(int heads, int q_count, int k_count, int head_width)
 {
     if (takes_prompt_attention(q_count, heads))
@@ -996,9 +1009,7 @@ hipError_t query_attention(hipStream_t stream, const float* q, int q_count, cons
     }
     if (e != hipSuccess || splits == 1)
         return e;
-    hipLaunchKernelGGL(attention_combine_kernel, dim3(heads * q_count), dim3(kBlock), 0, stream, partials, q_count,
-                       width, 64, splits, out);
-    return hipGetLastError();
+    return combine(stream, partials, q_count, width, heads, splits, out);
 }
 
 hipError_t attention(hipStream_t stream, const float* q, int q_count, const float* keys,
@@ -1035,9 +1046,7 @@ hipError_t attention(hipStream_t stream, const float* q, int q_count, const floa
     hipError_t e = hipGetLastError();
     if (e != hipSuccess || chunks == 1)
         return e;
-    hipLaunchKernelGGL(attention_combine_kernel, dim3(heads * q_count), dim3(kBlock), 0, stream,
-                       workspace, q_count, width, head_width, chunks, out);
-    return hipGetLastError();
+    return combine(stream, workspace, q_count, width, heads, chunks, out);
 }
 
 int argmax_groups(int row_length)
