@@ -161,6 +161,18 @@ def test_batch_split_sizing_and_refusals_on_the_host():
     assert "FAIL" not in result.stdout and result.stdout.count("ok ") == 32, result.stdout
 
 
+def test_every_gpu_is_prepared_once():
+    # The products' kernels ask for more LDS than a launch gets unasked, on each
+    # GPU a process uses; the once-per-device guard is host code
+    # (csrc/once_per_device.h), checked here on the CPU under ASan/UBSan.
+    import subprocess
+    path = os.path.join(ROOT, "tests", "native", "_build", "once_per_device_check")
+    subprocess.run(["make", "-s", "_build/once_per_device_check"], cwd=os.path.join(ROOT, "tests", "native"), check=True)
+    result = subprocess.run([path], capture_output=True, text=True, timeout=60)
+    assert result.returncode == 0, result.stdout + result.stderr
+    assert "FAIL" not in result.stdout and result.stdout.count("ok ") == 8, result.stdout
+
+
 def test_headers_compile_as_c99(tmp_path):
     # The C ABI is meant for C callers (cgo, ctypes, plain C): both headers
     # must stand alone as C99, with no C++ in their C view.

@@ -1427,23 +1427,11 @@ bool normed_fits(int rows, int inner)
     return row_tiles(rows) <= 2 && inner <= kNormedWidth && inner % 32 == 0;
 }
 
-int compute_units()
-{
-    static const int units = [] {
-        int device = 0, count = 0;
-        if (hipGetDevice(&device) == hipSuccess
-            && hipDeviceGetAttribute(&count, hipDeviceAttributeMultiprocessorCount, device) == hipSuccess && count > 0)
-            return count;
-        return 256;
-    }();
-    return units;
-}
-
 template <int WT>
 hipError_t launch_normed_product(hipStream_t stream, const Product& a)
 {
     const int tiles = (a.out + 15) / 16;
-    const bool pair = tiles > compute_units();
+    const bool pair = tiles > wsp::ops::compute_units();
     const dim3 grid(pair ? (tiles + 1) / 2 : tiles);
     const bool two_rows = row_tiles(a.rows) != 1;
     if (!pair && !two_rows)
@@ -2224,6 +2212,8 @@ int wsp_batch_create(const wsp_decoder_shape* shape, int streams, int max_step_t
                                       wsp::batch::kMaxSweepGroups});
     const int groups = wsp::ops::argmax_groups(s.vocabulary_size);
     hipError_t e = hipSetDevice(device);
+    if (e == hipSuccess)
+        e = wsp::ops::prepare_split_products();
     if (e == hipSuccess)
         e = allocate(b, &b->self_keys, (size_t) s.layers * self_layer_stride(b));
     if (e == hipSuccess)

@@ -73,6 +73,8 @@ int wsp_hip_ctx_create(const wsp_decoder_shape* shape, int device, void* stream,
 
     int status = hip_status(ctx, hipSetDevice(device), "hipSetDevice");
     if (status == WSP_OK)
+        status = hip_status(ctx, wsp::ops::prepare_split_products(), "products");
+    if (status == WSP_OK)
     {
         const int head_width = shape->width / shape->heads;
         const int longest = std::max(shape->max_positions, shape->cross_positions);

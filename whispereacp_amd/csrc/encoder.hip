@@ -139,18 +139,6 @@ __device__ __forceinline__ f32x4 mfma3(const f16x8& ah, const f16x8& al, const f
     return __builtin_amdgcn_mfma_f32_16x16x32_f16(al, bh, c, 0, 0, 0);
 }
 
-int compute_units()
-{
-    static const int units = [] {
-        int device = 0, count = 0;
-        if (hipGetDevice(&device) == hipSuccess
-            && hipDeviceGetAttribute(&count, hipDeviceAttributeMultiprocessorCount, device) == hipSuccess && count > 0)
-            return count;
-        return 256;
-    }();
-    return units;
-}
-
 // K and V arrive cut into fp16 hi and lo (k_halves [2][pitch][width], vt_halves
 // transposed [2][width][pitch] with each 32 keys in attention_place order, pitch
 // a multiple of the key tile): the q/k/v product writes them, or halves_kernel.
@@ -548,6 +536,8 @@ int wsp_encoder_create(const wsp_encoder_shape* shape, int device, void* stream,
     const size_t d = (size_t) s.width;
     hipError_t status = hipSetDevice(device);
     if (status == hipSuccess)
+        status = wsp::ops::prepare_split_products();
+    if (status == hipSuccess)
         status = encoder_allocate(e, &e->columns, std::max(frames * s.mel_bins * 3, positions * d * 3));
     if (status == hipSuccess)
         status = encoder_allocate(e, &e->conv, std::max(frames, 3 * positions) * d);
@@ -692,7 +682,7 @@ int wsp_encoder_encode(wsp_encoder* e, const wsp_encoder_tensors* T, const float
     ops::SplitProduct conv2 = convolution(e->conv, positions, 3 * d, T->conv2_w, T->conv2_b, e->hidden,
                                           ops::kProductGelu | ops::kProductResidual);
     conv2.residual = T->positions;
-    if (tiles(positions) >= compute_units() && ops::fp32_split_fits(conv1) && ops::fp32_split_fits(conv2))
+    if (tiles(positions) >= ops::compute_units() && ops::fp32_split_fits(conv1) && ops::fp32_split_fits(conv2))
     {
         if ((status = ops::fp32_split(st, conv1)) != hipSuccess)
             return encoder_hip(e, status, "conv1");
@@ -846,12 +836,12 @@ int wsp_encoder_encode(wsp_encoder* e, const wsp_encoder_tensors* T, const float
             // each, and the splits combined after.
             const int narrow_blocks = (positions + 16 * kFlashWaves - 1) / (16 * kFlashWaves) * heads;
             int splits = 1;
-            if (narrow_blocks < compute_units() && e->flash_partials != nullptr)
-                splits = std::max(1, std::min({kMaxFlashSplits, (compute_units() + narrow_blocks - 1) / narrow_blocks,
+            if (narrow_blocks < ops::compute_units() && e->flash_partials != nullptr)
+                splits = std::max(1, std::min({kMaxFlashSplits, (ops::compute_units() + narrow_blocks - 1) / narrow_blocks,
                                                positions / 64}));
             const int span = ((positions + splits - 1) / splits + kFlashKeys - 1) / kFlashKeys * kFlashKeys;
             float* partials = splits > 1 ? e->flash_partials : nullptr;
-            const bool wide = 8 * wide_blocks >= 7 * compute_units();
+            const bool wide = 8 * wide_blocks >= 7 * ops::compute_units();
             const dim3 grid = wide ? dim3((positions + 16 * kFlashWideWaves - 1) / (16 * kFlashWideWaves), heads)
                                    : dim3((positions + 16 * kFlashWaves - 1) / (16 * kFlashWaves), heads, splits);
             const int key_span = wide ? positions : span;

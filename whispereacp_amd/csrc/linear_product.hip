@@ -570,18 +570,6 @@ __global__ void __launch_bounds__(kCutThreads) cut_product_kernel(RowProduct a)
         }
 }
 
-int compute_units()
-{
-    static const int units = [] {
-        int device = 0, count = 0;
-        if (hipGetDevice(&device) == hipSuccess
-            && hipDeviceGetAttribute(&count, hipDeviceAttributeMultiprocessorCount, device) == hipSuccess && count > 0)
-            return count;
-        return 256;
-    }();
-    return units;
-}
-
 bool aligned(const void* p, size_t bytes)
 {
     return reinterpret_cast<uintptr_t>(p) % bytes == 0;

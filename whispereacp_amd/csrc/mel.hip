@@ -422,6 +422,8 @@ int wsp_mel_create(const wsp_mel_shape* shape, int device, void* stream, wsp_mel
     auto angle = [&](int b, int t) { return two_pi * (double) (((long long) b * t) % fft) / fft; };
     hipError_t status = hipSetDevice(device);
     if (status == hipSuccess)
+        status = wsp::ops::prepare_split_products();
+    if (status == hipSuccess)
         status = mel_allocate(m, &m->window, fft);
     if (status == hipSuccess)
         status = mel_allocate(m, &m->peaks, std::max(wsp::mel::kLogBlocks, (s.frame_count + 15) / 16));

@@ -14,6 +14,9 @@ constexpr int kSplitRowLimit = 16;
 constexpr int kMaxHeadWidth = 64;
 constexpr int kAttentionChunkKeys = 1024; // longest key chunk one workgroup scores
 
+// CUs of the current device.
+int compute_units();
+
 // One of the matrices side by side in a product: W [columns][inner], its bias
 // (or null), its output, and the factor its sums are multiplied by before the
 // bias (the reciprocal of the power of two its stored weights carry, exact; 1
@@ -66,6 +69,10 @@ struct SplitProduct
     void* y2_halves_t;
     int halves_pitch;
 };
+
+// What split_product and fp32_split ask of the current device before their first
+// launch there (their stages pass the LDS a launch gets unasked).
+hipError_t prepare_split_products();
 
 // 16-bit weights, inner a multiple of 64, columns of 128.
 bool split_product_fits(int wdtype, int inner, int columns);

@@ -8,6 +8,8 @@
 #include "ops.h"
 
 #include <algorithm>
+#include <array>
+#include <atomic>
 #include <cmath>
 
 namespace wsp::ops
@@ -870,6 +872,20 @@ hipError_t launch_gemv(hipStream_t stream, const float* x, int rows, int inner, 
 }
 
 } // namespace
+
+int compute_units()
+{
+    static std::array<std::atomic<int>, 64> known {};
+    int device = 0, count = 0;
+    if (hipGetDevice(&device) != hipSuccess || device < 0 || device >= (int) known.size())
+        return 256;
+    if ((count = known[device].load(std::memory_order_relaxed)) > 0)
+        return count;
+    if (hipDeviceGetAttribute(&count, hipDeviceAttributeMultiprocessorCount, device) != hipSuccess || count <= 0)
+        return 256;
+    known[device].store(count, std::memory_order_relaxed);
+    return count;
+}
 
 hipError_t linear(hipStream_t stream, const float* x, int rows, int inner, const void* weight,
                   int wdtype, const float* bias, float* y, int out, int flags, const Scratch& scratch)

@@ -37,6 +37,7 @@
 //    384 -> 1152  64 x 128: 6.5 (7.9)    1536 -> 384   32 x 128: 9.8 (20)
 // and at 300 rows 5120 -> 1280 in 32 x 64 tiles 18.5 (57).
 #include "device_common.h"
+#include "once_per_device.h"
 #include "ops.h"
 
 #include <algorithm>
@@ -421,28 +422,55 @@ __global__ void __launch_bounds__(T::kWaves * kWave) split_product_kernel(SplitP
 }
 
 template <class T, int WT>
+hipError_t allow()
+{
+    return hipFuncSetAttribute(reinterpret_cast<const void*>(&split_product_kernel<T, WT>),
+                               hipFuncAttributeMaxDynamicSharedMemorySize, T::S * T::kStageBytes);
+}
+
+template <class T, int WT>
 hipError_t launch(hipStream_t stream, const SplitProduct& a)
 {
-    constexpr int bytes = T::S * T::kStageBytes;
-    static const hipError_t allowed = hipFuncSetAttribute(reinterpret_cast<const void*>(&split_product_kernel<T, WT>),
-                                                          hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
-    if (allowed != hipSuccess)
-        return allowed;
     hipLaunchKernelGGL((split_product_kernel<T, WT>), dim3((a.count * a.columns + T::TN - 1) / T::TN, (a.rows + T::TM - 1) / T::TM),
-                       dim3(T::kWaves * kWave), bytes, stream, a);
+                       dim3(T::kWaves * kWave), T::S * T::kStageBytes, stream, a);
     return hipGetLastError();
 }
 
-int compute_units()
+template <int WT>
+struct Tiles
 {
-    static const int units = [] {
-        int device = 0, count = 0;
-        if (hipGetDevice(&device) == hipSuccess
-            && hipDeviceGetAttribute(&count, hipDeviceAttributeMultiprocessorCount, device) == hipSuccess && count > 0)
-            return count;
-        return 256;
-    }();
-    return units;
+    using Widest = Tile<WT, 128, 256, 2, 4, 2>;
+    using Shared = Tile<WT, 64, 128, 2, 4, 2>; // (two blocks of a CU)
+    using Alone = Tile<WT, 64, 128, 2, 4, 4>;
+    using Short = Tile<WT, 32, 128, 2, WT == kF16 ? 4 : 2, 4>; // (bf16: 28 loads a stage)
+    using Least = Tile<WT, 32, 64, 2, 2, 4>;
+};
+
+template <>
+struct Tiles<kF32>
+{
+    using Whole = Tile<kF32, 64, 64, 2, 2, 2>;
+    using Half = Tile<kF32, 32, 64, 2, 2, 2>;
+    using Quarter = Tile<kF32, 32, 32, 2, 2, 4>;
+};
+
+template <int WT, class... T>
+hipError_t allow_each()
+{
+    hipError_t e = hipSuccess;
+    (void) ((e == hipSuccess && (e = allow<T, WT>()) != hipSuccess) || ...);
+    return e;
+}
+
+template <int WT>
+hipError_t allow_tiles()
+{
+    using T = Tiles<WT>;
+    if constexpr (WT == kF32)
+        return allow_each<WT, typename T::Whole, typename T::Half, typename T::Quarter>();
+    else
+        return allow_each<WT, typename T::Widest, typename T::Shared, typename T::Alone, typename T::Short,
+                          typename T::Least>();
 }
 
 // The largest tile that still occupies half the CUs (the bytes a product moves
@@ -463,14 +491,14 @@ hipError_t launch_tiles(hipStream_t stream, const SplitProduct& a)
     const int out = a.count * a.columns;
     auto blocks = [&](int tm, int tn) { return (long long) ((a.rows + tm - 1) / tm) * (out / tn); };
     if (a.columns % 256 == 0 && (a.inner > 512 ? 2 : 1) * blocks(128, 256) >= units)
-        return launch<Tile<WT, 128, 256, 2, 4, 2>, WT>(stream, a);
+        return launch<typename Tiles<WT>::Widest, WT>(stream, a);
     if (blocks(64, 128) > units)
-        return launch<Tile<WT, 64, 128, 2, 4, 2>, WT>(stream, a);
+        return launch<typename Tiles<WT>::Shared, WT>(stream, a);
     if (2 * blocks(64, 128) >= units)
-        return launch<Tile<WT, 64, 128, 2, 4, 4>, WT>(stream, a);
+        return launch<typename Tiles<WT>::Alone, WT>(stream, a);
     if (2 * blocks(32, 128) >= units)
-        return launch<Tile<WT, 32, 128, 2, WT == kF16 ? 4 : 2, 4>, WT>(stream, a); // (bf16: 28 loads a stage)
-    return launch<Tile<WT, 32, 64, 2, 2, 4>, WT>(stream, a);
+        return launch<typename Tiles<WT>::Short, WT>(stream, a);
+    return launch<typename Tiles<WT>::Least, WT>(stream, a);
 }
 } // namespace
 
@@ -550,10 +578,10 @@ hipError_t fp32_split(hipStream_t stream, const SplitProduct& product)
     };
     const double whole = 1.0 * rounds(64, 64), half = 0.535 * rounds(32, 64), quarter = 0.3 * rounds(32, 32);
     if (whole <= half && whole <= quarter)
-        return launch<Tile<kF32, 64, 64, 2, 2, 2>, kF32>(stream, a);
+        return launch<Tiles<kF32>::Whole, kF32>(stream, a);
     if (half <= quarter)
-        return launch<Tile<kF32, 32, 64, 2, 2, 2>, kF32>(stream, a);
-    return launch<Tile<kF32, 32, 32, 2, 2, 4>, kF32>(stream, a);
+        return launch<Tiles<kF32>::Half, kF32>(stream, a);
+    return launch<Tiles<kF32>::Quarter, kF32>(stream, a);
 }
 
 hipError_t split_product(hipStream_t stream, const SplitProduct& product)
@@ -565,5 +593,20 @@ hipError_t split_product(hipStream_t stream, const SplitProduct& product)
     if (a.rows_per_group <= 0)
         a.rows_per_group = a.rows;
     return a.wdtype == kF16 ? launch_tiles<kF16>(stream, a) : launch_tiles<kBF16>(stream, a);
+}
+
+hipError_t prepare_split_products()
+{
+    static OncePerDevice prepared;
+    int device = 0;
+    const hipError_t e = hipGetDevice(&device);
+    if (e != hipSuccess)
+        return e;
+    return prepared(device, [] {
+        hipError_t status = allow_tiles<kF16>();
+        if (status == hipSuccess)
+            status = allow_tiles<kBF16>();
+        return status == hipSuccess ? allow_tiles<kF32>() : status;
+    });
 }
 } // namespace wsp::ops
