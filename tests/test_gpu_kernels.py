@@ -167,6 +167,35 @@ def test_linear_of_more_rows_than_a_launch_takes(ctx, dtype, inner, out):
         assert float(error.max()) <= 1e-5 + 2.4e-7 * inner
 
 
+@pytest.mark.parametrize("dtype,leading,last", [("F16", 1.0, 2.0 ** -12), ("BF16", 1.0, 2.0 ** -10),
+                                                ("BF16", 1.0 + 2.0 ** -10, 2.0 ** -22)])
+@pytest.mark.parametrize("rows,inner,out", [
+    (17, 1024, 128), (300, 1056, 1152),                                           # few rows, few tiles
+    (1500, 160, 1536), (1500, 128, 384), (3000, 96, 5632),                        # parts cut on the way
+    (300, 1280, 1280), (1500, 1280, 1280), (1500, 768, 384), (1500, 768, 2304), (1500, 768, 5120)])  # stored parts
+def test_linear_keeps_every_part(ctx, dtype, leading, last, rows, inner, out):
+    # Weights +1 and -1 in turn, over which the leading parts of x cancel
+    # exactly, and a last part (fp16's second, bf16's second or third) only
+    # where the weight is +1: the product is that part alone, inner / 2 times,
+    # and zero where a kernel drops it. Every product step sums 32 consecutive k,
+    # over which the leading parts leave nothing, so a sum's terms and partial
+    # sums are of magnitude one and it is exact to 2^-23, a 1/32 of what it holds
+    # of the smallest last part; the bound is four times that. (Up to 16 rows the
+    # products are in fp32 and sum even and odd k apart: partial sums of 64 there
+    # would be exact to 2^-17 only.)
+    import torch
+    sign = np.where(np.arange(inner) % 2 == 0, 1.0, -1.0).astype(np.float32)
+    x = np.broadcast_to((leading + np.where(sign > 0, last, 0.0)).astype(np.float32), (rows, inner))
+    assert np.array_equal(x[0].astype(np.float64), leading + np.where(sign > 0, last, 0.0))
+    w = torch.from_numpy(np.broadcast_to(sign, (out, inner)).copy()).cuda()
+    w = w.half() if dtype == "F16" else w.bfloat16()
+    y = dev(np.full((rows, out), np.nan, np.float32))
+    ctx.linear(dev(x.copy()), rows, inner, w, 1 if dtype == "F16" else 2, None, y, out, 0)
+    sync()
+    expected = last * inner / 2
+    assert np.max(np.abs(y.cpu().numpy().astype(np.float64) - expected)) <= expected / 8
+
+
 @pytest.mark.parametrize("dtype", ["F16", "BF16"])
 @pytest.mark.parametrize("rows,inner,out", [(1100, 4096, 256), (2101, 4096, 128), (300, 16384, 512)])
 def test_linear_beyond_the_scratch(dtype, rows, inner, out):
@@ -554,6 +583,20 @@ def test_cross_kv_projection_matches_oracle(ctx, oracle, dtype, width):
     xd = x.astype(np.float64)
     assert worst_error(k_out.cpu().numpy(), oracle.linear(xd, wk, None)) < 1e-5
     assert worst_error(v_out.cpu().numpy(), oracle.linear(xd, wv, bv)) < 1e-5
+
+
+def test_narrow_heads_prompt_attention_is_deterministic_and_independent_of_the_last_block(ctx):
+    # Heads of other than 64 channels: 16 queries over 1500 keys split across
+    # blocks whose partials the last one to finish combines in split order, with
+    # per-head counters that each launch leaves zero.
+    q, k, v = (dev(S.normal_values(n * 384, seed, 1.0).reshape(n, 384)) for seed, n in ((4, 16), (5, 1500), (6, 1500)))
+    outs = []
+    for _ in range(5):
+        out = dev(np.zeros((16, 384), np.float32))
+        ctx.attention(q, 16, k, v, 1500, 384, 12, False, 0.125, out)
+        sync()
+        outs.append(out.cpu().numpy())
+    assert all(np.array_equal(outs[0], o) for o in outs[1:])
 
 
 def test_prompt_attention_is_deterministic_and_independent_of_the_last_block(ctx):

@@ -49,6 +49,34 @@ def test_other_shapes_match_oracle(oracle, samples, fft, hop, frames, mels):
     assert float(np.max(np.abs(got - expected))) <= 1e-4
 
 
+@pytest.mark.parametrize("samples,fft,hop,frames,mels", [
+    (8000, 600, 160, 33, 20),    # more values of a folded row than one pass of a block folds
+    (8000, 602, 160, 33, 20),    # the same folded once
+    (20000, 1024, 160, 40, 80),  # and a filterbank too large to go through the block's memory
+    (4000, 400, 160, 17, 200)])  # as is one of many bands
+def test_longer_transforms_and_filterbanks_match_oracle(oracle, samples, fft, hop, frames, mels):
+    s = S.MelShape(samples, fft, hop, frames, mels)
+    x = S.tone_and_noise(s.sample_count)
+    f = S.triangular_filters(s.mel_count, s.bin_count)
+    got = gpu_mel(s, x, f)
+    expected = oracle.mel_spectrogram(x, f, s.fft_length, s.hop_length, s.frame_count)
+    assert float(np.max(np.abs(got - expected))) <= 1e-4
+
+
+def test_a_filterbank_may_start_at_any_float(oracle):
+    # One float past a 16-byte boundary it is read from memory: the same sums.
+    from whispereacp_amd.mel import MelSpectrogram
+    s = S.reduced_mel_shape()
+    x, f = S.tone_and_noise(s.sample_count), S.triangular_filters(s.mel_count, s.bin_count)
+    moved = torch.empty(f.size + 1, dtype=torch.float32, device="cuda")[1:].reshape(f.shape)
+    moved.copy_(torch.from_numpy(f))
+    assert moved.data_ptr() % 16 == 4
+    out = torch.empty((s.mel_count, s.frame_count), dtype=torch.float32, device="cuda")
+    MelSpectrogram(s).encode(torch.from_numpy(x).cuda(), moved, out)
+    torch.cuda.synchronize()
+    assert np.array_equal(out.cpu().numpy(), gpu_mel(s, x, f))
+
+
 def test_whisper_shape_spans_two_and_matches_oracle(oracle):
     s = S.MelShape()
     x = S.tone_and_noise(s.sample_count)
