@@ -68,7 +68,9 @@ typedef struct wsp_hip_ctx wsp_hip_ctx;
 
 /* Binds a context to `device` and `stream` (a hipStream_t; null is the
  * default stream) and sizes its workspaces for `shape` (attention partials,
- * argmax candidates). Replaces KernelNet::prepare's scratch and the
+ * argmax candidates, and the 16-bit parts of a product's rows: six bytes for
+ * each value of the longest input over the widest layer, 46 MB at large-v3 and
+ * 16 MB at least). Replaces KernelNet::prepare's scratch and the
  * SingleQueryAttention/Argmax prepare() sizing (Net/KernelNet.cpp:133-207,
  * Kernels/SingleQueryAttention.cpp:32-60, Kernels/Argmax.cpp:26-40). */
 int wsp_hip_ctx_create(const wsp_decoder_shape* shape, int device, void* stream,
@@ -84,12 +86,18 @@ void* wsp_hip_stream(const wsp_hip_ctx* ctx);
 /* y[r, o] = act(Σ_k x[r,k]·W[o,k] + b[o]) (+ y[r,o] when RESIDUAL).
  * x [rows, inner] f32, W [out, inner] row-major in `wdtype`, bias [out] f32 or
  * null (zero, which replaces the zero-bias buffers at
- * Net/KernelNet.cpp:440-458), y [rows, out] f32. Up to four rows take the split
- * GEMV (as do 5 to 16 whose inner extent or addresses are not whole vectors),
- * more the matrix cores: in exact 16-bit parts of x for more than 16 rows of
- * 16-bit weights with inner % 32 == 0 and out % 128 == 0, else in fp32. Replaces KernelNet::dispatchProjection
- * (Net/KernelNet.cpp:817-859) over SplitLinear / HalfWeightSplitLinear
- * (Kernels/Linear.h:129-276) and LinearProduct (Kernels/SimdTiledMatMul.h:470-486). */
+ * Net/KernelNet.cpp:440-458), y [rows, out] f32; x and weight may start at any
+ * of their values. Up to four rows take the split GEMV (as do 5 to 16 whose
+ * inner extent or addresses are not whole vectors), more the matrix cores: in
+ * 16-bit parts of x for more than 16 rows of 16-bit weights with inner % 32 == 0,
+ * out % 128 == 0 and x at 16 bytes, else in fp32. The parts are three bf16 ones
+ * for bf16 weights, exact, and two fp16 ones for fp16 weights: within 2^-22 of a
+ * value or 2^-25, whichever is larger, for |x| < 65504 (past that the parts
+ * are infinite and the outputs NaN). They go through the context's scratch, so
+ * calls on one context have to be ordered. Replaces
+ * KernelNet::dispatchProjection (Net/KernelNet.cpp:817-859) over SplitLinear /
+ * HalfWeightSplitLinear (Kernels/Linear.h:129-276) and LinearProduct
+ * (Kernels/SimdTiledMatMul.h:470-486). */
 int wsp_hip_linear(wsp_hip_ctx* ctx, const float* x, int rows, int inner, const void* weight,
                    int wdtype, const float* bias, float* y, int out, int flags);
 
@@ -126,8 +134,8 @@ int wsp_hip_embed(wsp_hip_ctx* ctx, const uint32_t* tokens, int count, const flo
  * width / heads columns. scale multiplies the summed dot product. One query
  * takes the split-key form (Kernels/SingleQueryAttention.h:505-556); several
  * take the causal multi-query form with the mask semantics of
- * Kernels/Attention.h:34-47, on the matrix cores for heads of 64 channels. Replaces KernelNet::runCachedAttention
- * (Net/KernelNet.cpp:951-1013). Head width must be a multiple of 4, at most 64
+ * Kernels/Attention.h:34-47, on the matrix cores for heads of 64 channels.
+ * Replaces KernelNet::runCachedAttention (Net/KernelNet.cpp:951-1013). Head width must be a multiple of 4, at most 64
  * (the reference's own limit, Kernels/SingleQueryAttention.cpp:32-45). */
 int wsp_hip_attention(wsp_hip_ctx* ctx, const float* q, int q_count, const float* keys,
                       const float* values, int k_count, int width, int heads, int causal,
@@ -283,7 +291,8 @@ int wsp_hip_raise_device_status(wsp_hip_ctx* ctx);
  * and every stream's rows equal what Decoder::step computes for that stream
  * alone (Decoder/Decoder.cpp:270-308). Projections need 16-bit storage (F16
  * or BF16): they run on the matrix cores with the fp32 activations split into
- * exact 16-bit parts. */
+ * 16-bit parts (as wsp_hip_linear's). A batch holds up to 64 MB, or one
+ * stream's encoder rows, of such parts for wsp_batch_begin. */
 
 /* One layer's cross-attention key and value projections (Decoder/DecoderWeights.h:25-63). */
 typedef struct wsp_cross_tensors

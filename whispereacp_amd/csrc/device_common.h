@@ -229,11 +229,13 @@ __device__ __forceinline__ void normalise_row(const float* __restrict__ src, con
         v[i] = v[i] * rstd * scales[i] + shifts[i];
 }
 
-// x as exact 16-bit parts for products with 16-bit weights of type WT
-// (kF16: fp16 hi + lo, for |x| < 65504; kBF16: three bf16 parts); part p in
-// the low 16 bits of bits[p], and x equals the sum of the parts.
+// x as 16-bit parts for products with 16-bit weights of type WT; part p in the
+// low 16 bits of bits[p]. kBF16: three bf16 parts whose sum is x. kF16: fp16 hi
+// + lo, for |x| < 65504, whose sum is within 2^-22 of x's magnitude or 2^-25
+// (half the last place of fp16's least numbers), whichever is larger; past that
+// hi is infinite and lo NaN.
 template <int WT>
-__device__ __forceinline__ void exact_parts(float x, uint32_t (&bits)[3])
+__device__ __forceinline__ void cut_parts(float x, uint32_t (&bits)[3])
 {
     if constexpr (WT == kF16)
     {

@@ -148,7 +148,7 @@ __device__ __forceinline__ f32x4 mfma3(const f16x8& ah, const f16x8& al, const f
 //
 // Key splits: blockIdx.z takes keys [z·span, min((z + 1)·span, count)); with
 // one split the block writes the normalised rows to out (OUT = kF32) or as
-// the exact 16-bit parts of the output product's input (OUT = kF16, kBF16:
+// the 16-bit parts of the output product's input (OUT = kF16, kBF16:
 // part p at out_parts + p·out_part_stride), with several it writes (max, sum,
 // row) partials [split][head][query][66] for flash_combine_kernel.
 template <int WAVES, int OUT>
@@ -351,7 +351,7 @@ __global__ void __launch_bounds__(WAVES * 64) flash_attention_kernel(const float
                 uint32_t bits[4][3];
 #pragma unroll
                 for (int r = 0; r < 4; ++r)
-                    exact_parts<OUT>(o[t][r] * inv, bits[r]);
+                    cut_parts<OUT>(o[t][r] * inv, bits[r]);
 #pragma unroll
                 for (int p = 0; p < (OUT == kF16 ? 2 : 3); ++p)
                     *reinterpret_cast<uint2*>(out_parts + p * out_part_stride + at)
@@ -417,7 +417,7 @@ __global__ void __launch_bounds__(4 * kFlashWidth) flash_combine_kernel(const fl
     else
     {
         uint32_t bits[3];
-        exact_parts<OUT>(v, bits);
+        cut_parts<OUT>(v, bits);
 #pragma unroll
         for (int p = 0; p < (OUT == kF16 ? 2 : 3); ++p)
             out_parts[p * out_part_stride + at] = (uint16_t) bits[p];
@@ -454,7 +454,7 @@ struct wsp_encoder
     float* v = nullptr;
     float* att = nullptr;
     float* ff = nullptr;      // [positions, feed_forward_width]
-    // 16-bit weights: a product's input as exact 16-bit parts (split_product):
+    // 16-bit weights: a product's input as 16-bit parts (split_product):
     // up to three [positions, width] parts, and fc2's [positions, feed_forward_width].
     void* parts = nullptr;
     void* ff_parts = nullptr;

@@ -21,7 +21,7 @@
 // registers (a lane's eight consecutive k; any assignment of k to lanes serves
 // as long as both operands share it), and the eight partial tiles are added in
 // wave order through LDS, so the result does not depend on timing. SPLIT takes
-// 16-bit weights in their own type with X cut into exact 16-bit parts (as
+// 16-bit weights in their own type with X cut into 16-bit parts (as
 // split_product's), otherwise everything is fp32.
 //
 // In these two W is the matrix cores' row operand, X their column operand: a
@@ -361,8 +361,8 @@ __global__ void __launch_bounds__(kRowWaves * kWave) row_product_kernel(RowProdu
                 for (int j = 0; j < 4; ++j)
                 {
                     uint32_t b0[3], b1[3];
-                    exact_parts<WT>(x[mt][2 * j], b0);
-                    exact_parts<WT>(x[mt][2 * j + 1], b1);
+                    cut_parts<WT>(x[mt][2 * j], b0);
+                    cut_parts<WT>(x[mt][2 * j + 1], b1);
 #pragma unroll
                     for (int p = 0; p < 3; ++p)
                         xb[mt][p][j] = b0[p] | (b1[p] << 16);
@@ -507,7 +507,7 @@ __global__ void __launch_bounds__(kCutThreads) cut_product_kernel(RowProduct a)
             uint32_t bits[4][3];
 #pragma unroll
             for (int e = 0; e < 4; ++e)
-                exact_parts<WT>(xv[i][e], bits[e]);
+                cut_parts<WT>(xv[i][e], bits[e]);
 #pragma unroll
             for (int p = 0; p < P; ++p)
                 cut[i][p] = uint2 {bits[0][p] | (bits[1][p] << 16), bits[2][p] | (bits[3][p] << 16)};

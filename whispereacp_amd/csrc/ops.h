@@ -30,8 +30,8 @@ struct ProductMatrix
 };
 constexpr int kMaxMatrices = 64;
 
-// The products over X as split_product's kernel reads it: exact 16-bit parts
-// for 16-bit W (three bf16 parts, or fp16 hi + lo), part p at
+// The products over X as split_product's kernel reads it: 16-bit parts for
+// 16-bit W (cut_parts: three bf16 parts, or fp16 hi + lo), part p at
 // parts + p·part_stride + r·inner, or fp32 X for fp32 W. `count` matrices of
 // `columns` columns share the launch. Row r of a column lands at
 // y[(r / rows_per_group)·group_stride + (r % rows_per_group)·ldy + c]
@@ -152,7 +152,9 @@ constexpr size_t kQueryAttentionFloats = kAttentionCounters + (size_t) kQueryBlo
 // workspace (floats) it needs: the counters, then the partials —
 // chunks * (head_width + 2) per (head, query) for one query or more than
 // kMaxPromptQueries, splits * kMaxPromptQueries * (kMaxHeadWidth + 2) per head
-// for a prompt step.
+// for a prompt step. The entry points refuse what their workspace does not hold
+// of this, several queries of 64-channel heads too, which never take more than
+// kQueryAttentionFloats.
 int attention_chunks(int heads, int q_count, int k_count);
 int prompt_attention_splits(int heads, int k_count);
 size_t attention_workspace_floats(int heads, int q_count, int k_count, int head_width);

@@ -4,11 +4,12 @@
 // products of every layer and the convolutions; the cross keys and values of
 // every layer, and long prompts, through linear_product.hip).
 //
-// For 16-bit W, X is stored once in exact 16-bit parts (three bf16 parts for bf16 weights,
-// fp16 hi + lo for fp16 weights, |x| < 65504), part-major: part p of row r at
-// parts + p·part_stride + r·inner. Every matrix-core product of a part with W
-// is exact, and the fp32 sums match an fp32 product with widened weights to
-// fp32 rounding. The parts are written by split_rows (from fp32 rows) or by a
+// For 16-bit W, X is stored once in 16-bit parts (cut_parts: three bf16 parts for
+// bf16 weights, together exact; fp16 hi + lo for fp16 weights, within 2^-22 of
+// |x| < 65504 or 2^-25), part-major: part p of row r at parts + p·part_stride +
+// r·inner. Every matrix-core product of a part with W is exact, and the fp32
+// sums match an fp32 product with widened weights to fp32 rounding (fp16: to the
+// parts'). The parts are written by split_rows (from fp32 rows) or by a
 // product's own epilogue (fc1 writes its GELU output as parts for fc2), so
 // the products' inner loops carry no conversion work.
 //
@@ -94,7 +95,7 @@ __device__ __forceinline__ float4v multiply(u32x4 a, u32x4 b, float4v c)
 template <int WT>
 __device__ __forceinline__ void split(float x, uint32_t (&bits)[3])
 {
-    exact_parts<WT>(x, bits);
+    cut_parts<WT>(x, bits);
 }
 
 // Eight consecutive values of a row as parts: part p's eight 16-bit values in
