@@ -34,8 +34,6 @@ namespace wsp::batch
 namespace
 {
 typedef uint16_t u16;
-typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
-typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
 constexpr int kProductThreads = 512; // 8 waves split the inner dimension of a 16-column tile
 constexpr int kProductWaves = kProductThreads / kWave;
@@ -43,12 +41,6 @@ constexpr int kAttendThreads = 256;  // 16 key groups x 16 lanes of four channel
 constexpr int kTileKeys = 128;       // keys an attention block holds per pass
 constexpr int kNormThreads = 256;
 constexpr int kMaxRowTiles = 8;      // 16-row tiles per product: 128 rows
-
-template <int WT>
-constexpr int parts_of()
-{
-    return WT == kF16 ? 2 : 3;
-}
 
 // x as 16-bit parts at out[p * part_stride + index].
 template <int WT>
@@ -214,15 +206,6 @@ __device__ __forceinline__ void split_value(float x, u16 (&out)[parts_of<WT>()])
             rest -= (float) b;
         }
     }
-}
-
-template <int WT>
-__device__ __forceinline__ float4v mfma16(u32x4 a, u32x4 b, float4v c)
-{
-    if constexpr (WT == kF16)
-        return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(half8, a), __builtin_bit_cast(half8, b), c, 0, 0, 0);
-    else
-        return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
 }
 
 // ---------------------------------------------------------------------------

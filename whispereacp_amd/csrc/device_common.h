@@ -11,6 +11,8 @@ constexpr int kWave = 64;
 
 typedef _Float16 half8 __attribute__((ext_vector_type(8)));
 typedef _Float16 half4 __attribute__((ext_vector_type(4)));
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 typedef float float4v __attribute__((ext_vector_type(4)));
 typedef float float4u __attribute__((ext_vector_type(4), aligned(4))); // the same at any float
 
@@ -72,7 +74,6 @@ __device__ __forceinline__ float sum16(float v)
 // 16 bytes from global memory.
 __device__ __forceinline__ uint4 load_global16(const void* p)
 {
-    typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
     const u32x4 v = *global(static_cast<const u32x4*>(p));
     return make_uint4(v[0], v[1], v[2], v[3]);
 }
@@ -256,6 +257,32 @@ __device__ __forceinline__ void cut_parts(float x, uint32_t (&bits)[3])
             rest -= (float) b;
         }
     }
+}
+
+// How many parts those are (an fp32 weight's rows are read as they are).
+template <int WT>
+constexpr int parts_of()
+{
+    return WT == kF32 ? 1 : WT == kF16 ? 2 : 3;
+}
+
+// c + a·b over 32 k of 16-bit values of type WT, a 16 x 16 tile.
+template <int WT>
+__device__ __forceinline__ float4v mfma16(u32x4 a, u32x4 b, float4v c)
+{
+    if constexpr (WT == kF16)
+        return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(half8, a), __builtin_bit_cast(half8, b), c, 0,
+                                                       0, 0);
+    else
+        return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c,
+                                                        0, 0, 0);
+}
+
+// The 16-byte slot of chunk c of LDS row r, rows of eight chunks (128 bytes): one
+// chunk of eight consecutive rows lies in eight different bank groups.
+__device__ __forceinline__ int chunk_slot(int r, int c)
+{
+    return 8 * r + (c ^ (r & 7));
 }
 
 // The LDS byte address of a shared-memory pointer.

@@ -120,7 +120,6 @@ constexpr int kFlashStages = 2; // 32 KB each
 typedef _Float16 f16x4 __attribute__((ext_vector_type(4)));
 typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
-typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
 __device__ __forceinline__ _Float16 half_hi(float x)
 {
@@ -241,7 +240,6 @@ __global__ void __launch_bounds__(WAVES * 64) flash_attention_kernel(const float
         const int first = k_begin + tile * kFlashKeys;
         const f16x8* const ks = reinterpret_cast<const f16x8*>(stages[stage]);
         const f16x8* const vs = ks + 2 * kPartBytes / 16;
-        auto at = [&](int row, int chunk) { return 8 * row + (chunk ^ (row & 7)); };
 
         // S^T for keys 16 mt + 4 g + r of the tile, query li.
         f32x4 st_[2 * KB];
@@ -252,7 +250,7 @@ __global__ void __launch_bounds__(WAVES * 64) flash_attention_kernel(const float
 #pragma unroll
             for (int s = 0; s < 2; ++s)
             {
-                const int from = at(16 * mt + li, 4 * s + g);
+                const int from = chunk_slot(16 * mt + li, 4 * s + g);
                 st_[mt] = mfma3(ks[from], ks[kPartBytes / 16 + from], qh[s], ql[s], st_[mt]);
             }
         }
@@ -307,7 +305,7 @@ __global__ void __launch_bounds__(WAVES * 64) flash_attention_kernel(const float
 #pragma unroll
             for (int b = 0; b < KB; ++b)
             {
-                const int from = at(16 * t + li, 4 * b + g);
+                const int from = chunk_slot(16 * t + li, 4 * b + g);
                 o[t] = mfma3(vs[from], vs[kPartBytes / 16 + from], ph[b], pl[b], o[t]);
             }
         }

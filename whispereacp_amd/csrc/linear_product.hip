@@ -40,9 +40,7 @@ namespace wsp::ops
 namespace
 {
 typedef uint16_t u16;
-typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
-typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
-typedef uint32_t u32x4u __attribute__((ext_vector_type(4), aligned(2))); // the same at any 16-bit value
+typedef uint32_t u32x4u __attribute__((ext_vector_type(4), aligned(2))); // u32x4 at any 16-bit value
 
 // Up to three matrices a launch here.
 constexpr int kMatrices = 3;
@@ -148,12 +146,6 @@ constexpr int kTileThreads = 256;
 constexpr int kTileRows = 32, kTileColumns = 64;
 constexpr int kTileStep = 32;
 
-// Slot of chunk c (four k) of LDS row r.
-__device__ __forceinline__ int slot(int r, int c)
-{
-    return 8 * r + (c ^ (r & 7));
-}
-
 template <int WT, bool VEC>
 __global__ void __launch_bounds__(kTileThreads, 2) fp32_tile_kernel(RowProduct a)
 {
@@ -200,13 +192,13 @@ __global__ void __launch_bounds__(kTileThreads, 2) fp32_tile_kernel(RowProduct a
         for (int j = 0; j < XC; ++j)
         {
             xr[j].values(v, left);
-            xs[buf][slot(sr + RP * j, sc)] = float4v {v[0], v[1], v[2], v[3]};
+            xs[buf][chunk_slot(sr + RP * j, sc)] = float4v {v[0], v[1], v[2], v[3]};
         }
 #pragma unroll
         for (int j = 0; j < WC; ++j)
         {
             wr[j].values(v, left);
-            ws[buf][slot(sr + RP * j, sc)] = float4v {v[0], v[1], v[2], v[3]};
+            ws[buf][chunk_slot(sr + RP * j, sc)] = float4v {v[0], v[1], v[2], v[3]};
         }
     };
 
@@ -230,10 +222,10 @@ __global__ void __launch_bounds__(kTileThreads, 2) fp32_tile_kernel(RowProduct a
         auto operands = [&](int kk, int set) {
 #pragma unroll
             for (int mt = 0; mt < MT; ++mt)
-                xf[set][mt] = xs[buf][slot(16 * (MT * wm + mt) + li, 4 * kk + g)];
+                xf[set][mt] = xs[buf][chunk_slot(16 * (MT * wm + mt) + li, 4 * kk + g)];
 #pragma unroll
             for (int nt = 0; nt < NT; ++nt)
-                wf[set][nt] = ws[buf][slot(16 * (NT * wn + nt) + li, 4 * kk + g)];
+                wf[set][nt] = ws[buf][chunk_slot(16 * (NT * wn + nt) + li, 4 * kk + g)];
         };
         operands(0, 0);
 #pragma unroll
@@ -281,17 +273,6 @@ __global__ void __launch_bounds__(kTileThreads, 2) fp32_tile_kernel(RowProduct a
 constexpr int kRowWaves = 8;
 constexpr int kRowChunk = 32; // k a wave takes at a time
 
-template <int WT>
-__device__ __forceinline__ float4v mfma16(u32x4 a, u32x4 b, float4v c)
-{
-    if constexpr (WT == kF16)
-        return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(half8, a), __builtin_bit_cast(half8, b), c, 0,
-                                                       0, 0);
-    else
-        return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c,
-                                                        0, 0, 0);
-}
-
 // One chunk's operands of a lane: eight k of MT rows and NT columns.
 template <int WT, int MT, int NT>
 struct RowChunk
@@ -304,7 +285,7 @@ template <int WT, int MT, int NT, bool SPLIT>
 __global__ void __launch_bounds__(kRowWaves * kWave) row_product_kernel(RowProduct a)
 {
     static_assert(!SPLIT || WT != kF32, "parts go with 16-bit weights");
-    constexpr int P = WT == kF16 ? 2 : 3;
+    constexpr int P = parts_of<WT>();
     // Interleaved sums per tile: shorter chains of dependent products (a single
     // one issues every 46 clocks instead of 32) and of roundings. With parts,
     // the first part and the smaller ones are summed apart.
@@ -460,7 +441,7 @@ constexpr int kCutRow = kCutStep + 16; // 16-bit values an LDS row: at 96 bytes 
 template <int WT, int TM>
 __global__ void __launch_bounds__(kCutThreads) cut_product_kernel(RowProduct a)
 {
-    constexpr int P = WT == kF16 ? 2 : 3, NT = 4;
+    constexpr int P = parts_of<WT>(), NT = 4;
     constexpr int MT = TM / 32;                       // 16-row tiles a wave
     constexpr int kValues = TM * kCutStep / kCutThreads; // of X a thread moves a step: 16, 8 or 4
     constexpr int kRowThreads = kCutStep / kValues;

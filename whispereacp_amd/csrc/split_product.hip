@@ -48,19 +48,11 @@ namespace wsp::ops
 namespace
 {
 typedef uint16_t u16;
-typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
-typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
 constexpr int kRowBytes = 128;              // of a tile row per step: 64 16-bit values or 32 fp32
 constexpr int kChunks = kRowBytes / 16;
 constexpr int kLoadRows = 1024 / kRowBytes; // tile rows one wave load (1 KB) covers
 constexpr int kSplitThreads = 256;
-
-template <int WT>
-constexpr int parts_of()
-{
-    return WT == kF32 ? 1 : WT == kF16 ? 2 : 3;
-}
 
 template <int WT>
 constexpr int value_bytes()
@@ -84,18 +76,8 @@ __device__ __forceinline__ float4v multiply(u32x4 a, u32x4 b, float4v c)
             c = __builtin_amdgcn_mfma_f32_16x16x4f32(__uint_as_float(a[e]), __uint_as_float(b[e]), c, 0, 0, 0);
         return c;
     }
-    else if constexpr (WT == kF16)
-        return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(half8, a), __builtin_bit_cast(half8, b), c, 0,
-                                                       0, 0);
     else
-        return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c,
-                                                        0, 0, 0);
-}
-
-template <int WT>
-__device__ __forceinline__ void split(float x, uint32_t (&bits)[3])
-{
-    cut_parts<WT>(x, bits);
+        return mfma16<WT>(a, b, c);
 }
 
 // Eight consecutive values of a row as parts: part p's eight 16-bit values in
@@ -107,8 +89,8 @@ __device__ __forceinline__ void split8(const float (&v)[8], u32x4 (&out)[3])
     for (int j = 0; j < 4; ++j)
     {
         uint32_t b0[3], b1[3];
-        split<WT>(v[2 * j], b0);
-        split<WT>(v[2 * j + 1], b1);
+        cut_parts<WT>(v[2 * j], b0);
+        cut_parts<WT>(v[2 * j + 1], b1);
 #pragma unroll
         for (int p = 0; p < 3; ++p)
             out[p][j] = b0[p] | (b1[p] << 16);
@@ -157,18 +139,12 @@ __global__ void __launch_bounds__(kWave) layernorm_parts_kernel(const float* __r
         uint32_t bits[4][3];
 #pragma unroll
         for (int e = 0; e < 4; ++e)
-            split<WT>(v[i][e], bits[e]);
+            cut_parts<WT>(v[i][e], bits[e]);
 #pragma unroll
         for (int p = 0; p < P; ++p)
             *reinterpret_cast<uint2*>(parts + p * part_stride + row + at)
                 = uint2 {bits[0][p] | (bits[1][p] << 16), bits[2][p] | (bits[3][p] << 16)};
     }
-}
-
-// Slot of chunk c of tile row r (16-byte slots).
-__device__ __forceinline__ int slot(int r, int c)
-{
-    return kChunks * r + (c ^ (r & 7));
 }
 
 // WM x WN waves, each TM / WM rows by TN / WN columns; S stage buffers.
@@ -276,7 +252,7 @@ __global__ void __launch_bounds__(T::kWaves * kWave) split_product_kernel(SplitP
                 const int first = a.inner % kStep / 4; // (inner is a multiple of 4)
                 for (int i = tid; i < (T::TM + T::TN) * kChunks; i += T::kWaves * kWave)
                     if (i % kChunks >= first)
-                        reinterpret_cast<u32x4*>(st)[slot(i / kChunks, i % kChunks)] = u32x4 {0, 0, 0, 0};
+                        reinterpret_cast<u32x4*>(st)[chunk_slot(i / kChunks, i % kChunks)] = u32x4 {0, 0, 0, 0};
                 __syncthreads();
             }
 #pragma unroll
@@ -288,10 +264,10 @@ __global__ void __launch_bounds__(T::kWaves * kWave) split_product_kernel(SplitP
             for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
                 for (int p = 0; p < P; ++p)
-                    af[mt][p] = reinterpret_cast<const u32x4*>(st + p * T::kABytes)[slot(16 * (MT * wm + mt) + li, c)];
+                    af[mt][p] = reinterpret_cast<const u32x4*>(st + p * T::kABytes)[chunk_slot(16 * (MT * wm + mt) + li, c)];
 #pragma unroll
             for (int nt = 0; nt < NT; ++nt)
-                bf[nt] = reinterpret_cast<const u32x4*>(st + P * T::kABytes)[slot(16 * (NT * wn + nt) + li, c)];
+                bf[nt] = reinterpret_cast<const u32x4*>(st + P * T::kABytes)[chunk_slot(16 * (NT * wn + nt) + li, c)];
 #pragma unroll
             for (int p = 0; p < P; ++p)
 #pragma unroll
@@ -342,7 +318,7 @@ __global__ void __launch_bounds__(T::kWaves * kWave) split_product_kernel(SplitP
                 uint32_t bits[4][3];
 #pragma unroll
                 for (int r = 0; r < 4; ++r)
-                    split<WT>(v[r], bits[r]);
+                    cut_parts<WT>(v[r], bits[r]);
                 u16* o = static_cast<u16*>(a.out_parts) + (size_t) row * width + c;
 #pragma unroll
                 for (int p = 0; p < P; ++p)
