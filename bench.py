@@ -692,7 +692,7 @@ def bench_encoder(args):
                                f"kernel over pre-split rows, timed in its kernel trace",
                      "flops_per_launch": 2.0 * T * d * f,
                      "note": "algorithmic flops; the matrix cores do 2x (fp16) or 3x (bf16) of them, one "
-                             "product per exact 16-bit part of the fp32 activations"},
+                             "product per 16-bit part of the fp32 activations"},
         "cpu_baseline": baseline,
         "host_seconds": round(host_s, 4),
     }

@@ -1,11 +1,12 @@
 // wsp_hip_attention_static: wsp_hip_attention without a context, for callers
 // that cannot allocate device memory (code under HIP graph capture, tight
 // serving loops, harnesses that forbid hipMalloc). It runs the same kernels
-// (ops.hip: query_attention_kernel for two and more queries of 64-channel heads,
-// prompt_attention_kernel for 2 to 16 of other heads, else
-// attention_chunk_kernel; attention_combine_kernel behind the first and the
-// last); their split-key partials, which the context-bound entry point keeps in a workspace allocated
-// at wsp_hip_ctx_create, live here in one file-scope device array per GPU.
+// (ops.hip: query_attention_kernel for two and more queries of 64-channel heads
+// but for many over few keys, prompt_attention_kernel for 2 to 16 of other
+// heads, else attention_chunk_kernel; attention_combine_kernel behind the first
+// and the last); their split-key partials, which the context-bound entry point
+// keeps in a workspace allocated at wsp_hip_ctx_create, live here in one
+// file-scope device array per GPU.
 //
 // The array is fixed in size (kStaticAttentionFloats floats, 4 MiB) and held
 // by every GPU the library runs on until the process ends. Every call on a GPU
