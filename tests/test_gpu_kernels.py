@@ -105,7 +105,9 @@ def test_linear_paths(ctx, dtype, rows, inner, out):
 @pytest.mark.parametrize("rows,inner,out,flags", [
     (1500, 96, 384, 0), (1500, 160, 1536, 3), (3001, 32, 5632, 2),  # K in odd 32s: tiles of 32, 64 and 128 rows
     (1500, 384, 768, 1), (701, 128, 1152, 2), (1500, 96, 128, 3),   # short K; few tiles
-    (500, 96, 640, 0), (513, 1056, 1152, 0), (2000, 256, 2048, 0)]) # on either side of the rules
+    (4501, 768, 256, 0), (4501, 512, 768, 2),                       # few columns
+    (500, 96, 640, 0), (513, 1056, 1152, 0), (2000, 256, 2048, 0),  # on either side of the rules
+    (3001, 640, 3072, 0)])                                          # a part-filled second round
 def test_linear_of_parts_cut_on_the_way(ctx, dtype, rows, inner, out, flags):
     # Many rows of 16-bit weights that do not go through stored parts, against
     # float64; the bound is test_linear_matches_oracle's.

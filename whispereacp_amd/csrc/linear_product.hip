@@ -675,20 +675,26 @@ hipError_t unstored_parts_product(hipStream_t stream, const Products& p)
 // together) X is stored as parts, every matrix going through split_product in
 // launches of up to 64; fewer, and what split_product or the scratch does not
 // take, without (96 x 768 -> 768 runs 5.3 us there, 96 x 3072 -> 768 13; 200 x
-// 5120 -> 1280 39, against 20 with the parts' launch). So do short K over many
-// rows where split_product's tiles make one round at most: the launch that stores
-// the parts is then not made up for (1500 x 384 -> 768 in three parts 14.3 us,
-// 11.3 without; 3000 x 384 -> 384 in two 12.7 and 10.7; but 448 x 384 -> 1152
-// 7.5 and 9.7, 1500 x 512 -> 1152 in two 14.8 and 15.6).
+// 5120 -> 1280 39, against 20 with the parts' launch). So do, where one launch
+// takes every matrix, two shapes that do not make up for the launch that stores
+// the parts: short K over many rows whose tiles in split_product are one round
+// at most (300 x 64 -> 768 7.0 us, 5.5 without; 1500 x 384 -> 768 in three parts 14.3, 11.3 without; 3000 x 384 ->
+// 384 in two 12.7 and 10.7; but 448 x 384 -> 1152 7.5 and 9.7, 1500 x 512 ->
+// 1152 in two 14.8 and 15.6), and few columns under very many rows (12000 x 768 ->
+// 768 in three parts 79.7 and 67.8, in two 62.3 and 56.8 but 6000 x 1280 -> 768
+// 50.6 and 53.7: in two up to 512 of K).
 template <int WT>
 hipError_t parts_product(hipStream_t stream, const Products& p, const Scratch& scratch)
 {
     const long long units = compute_units(), out = (long long) p.columns * p.count, outputs = p.rows * out;
     auto blocks = [&](int tm, int tn) { return (p.rows + tm - 1) / tm * (out / tn); };
     const int slab = slab_rows(p, scratch);
-    const bool short_inner = p.inner <= (WT == kF16 ? 384 : 512) && p.rows >= 700 && blocks(64, 128) <= units
-                             && 2 * blocks(WT == kF16 ? 64 : 32, 128) >= units;
-    if (outputs <= 1 << 17 || short_inner || slab == 0 || !whole_vectors(p, 8)
+    const bool short_inner = p.count <= kMatrices && blocks(64, 128) <= units
+                             && (p.inner <= 64 || (p.inner <= (WT == kF16 ? 384 : 512) && p.rows >= 700
+                                                   && 2 * blocks(WT == kF16 ? 64 : 32, 128) >= units));
+    const bool few_columns = p.count <= kMatrices && p.rows >= 4500
+                             && (WT == kF16 ? out <= 768 && p.inner <= 512 : out <= 1024);
+    if (outputs <= 1 << 17 || short_inner || few_columns || slab == 0 || !whole_vectors(p, 8)
         || !split_product_fits(p.wdtype, p.inner, p.columns) || (size_t) p.columns * p.inner >= 1u << 30) // (32-bit byte offsets)
         return unstored_parts_product<WT>(stream, p);
     hipError_t e = hipSuccess;

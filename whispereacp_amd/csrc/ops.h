@@ -14,7 +14,7 @@ constexpr int kSplitRowLimit = 16;
 constexpr int kMaxHeadWidth = 64;
 constexpr int kAttentionChunkKeys = 1024; // longest key chunk one workgroup scores
 
-// CUs of the current device.
+// CUs of a GPU.
 int compute_units();
 
 // One of the matrices side by side in a product: W [columns][inner], its bias

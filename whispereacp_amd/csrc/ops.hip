@@ -8,8 +8,6 @@
 #include "ops.h"
 
 #include <algorithm>
-#include <array>
-#include <atomic>
 #include <cmath>
 
 namespace wsp::ops
@@ -873,18 +871,18 @@ hipError_t launch_gemv(hipStream_t stream, const float* x, int rows, int inner, 
 
 } // namespace
 
+// (Asked once: a node's GPUs are alike, the number only steers the choice of
+// tiles, and to ask for the current device at each launch costs 0.3 us.)
 int compute_units()
 {
-    static std::array<std::atomic<int>, 64> known {};
-    int device = 0, count = 0;
-    if (hipGetDevice(&device) != hipSuccess || device < 0 || device >= (int) known.size())
+    static const int units = [] {
+        int device = 0, count = 0;
+        if (hipGetDevice(&device) == hipSuccess
+            && hipDeviceGetAttribute(&count, hipDeviceAttributeMultiprocessorCount, device) == hipSuccess && count > 0)
+            return count;
         return 256;
-    if ((count = known[device].load(std::memory_order_relaxed)) > 0)
-        return count;
-    if (hipDeviceGetAttribute(&count, hipDeviceAttributeMultiprocessorCount, device) != hipSuccess || count <= 0)
-        return 256;
-    known[device].store(count, std::memory_order_relaxed);
-    return count;
+    }();
+    return units;
 }
 
 hipError_t linear(hipStream_t stream, const float* x, int rows, int inner, const void* weight,

@@ -455,10 +455,12 @@ hipError_t allow_tiles()
 // CUs idle for all of it): 128 x 256, 64 x 128, 32 x 128, else 32 x 64. At 1500
 // rows 1536 -> 384 ran 9.8 us as 141 blocks of 32 x 128, 13.6 as 72 of 64 x 128
 // and 14.5 as 282 of 32 x 64; 768 -> 2304 17.3 as 432 of 64 x 128, 19.9 in 64 x
-// 64 and 23 as 108 of 128 x 256. Up to 512 of K, 128 x 256 tiles also have to
-// give every CU a block (3000 x 256 -> 2048, fp16: 18.3 us as 752 blocks of 64 x
-// 128, 21.6 as 192 of 128 x 256; 1500 x 512 -> 5120 27.1 and 27.7; 768 of K 34.1
-// and 34.0). With at most one 64 x 128 block a CU, four
+// 64 and 23 as 108 of 128 x 256. 128 x 256 tiles of several rounds over the
+// CUs, or of up to 512 of K, also have to keep four fifths of their rounds busy,
+// unless the columns are few and the rows' parts the larger operand: 3000 x 1280
+// -> 3072 in two rounds of 288 (56%) 78.1 us, 65.3 as 1128 blocks of 64 x 128;
+// 3000 x 256 -> 2048 as 192 (75%) 21.6 and 18.3; but 4500 x 512 -> 1536 as 216
+// (84%) 29.1 and 29.9, 6000 x 512 -> 1024 as 188 29.3 and 31.6. With at most one 64 x 128 block a CU, four
 // stages hide the loads (5120 -> 1280: 45 us against 60 with two); with more,
 // two let the blocks share a CU (768 -> 2304: 17.3 against 19.6 with four).
 template <int WT>
@@ -467,7 +469,9 @@ hipError_t launch_tiles(hipStream_t stream, const SplitProduct& a)
     const long long units = compute_units();
     const int out = a.count * a.columns;
     auto blocks = [&](int tm, int tn) { return (long long) ((a.rows + tm - 1) / tm) * (out / tn); };
-    if (a.columns % 256 == 0 && (a.inner > 512 ? 2 : 1) * blocks(128, 256) >= units)
+    const long long widest = blocks(128, 256), rounds = (widest + units - 1) / units;
+    if (a.columns % 256 == 0 && 2 * widest >= units
+        && (out <= 1024 || (rounds == 1 && a.inner > 512) || 5 * widest >= 4 * rounds * units))
         return launch<typename Tiles<WT>::Widest, WT>(stream, a);
     if (blocks(64, 128) > units)
         return launch<typename Tiles<WT>::Shared, WT>(stream, a);
